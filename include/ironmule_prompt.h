@@ -1,0 +1,61 @@
+/*
+ * ironmule_prompt.h — C ABI of the 4-bit products for more than 32 activation rows on MI355X
+ * (gfx950), in libironmule_qmv.so: prompts and expert batches.
+ *
+ * The weights are read as they are stored (w, scales, biases of ironmule_qmv.h); the
+ * activations are packed first, into the order the matrix instructions read.  Each output is
+ * sum_k (s q + b) x with exact products and fp32 sums.
+ *
+ * Contract (as for ironmule_qmv.h): device pointers allocated by the caller, work queued on
+ * `stream`, no allocation or synchronisation per call, int32 return codes with
+ * imq_last_error() for the message.
+ */
+#ifndef IRONMULE_PROMPT_H
+#define IRONMULE_PROMPT_H
+
+#include <stddef.h>
+#include <stdint.h>
+
+#include "ironmule_qmv.h"
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+#define IMQ_PROMPT_MAX_PROBLEMS 3
+#define IMQ_PROMPT_MAX_ROWS (1 << 20)
+#define IMQ_PROMPT_MAX_K (1 << 17)
+
+/* Bytes of packed activations for M rows of K values (0: M or K out of range). */
+IMQ_API size_t imq_prompt_packed_bytes(int32_t M, int32_t K);
+
+/* Packs x, M bf16 rows of K values ldx elements apart (16-byte aligned, ldx a multiple of 8),
+ * into `packed` (imq_prompt_packed_bytes, 16-byte aligned).  One packing serves every product
+ * of the same rows. */
+IMQ_API int32_t imq_prompt_pack(const uint16_t* x, int64_t ldx, int32_t M, int32_t K, void* packed, void* stream);
+
+/* Bytes of workspace imq_prompt_product takes for these problems (0: none). */
+IMQ_API size_t imq_prompt_product_workspace(const imq_problem* p, int32_t count, int32_t M);
+
+/* y_i = x W_i^T for the packed rows x and 1 to 3 weights of the same K (x and ldx of the
+ * problems are not read); y bf16 or fp32, rows ldy apart.  The workspace needs no
+ * preparation; calls that share one must not overlap.
+ * Replaces the prompt path of ironmule/cuda_native.py:177-179 (dequantise, then a matrix
+ * product). */
+IMQ_API int32_t imq_prompt_product(const imq_problem* p, int32_t count, const void* packed, int32_t M,
+                                   int32_t group_size, int32_t bits, int32_t y_dtype, void* workspace,
+                                   size_t workspace_bytes, void* stream);
+
+/* imq_prompt_pack and imq_prompt_product of one weight in one call; the workspace (16-byte
+ * aligned) holds the packed rows and the product's. */
+IMQ_API size_t imq_prompt_matmul_workspace(int32_t M, int32_t N, int32_t K);
+IMQ_API int32_t imq_prompt_matmul(const uint32_t* w, const uint16_t* scales, const uint16_t* biases,
+                                  const uint16_t* x, int64_t ldx, void* y, int64_t ldy, int32_t M, int32_t N,
+                                  int32_t K, int32_t group_size, int32_t bits, int32_t y_dtype, void* workspace,
+                                  size_t workspace_bytes, void* stream);
+
+#ifdef __cplusplus
+}
+#endif
+
+#endif /* IRONMULE_PROMPT_H */

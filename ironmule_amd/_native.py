@@ -25,7 +25,8 @@ ROOT = os.path.dirname(PKG)
 LIB_PATH = os.path.join(PKG, "libironmule_qmv.so")
 HEADER_PATH = os.path.join(ROOT, "include", "ironmule_qmv.h")
 HEADER_PATHS = [HEADER_PATH, os.path.join(ROOT, "include", "ironmule_decode.h"),
-                os.path.join(ROOT, "include", "ironmule_step.h")]
+                os.path.join(ROOT, "include", "ironmule_step.h"),
+                os.path.join(ROOT, "include", "ironmule_prompt.h")]
 
 GROUP_SIZE = 64
 BITS = 4
@@ -151,6 +152,15 @@ _SIGNATURES = {
                                     _I32, _I32, _I32, ctypes.c_float, ctypes.c_float, _P, _P, _P],
                                    _I32),
     "imq_silu_mul": ([_P, _P, _P, _I64, _P], _I32),
+    # more than 32 rows (include/ironmule_prompt.h)
+    "imq_prompt_packed_bytes": ([_I32, _I32], ctypes.c_size_t),
+    "imq_prompt_pack": ([_P, _I64, _I32, _I32, _P, _P], _I32),
+    "imq_prompt_product_workspace": ([ctypes.POINTER(Problem), _I32, _I32], ctypes.c_size_t),
+    "imq_prompt_product": ([ctypes.POINTER(Problem), _I32, _P, _I32, _I32, _I32, _I32, _P, ctypes.c_size_t, _P],
+                           _I32),
+    "imq_prompt_matmul_workspace": ([_I32, _I32, _I32], ctypes.c_size_t),
+    "imq_prompt_matmul": ([_P, _P, _P, _P, _I64, _P, _I64, _I32, _I32, _I32, _I32, _I32, _I32, _P, ctypes.c_size_t,
+                           _P], _I32),
     # persistent programs (include/ironmule_step.h)
     "imq_decode_program_create": ([ctypes.POINTER(StepDesc), ctypes.POINTER(_P)], _I32),
     "imq_qmv_program_create": ([ctypes.POINTER(QmvStage), _I32, ctypes.POINTER(_P)], _I32),
@@ -453,6 +463,52 @@ def dequant(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
         out = torch.empty((n, k), dtype=out_dtype, device=w.device)
     _check(lib().imq_dequant(_ptr(w), _ptr(scales), _ptr(biases), _ptr(out),
                              _DTYPE_CODE[out_dtype], n, k, GROUP_SIZE, BITS, _stream(stream)))
+    return out
+
+
+# --------------------------------------------------------------- more than 32 rows
+
+MAX_PROMPT_ROWS = 1 << 20
+MAX_PROMPT_K = 1 << 17
+
+
+def takes_prompt(x: torch.Tensor, k: int) -> bool:
+    """Whether prompt_matmul takes these bf16 rows of k values: a plain tensor that nothing
+    differentiates, traces or maps (those calls need operations torch knows), within the
+    kernels' sizes."""
+    rows = x.numel() // k
+    return (x.dtype == torch.bfloat16 and x.is_cuda and 1 <= rows <= MAX_PROMPT_ROWS and k <= MAX_PROMPT_K
+            and type(x) in (torch.Tensor, torch.nn.Parameter)
+            and not (x.requires_grad and torch.is_grad_enabled())
+            and torch.autograd.forward_ad._current_level < 0
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and torch._C._len_torch_dispatch_stack() == 0)
+
+
+def _aligned_rows(x: torch.Tensor, k: int) -> tuple[torch.Tensor, int]:
+    """x as (rows, k) bf16 rows the kernels can load 16 bytes at a time, and their stride."""
+    x2 = x.reshape(-1, k)
+    ld = int(x2.stride(0)) if x2.shape[0] > 1 else k
+    if x2.stride(1) != 1 or ld < k or ld % 8 or x2.data_ptr() % 16:
+        x2, ld = x2.clone(memory_format=torch.contiguous_format), k
+    return x2, ld
+
+
+def prompt_matmul(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor, x: torch.Tensor,
+                  out_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
+    """y = x @ dequantize(w, scales, biases).T for any number of bf16 rows (imq_prompt_matmul):
+    exact products of the 4-bit weights as they are stored, fp32 sums, y bf16 or fp32 (M, N),
+    on the current stream."""
+    n, k = check_weights(w, scales, biases)
+    if x.dtype != torch.bfloat16 or x.dim() < 1 or int(x.shape[-1]) != k:
+        raise ValueError(f"x must be bf16 rows of {k} values")
+    x2, ld = _aligned_rows(x, k)
+    m = int(x2.shape[0])
+    out = torch.empty((m, n), dtype=out_dtype, device=w.device)
+    nbytes = int(lib().imq_prompt_matmul_workspace(m, n, k))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=w.device)
+    _check(lib().imq_prompt_matmul(_ptr(w), _ptr(scales), _ptr(biases), _ptr(x2), ld, _ptr(out), n, m, n, k,
+                                   GROUP_SIZE, BITS, _DTYPE_CODE[out_dtype], _ptr(ws), nbytes, _stream(None)))
     return out
 
 

@@ -1,0 +1,738 @@
+// MI355X (gfx950) kernels for more than 32 activation rows (prompts, expert batches) and
+// their C ABI (include/ironmule_prompt.h): activations packed into MFMA operand order, and a
+// matrix product that reads the 4-bit weights as they are stored.
+
+#include <hip/hip_runtime.h>
+#include <math.h>
+#include <stdint.h>
+#include <string.h>
+
+#include <string>
+
+#include "../../include/ironmule_prompt.h"
+#include "common.h"
+#include "runtime.h"
+
+namespace {
+
+using namespace imq_dev;
+
+using imq_rt::aligned;
+using imq_rt::current_device;
+using imq_rt::DeviceInfo;
+using imq_rt::fail;
+using imq_rt::ok;
+
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+
+constexpr int kThreads = 256;
+
+// ------------------------------------------------------------ packed activations
+//
+// Rows are packed in blocks of 32, columns in chunks of four groups (256 columns).  A
+// (block, chunk) is kChunkBytes: four groups of 4 KB, then 2 KB of group sums.
+//   group    piece c (columns 8c .. 8c+7 of the group) of row m at c * 512 + m * 16, its eight
+//            bf16 in the pair order of the unpacked nibbles (x0 x4 x1 x5 x2 x6 x3 x7): lane
+//            (m, h) of an MFMA reads piece 4 h + j as its A operand of k-step j.
+//   sums     X = the row's sum over the group, as three bf16 terms (hi + mid + lo = X to 24
+//            bits): half (t, h) at (2 t + h) * 512, row m at m * 16, eight bf16
+//            (X of groups 0..3, then -16 X of groups 0..3), of hi for (0, 0), mid for (0, 1),
+//            lo for (1, 0) and zero for (1, 1): the A operands of two k-steps against
+//            (biases of the four groups, scales of the four groups).
+// A row holding a value that could overflow fp32 sums (|x| >= 2^96, infinities, NaN) has its
+// bit set in the (block, chunk)'s flag word and zeros for sums: its outputs are
+// computed value by value.
+constexpr int kGroupBytes = 4096;
+constexpr int kSumBytes = 2048;
+constexpr int kChunkBytes = 4 * kGroupBytes + kSumBytes;
+constexpr uint32_t kHuge = 0x6f80u;  // bf16 exponent field of 2^96
+
+__device__ __forceinline__ uint32_t exponent_max(uint32_t u, uint32_t m) {
+  const uint32_t lo = u & 0x7f80u, hi = (u >> 16) & 0x7f80u;
+  m = m > lo ? m : lo;
+  return m > hi ? m : hi;
+}
+
+// A (block, chunk) from row-major x into its LDS image, 16 bytes (one piece) per step of a
+// thread; `piece` 0..31 of the chunk (columns 8 piece ..), `row` 0..31 of the block.  The 32
+// lanes of a half wavefront hold one row's chunk.
+__device__ __forceinline__ void pack_piece(uint4 d, int piece, int row, char* image, uint32_t* flag) {
+  const int g = piece >> 3, c = piece & 7;
+  *reinterpret_cast<uint4*>(image + g * kGroupBytes + c * 512 + row * 16) = pair_order(d);
+  uint32_t e = exponent_max(d.x, 0u);
+  e = exponent_max(d.y, e);
+  e = exponent_max(d.z, e);
+  e = exponent_max(d.w, e);
+  const uint64_t huge = __ballot(e >= kHuge);
+  const bool flagged = (uint32_t)(huge >> (threadIdx.x & 32)) != 0u;
+  float s = sum8(d);
+  s += dpp<0xB1>(s);   // lanes ^ 1
+  s += dpp<0x4E>(s);   // lanes ^ 2
+  s += dpp<0x141>(s);  // the other four of the eight
+  if (c != 0) return;
+  if (flagged) {
+    s = 0.0f;
+    if (g == 0) atomicOr(flag, 1u << row);
+  }
+  char* const at = image + 4 * kGroupBytes + row * 16 + g * 2;
+  float left = s;
+#pragma unroll
+  for (int t = 0; t < 3; ++t) {
+    const uint16_t part = f32_to_bf16_bits(left);
+    const float v = bf16_bits_to_f32(part);
+    left -= v;
+    *reinterpret_cast<uint16_t*>(at + t * 512) = part;
+    *reinterpret_cast<uint16_t*>(at + t * 512 + 8) = (uint16_t)(__float_as_uint(-16.0f * v) >> 16);
+  }
+  *reinterpret_cast<uint16_t*>(at + 3 * 512) = 0;
+  *reinterpret_cast<uint16_t*>(at + 3 * 512 + 8) = 0;
+}
+
+// One workgroup per (chunk, block).  `src` (may be null): the x row of each packed row, -1 for
+// a row of zeros; without it packed row r is x row r, zeros past M.
+__global__ __launch_bounds__(kThreads) void pack_rows_kernel(const uint16_t* __restrict__ x, int64_t ldx,
+                                                             const int32_t* __restrict__ src, int M, int K,
+                                                             char* __restrict__ packed,
+                                                             uint32_t* __restrict__ flags) {
+  __shared__ __attribute__((aligned(16))) char image[kChunkBytes];
+  __shared__ uint32_t flag;
+  const int chunk = blockIdx.x, block = blockIdx.y, chunks = gridDim.x;
+  const int tid = threadIdx.x, piece = tid & 31;
+  if (tid == 0) flag = 0u;
+  const int col = 256 * chunk + 8 * piece;
+  uint4 d[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = 32 * block + 8 * i + (tid >> 5);
+    const int64_t row = src ? src[r] : (r < M ? r : -1);
+    d[i] = make_uint4(0u, 0u, 0u, 0u);
+    if (row >= 0 && col < K) d[i] = *reinterpret_cast<const uint4*>(x + row * ldx + col);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; ++i) pack_piece(d[i], piece, 8 * i + (tid >> 5), image, &flag);
+  __syncthreads();
+  uint4* const out = reinterpret_cast<uint4*>(packed + ((int64_t)block * chunks + chunk) * kChunkBytes);
+  for (int i = tid; i < kChunkBytes / 16; i += kThreads) out[i] = reinterpret_cast<const uint4*>(image)[i];
+  if (tid == 0) flags[block * chunks + chunk] = flag;
+}
+
+// ------------------------------------------------------------ the product
+//
+// y[m][n] = sum_g s[n][g] sum_k (16 + q) x + (b[n][g] - 16 s[n][g]) sum_k x over the groups g.
+//
+// A workgroup of four wavefronts computes 32 TM rows x 128 columns over a K-range of whole
+// chunks; a wavefront all of the rows for 32 columns, on v_mfma_f32_32x32x16_bf16.
+//   * The packed rows go memory -> LDS by the buffer loads' LDS path, group by group, into a
+//     ring of four arrays, three groups ahead; the four wavefronts share them.
+//   * Each wavefront's weights go straight to registers a chunk ahead: lane (n, h) loads 16
+//     bytes per group, words 4h .. 4h+3 of its row, word 4h+j being its B operand of k-step j
+//     as the exact bf16 values 16 + q.
+//   * Per group each 32 x 32 tile takes four MFMAs from zero and 16 FMAs by the column's
+//     scale; per chunk two more MFMAs of the rows' group sums against the four biases and
+//     scales.  The products are exact and every sum is fp32.
+// One barrier per group.  Within a wavefront the scaling of one tile, the LDS reads of the
+// next and the unpacking of the next group's weights are issued between a tile's MFMAs.
+//
+// What bounds it (K = 2560, 512 workgroups of TM = 4, two per CU; a group takes 1.03 us):
+// MFMA busy 33% of the launch and the VALU about as long (16 FMAs and 8 unpackings per four
+// MFMAs), and the two overlap only in part: without any load or LDS read a group takes 0.61
+// us, the row loads add 0.29 and the weights 0.10.  About 1.04 PFLOP/s marginal, 750-870 TFLOP/s
+// with a launch's start and end.  128 columns x 64 rows as 2 x 2 tiles per wavefront (half the
+// LDS reads, twice the unpacking) and eight wavefronts over 256 columns measured the same;
+// 128 x 64 per wavefront 930 TFLOP/s on large launches, but its 256-column tiles leave a
+// prompt of 512 rows with too few workgroups.  Against imq_dequant and a library product (two
+// conversions of the activations besides): 1024 x 9728 x 2560 89.7 -> 79.5 us in fp16, 77 x
+// 2560 x 9728 70.9 -> 27.6 us in fp32.
+struct ProductProblem {
+  const uint32_t* w;
+  const uint16_t* s;
+  const uint16_t* b;
+  void* y;
+  int64_t ldy;    // with planes: the problem's first column in a plane
+  int32_t N;
+  int32_t tile0;  // first column tile of the launch
+};
+
+struct ProductArgs {
+  ProductProblem p[IMQ_PROMPT_MAX_PROBLEMS];
+  const char* packed;
+  const uint32_t* flags;
+  float* planes;          // fp32 partials (split, row, column of the launch), or null
+  const int32_t* expert;  // per row tile: the expert of its rows, -1 none; null: one weight
+  const int32_t* dest;    // per packed row: the output row, -1 none (with expert)
+  int64_t plane_stride;   // elements between splits
+  int64_t plane_ld;       // elements between rows of a plane
+  int32_t count, M, G, chunks, blocks;
+  int32_t row_tiles, col_tiles, splits, range;  // range: chunks per split
+  int32_t y_f32;
+};
+
+// A value every lane holds, in a scalar register.
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// s_waitcnt immediate that waits for vmcnt <= n and nothing else (gfx9 encoding)
+constexpr int vmcnt_imm(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8); }
+
+// Nibbles p and p + 4 of word u as the bf16 pair (16 + q_p, 16 + q_{p+4}), exact: q in
+// mantissa bits 3..6 of 16.0.
+__device__ __forceinline__ bf16x8_t nibbles16(uint32_t u, uint32_t magic) {
+  const u32x4_t t = {((u << 3) & 0x00780078u) | magic, ((u >> 1) & 0x00780078u) | magic,
+                     ((u >> 5) & 0x00780078u) | magic, ((u >> 9) & 0x00780078u) | magic};
+  return __builtin_bit_cast(bf16x8_t, t);
+}
+
+constexpr int kColumns = 128;  // of a workgroup
+
+template <int TM, bool AL>  // AL: G % 4 == 0 and 8-byte aligned scales and biases
+__global__ __launch_bounds__(kThreads, 2) void product_kernel(ProductArgs a) {
+  constexpr int kXB = TM;                      // row loads per wavefront and group
+  constexpr int kSB = TM > 1 ? TM / 2 : 1;     // sum loads per wavefront and chunk
+  constexpr int kSN = 2;                       // scale and bias loads per chunk, at least
+  __shared__ __attribute__((aligned(16))) uint4 x0[TM * 256];
+  __shared__ __attribute__((aligned(16))) uint4 x1[TM * 256];
+  __shared__ __attribute__((aligned(16))) uint4 x2[TM * 256];
+  __shared__ __attribute__((aligned(16))) uint4 x3[TM * 256];
+  __shared__ __attribute__((aligned(16))) uint4 xsum[4 * kSB * 64];
+
+  // Consecutive workgroups go to the XCDs in turn; each XCD takes a run of tiles in which
+  // the row tiles of a column tile are neighbours, so that its weights stay in one L2.
+  const int total = a.row_tiles * a.col_tiles * a.splits;
+  const int per = (total + 7) >> 3;
+  const int t = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
+  if (t >= total) return;
+  // (divisions leave a uniform value in a vector register: taken back to scalars)
+  const int cs = __builtin_amdgcn_readfirstlane(t / a.row_tiles), rt = t - cs * a.row_tiles;
+  const int ct = __builtin_amdgcn_readfirstlane(cs / a.splits), split = cs - ct * a.splits;
+  int expert = 0;
+  if (a.expert) {
+    expert = __builtin_amdgcn_readfirstlane(a.expert[rt]);
+    if (expert < 0) return;
+  }
+  int pi = 0;
+#pragma unroll
+  for (int i = 1; i < IMQ_PROMPT_MAX_PROBLEMS; ++i)
+    if (i < a.count && ct >= a.p[i].tile0) pi = i;
+  const ProductProblem P = pi == 0 ? a.p[0] : pi == 1 ? a.p[1] : a.p[2];
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int G = a.G, chunks = a.chunks, N = P.N;
+  const int q0 = split * a.range, q1 = min(chunks, q0 + a.range);
+
+  // this wavefront's columns: the problem's rows col0 .. of W.  Every load stays inside its
+  // tensor: lanes past the last row read the last one, groups and blocks past the end the last.
+  const int col0 = (ct - P.tile0) * kColumns + wave * 32;
+  const int rows = min(32, max(1, N - col0));
+  const int64_t wrow = (int64_t)expert * N + min(col0, N - 1);
+  const __amdgpu_buffer_rsrc_t wr = buffer_rsrc(P.w + wrow * (8 * G), (uint32_t)rows * (uint32_t)(32 * G));
+  const __amdgpu_buffer_rsrc_t sr = buffer_rsrc(P.s + wrow * G, (uint32_t)rows * (uint32_t)(2 * G));
+  const __amdgpu_buffer_rsrc_t br = buffer_rsrc(P.b + wrow * G, (uint32_t)rows * (uint32_t)(2 * G));
+  const uint32_t block_bytes = (uint32_t)chunks * kChunkBytes;
+  const int nblocks = min(TM, a.blocks - rt * TM);
+  const __amdgpu_buffer_rsrc_t xr =
+      buffer_rsrc(a.packed + (int64_t)rt * TM * block_bytes, (uint32_t)nblocks * block_bytes);
+  const uint32_t xoff = 16u * lane;
+  uint32_t piece[kXB], sums[kSB];  // this wavefront's 1 KB pieces of a group, and of a chunk's sums
+#pragma unroll
+  for (int e = 0; e < kXB; ++e) {
+    const int p = wave * kXB + e;
+    piece[e] = __builtin_amdgcn_readfirstlane((uint32_t)min(p >> 2, nblocks - 1) * block_bytes + (uint32_t)(p & 3) * 1024u);
+  }
+#pragma unroll
+  for (int e = 0; e < kSB; ++e) {
+    const int p = wave * kSB + e;  // with one block two wavefronts fill a spare part
+    sums[e] = __builtin_amdgcn_readfirstlane((uint32_t)min(p >> 1, nblocks - 1) * block_bytes +
+                                             (uint32_t)(p & 1) * 1024u + 4 * kGroupBytes);
+  }
+  const uint32_t r0 = (uint32_t)min(n, rows - 1);
+  const uint32_t woff = r0 * (uint32_t)(32 * G) + 16u * h, soff = r0 * (uint32_t)(2 * G);
+
+  f32x16_t acc[TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) acc[i] = f32x16_t{};
+  uint4 wq[4], nwq[4];        // this and the next chunk's weights
+  u32x2_t sc, bi, nsc, nbi;   // scales and biases
+  const uint32_t magic = in_vgpr(0x41804180u);
+
+  // a chunk's weights: the four loads of a lane share a cache line
+  auto load_w = [&](int q) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t at = uniform(32u * (uint32_t)min(4 * q + i, G - 1));
+      const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(wr, woff, at, 0);
+      nwq[i] = make_uint4(v.x, v.y, v.z, v.w);
+    }
+  };
+  auto load_scales = [&](int q) {
+    const int c = min(q, chunks - 1);
+    if (AL) {
+      nsc = __builtin_amdgcn_raw_buffer_load_b64(sr, soff, 8 * c, 0);
+      nbi = __builtin_amdgcn_raw_buffer_load_b64(br, soff, 8 * c, 0);
+    } else {  // rows of any alignment; groups past the row's end read zero
+      uint32_t s4[4], b4[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t o = 4 * c + e < G ? soff + 2u * (uint32_t)(4 * c + e) : kPastBuffer;
+        s4[e] = __builtin_amdgcn_raw_buffer_load_b16(sr, o, 0, 0);
+        b4[e] = __builtin_amdgcn_raw_buffer_load_b16(br, o, 0, 0);
+      }
+      nsc = u32x2_t{s4[0] | (s4[1] << 16), s4[2] | (s4[3] << 16)};
+      nbi = u32x2_t{b4[0] | (b4[1] << 16), b4[2] | (b4[3] << 16)};
+    }
+  };
+  auto load_x = [&](int q, int i, uint4* dst) {
+    const uint32_t base = (uint32_t)min(q, q1 - 1) * kChunkBytes + (uint32_t)i * kGroupBytes;
+#pragma unroll
+    for (int e = 0; e < kXB; ++e) {
+      const uint32_t at = uniform(piece[e] + base);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          xr, (__attribute__((address_space(3))) void*)(dst + (wave * kXB + e) * 64), 16, xoff, at, 0, 0);
+    }
+  };
+  auto load_sums = [&](int q) {
+#pragma unroll
+    for (int e = 0; e < kSB; ++e) {
+      const uint32_t at = uniform(sums[e] + (uint32_t)q * kChunkBytes);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          xr, (__attribute__((address_space(3))) void*)(xsum + (wave * kSB + e) * 64), 16, xoff, at, 0, 0);
+    }
+  };
+  // The pipeline over units, a unit being one row tile of one group: its four MFMAs run while
+  // the unit before it is scaled into its accumulator, the unit after it is read from LDS and
+  // the next group's weights are unpacked.  Unit u of group i uses buffers (i TM + u) & 1.
+  bf16x8_t xa[2][4], wb[2][4];
+  f32x16_t p[2];
+  float s[2];
+  auto read_unit = [&](const uint4* xs, int m, bf16x8_t* dst) __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) dst[k] = __builtin_bit_cast(bf16x8_t, xs[m * 256 + (4 * h + k) * 32 + n]);
+  };
+  auto unpack = [&](const uint4& src, int k, bf16x8_t* dst) __attribute__((always_inline)) {
+    dst[k] = nibbles16(k == 0 ? src.x : k == 1 ? src.y : k == 2 ? src.z : src.w, magic);
+  };
+  auto scale_unit = [&](float by, const f32x16_t& from, int m) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[m][e] = fmaf(by, from[e], acc[m][e]);
+  };
+  // group i (0..3, a constant at every call) of chunk q, its rows in xs, the next group's in
+  // xnext; xfree is the array the group three ahead goes to
+  auto group = [&](int i, const uint4* xs, const uint4* xnext, uint4* xfree, int q) __attribute__((always_inline)) {
+    // this wavefront's part of the next group has landed (all that the last group did not
+    // issue); past the barrier every wavefront's has, and nobody reads xfree
+    __builtin_amdgcn_sched_barrier(0);
+    if (i == 0 || i == 3)
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm(kXB));
+    else if (i == 1)
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm(kXB + kSB + 4));
+    else
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm(kXB + kSN));
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    load_x(q + (i + 3) / 4, (i + 3) % 4, xfree);
+    if (i == 0) {
+      load_sums(q);
+      load_w(q + 1);
+    }
+    if (i == 1) load_scales(q + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    const uint32_t two = i < 2 ? sc.x : sc.y;
+    s[i & 1] = __uint_as_float((i & 1) ? (two & 0xffff0000u) : (two << 16));
+#pragma unroll
+    for (int u = 0; u < TM; ++u) {
+      const int at = (i * TM + u) & 1;
+      if (u + 1 < TM)
+        read_unit(xs, u + 1, xa[at ^ 1]);
+      else
+        read_unit(xnext, 0, xa[at ^ 1]);
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        p[at] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[at][k], wb[i & 1][k], k ? p[at] : f32x16_t{}, 0, 0, 0);
+      if (u == 0)
+        scale_unit(s[(i & 1) ^ 1], p[at ^ 1], TM - 1);
+      else
+        scale_unit(s[i & 1], p[at ^ 1], u - 1);
+#pragma unroll
+      for (int k = u * 4 / TM; k < (u + 1) * 4 / TM; ++k) unpack(i < 3 ? wq[(i + 1) & 3] : nwq[0], k, wb[(i & 1) ^ 1]);
+      if (i == 3) {  // the chunk's group sums against its biases and scales
+        const int m = TM > 2 ? (u + 2) % TM : u;
+        const bf16x8_t u0 = __builtin_bit_cast(bf16x8_t, xsum[m * 128 + h * 32 + n]);
+        const bf16x8_t u1 = __builtin_bit_cast(bf16x8_t, xsum[m * 128 + 64 + h * 32 + n]);
+        const bf16x8_t c = __builtin_bit_cast(bf16x8_t, u32x4_t{bi.x, bi.y, sc.x, sc.y});
+        acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(u0, c, acc[m], 0, 0, 0);
+        acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(u1, c, acc[m], 0, 0, 0);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA,
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one operand read,
+        __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);  // six scalings and unpackings
+      }
+    }
+    if (i == 3) {
+      sc = nsc;
+      bi = nbi;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) wq[k] = nwq[k];
+    }
+  };
+
+  load_scales(q0);
+  load_w(q0);
+  __builtin_amdgcn_sched_barrier(0);
+  load_x(q0, 0, x0);
+  __builtin_amdgcn_sched_barrier(0);
+  load_x(q0, 1, x1);
+  __builtin_amdgcn_sched_barrier(0);
+  load_x(q0, 2, x2);
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(kXB));
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  read_unit(x0, 0, xa[0]);
+  sc = nsc;
+  bi = nbi;
+  s[1] = 0.0f;
+  p[1] = f32x16_t{};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) wq[k] = nwq[k];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) unpack(wq[0], k, wb[0]);
+  for (int qv = q0; qv < q1; ++qv) {
+    const int q = __builtin_amdgcn_readfirstlane(qv);
+    group(0, x0, x1, x3, q);
+    group(1, x1, x2, x0, q);
+    group(2, x2, x3, x1, q);
+    group(3, x3, x0, x2, q);
+  }
+  scale_unit(s[1], p[1], TM - 1);  // the range's last unit (4 TM is even)
+  wait_vmem();  // the loads past the range's end, before the LDS is given up
+
+  // rows with values too large for the sums above: every output by itself
+  const int col = col0 + n;
+#pragma unroll
+  for (int m = 0; m < TM; ++m) {
+    const int block = rt * TM + m;
+    uint32_t mask = 0u;
+    if (block < a.blocks)
+      for (int q = lane; q < chunks; q += 64) mask |= a.flags[(int64_t)block * chunks + q];
+    if (__ballot(mask != 0u) == 0) continue;
+    for (int r = 0; r < 32; ++r) {
+      if (__ballot((mask >> r) & 1u) == 0) continue;
+      const char* const xrow = a.packed + (int64_t)block * block_bytes + r * 16;
+      float v = 0.0f;
+      if (split == 0 && col < N) {
+        const int64_t row = wrow + n;
+        for (int g = 0; g < G; ++g) {
+          const float sg = bf16_bits_to_f32(P.s[row * G + g]), bg = bf16_bits_to_f32(P.b[row * G + g]);
+          const char* const xg = xrow + (int64_t)(g >> 2) * kChunkBytes + (g & 3) * kGroupBytes;
+          for (int k = 0; k < 4; ++k) {
+            const uint32_t u = P.w[(row * G + g) * 8 + 4 * h + k];
+            const uint4 d = *reinterpret_cast<const uint4*>(xg + (4 * h + k) * 512);
+            const uint32_t pair[4] = {d.x, d.y, d.z, d.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              v = fmaf(fmaf(sg, (float)((u >> (4 * e)) & 15u), bg), bf16_bits_to_f32(pair[e] & 0xffffu), v);
+              v = fmaf(fmaf(sg, (float)((u >> (4 * e + 16)) & 15u), bg), bf16_bits_to_f32(pair[e] >> 16), v);
+            }
+          }
+        }
+      }
+      v = add_xor32(v);
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        if (8 * (e >> 2) + 4 * h + (e & 3) == r) acc[m][e] = v;
+    }
+  }
+
+  // lane (n, h) holds column n of rows 8 (e / 4) + 4 h + e % 4
+  if (col >= N) return;
+#pragma unroll
+  for (int m = 0; m < TM; ++m)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int r = (rt * TM + m) * 32 + 8 * (e >> 2) + 4 * h + (e & 3);
+      int64_t row = r < a.M ? r : -1;
+      if (a.dest) row = r < a.blocks * 32 ? a.dest[r] : -1;
+      if (row < 0) continue;
+      if (a.planes)
+        a.planes[split * a.plane_stride + row * a.plane_ld + P.ldy + col] = acc[m][e];
+      else if (a.y_f32)
+        static_cast<float*>(P.y)[row * P.ldy + col] = acc[m][e];
+      else
+        static_cast<uint16_t*>(P.y)[row * P.ldy + col] = f32_to_bf16_bits(acc[m][e]);
+    }
+}
+
+// y = the splits' planes added in split order, for the launch's problems; four columns a
+// thread.
+struct SumArgs {
+  ProductProblem p[IMQ_PROMPT_MAX_PROBLEMS];  // ldy: the output's; tile0: the plane's column
+  const float* planes;
+  int64_t plane_stride, plane_ld;
+  int32_t count, M, splits, y_f32;
+};
+
+__global__ __launch_bounds__(kThreads) void sum_planes_kernel(SumArgs a) {
+  const int64_t at = 4 * ((int64_t)blockIdx.x * kThreads + threadIdx.x);
+  if (at >= a.plane_ld * a.M) return;
+  const float* src = a.planes + at;
+  float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  for (int s = 0; s < a.splits; ++s) {
+    const float4 u = *reinterpret_cast<const float4*>(src + s * a.plane_stride);
+    v.x += u.x;
+    v.y += u.y;
+    v.z += u.z;
+    v.w += u.w;
+  }
+  const int row = (int)(at / a.plane_ld), col = (int)(at - row * a.plane_ld);
+  const float out[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int i = 0; i < IMQ_PROMPT_MAX_PROBLEMS; ++i) {
+    if (i >= a.count) break;
+    const ProductProblem& P = a.p[i];
+    const int c = col - P.tile0;  // planes' columns of a problem start at a multiple of four
+    if (c < 0 || c >= P.N) continue;
+    const int64_t o = row * P.ldy + c;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (c + e < P.N) {
+        if (a.y_f32)
+          static_cast<float*>(P.y)[o + e] = out[e];
+        else
+          static_cast<uint16_t*>(P.y)[o + e] = f32_to_bf16_bits(out[e]);
+      }
+  }
+}
+
+// ------------------------------------------------------------ host side
+
+int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
+size_t round_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
+
+struct Plan {
+  int tm, splits, range;  // 32-row blocks of a tile, K-ranges, chunks per range
+  int row_tiles, col_tiles;
+};
+
+int column_tiles(const int32_t* N, int count) {
+  int tiles = 0;
+  for (int i = 0; i < count; ++i) tiles += ceil_div(N[i], kColumns);
+  return tiles;
+}
+
+// The tile height and the K-ranges with the least expected time.  Measured at K = 2560 (40
+// groups) over 32 to 2048 workgroups, a launch takes about 14 / 11 / 9 us, and per group and
+// workgroup of the busiest CU 0.56 / 0.31 / 0.20 us, with tiles of 128 / 64 / 32 rows: tall
+// tiles reuse the weights, short ones fill the CUs.  K-ranges add the planes' traffic (about
+// 4 TB/s each way) and the launch that adds them.
+Plan plan_product(const int32_t* N, int count, int M, int K, int cus) {
+  const int chunks = ceil_div(K, 256), col_tiles = column_tiles(N, count);
+  double columns = 0.0, best = 0.0;
+  for (int i = 0; i < count; ++i) columns += N[i];
+  Plan plan;
+  plan.tm = 0;
+  for (int tm = 4; tm >= 1; tm >>= 1) {
+    const double start = tm == 4 ? 14.0 : tm == 2 ? 11.0 : 9.0, group = tm == 4 ? 0.56 : tm == 2 ? 0.31 : 0.20;
+    const int row_tiles = ceil_div(M, 32 * tm);
+    for (int splits = 1; splits <= 8 && splits <= chunks; ++splits) {
+      const int range = ceil_div(chunks, splits);
+      if (ceil_div(chunks, range) != splits) continue;
+      double us = start + group * 4.0 * range * ceil_div((int64_t)row_tiles * col_tiles * splits, cus);
+      if (splits > 1) us += 5.0 + splits * (double)M * columns * 8.0 / 4e6;
+      if (plan.tm && us >= best) continue;
+      best = us;
+      plan = Plan{tm, splits, range, row_tiles, col_tiles};
+    }
+  }
+  return plan;
+}
+
+size_t flag_bytes(int64_t blocks, int chunks) { return round_up((size_t)blocks * chunks * 4, 256); }
+
+size_t packed_bytes(int64_t blocks, int K) {
+  const int chunks = ceil_div(K, 256);
+  return flag_bytes(blocks, chunks) + (size_t)blocks * chunks * kChunkBytes;
+}
+
+void pack_rows(const uint16_t* x, int64_t ldx, const int32_t* src, int M, int64_t blocks, int K, void* packed,
+               hipStream_t stream) {
+  const int chunks = ceil_div(K, 256);
+  char* const base = static_cast<char*>(packed);
+  hipLaunchKernelGGL(pack_rows_kernel, dim3(chunks, (uint32_t)blocks), dim3(kThreads), 0, stream, x, ldx, src, M, K,
+                     base + flag_bytes(blocks, chunks), reinterpret_cast<uint32_t*>(base));
+}
+
+template <int TM>
+void launch_product(const ProductArgs& a, bool al, uint32_t grid, hipStream_t stream) {
+  if (al)
+    hipLaunchKernelGGL((product_kernel<TM, true>), dim3(grid), dim3(kThreads), 0, stream, a);
+  else
+    hipLaunchKernelGGL((product_kernel<TM, false>), dim3(grid), dim3(kThreads), 0, stream, a);
+}
+
+// Fills the shape fields and launches; p[], planes and the expert tables are the caller's.
+int32_t run_product(ProductArgs& a, const Plan& p, const void* packed, int64_t blocks, int M, int K,
+                    hipStream_t stream) {
+  const int chunks = ceil_div(K, 256);
+  const char* base = static_cast<const char*>(packed);
+  a.flags = reinterpret_cast<const uint32_t*>(base);
+  a.packed = base + flag_bytes(blocks, chunks);
+  a.M = M;
+  a.G = K / 64;
+  a.chunks = chunks;
+  a.blocks = (int32_t)blocks;
+  a.row_tiles = p.row_tiles;
+  a.col_tiles = p.col_tiles;
+  a.splits = p.splits;
+  a.range = p.range;
+  bool al = a.G % 4 == 0;
+  for (int i = 0; i < a.count; ++i) al = al && aligned(a.p[i].s, 8) && aligned(a.p[i].b, 8);
+  const uint32_t grid = 8u * (uint32_t)ceil_div((int64_t)p.row_tiles * p.col_tiles * p.splits, 8);
+  if (p.tm == 4)
+    launch_product<4>(a, al, grid, stream);
+  else if (p.tm == 2)
+    launch_product<2>(a, al, grid, stream);
+  else
+    launch_product<1>(a, al, grid, stream);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(IMQ_ELAUNCH, std::string("product launch failed: ") + hipGetErrorString(e));
+  return ok();
+}
+
+int32_t check_weight(const uint32_t* w, const uint16_t* s, const uint16_t* b, int32_t N, int32_t K,
+                     int32_t group_size, int32_t bits) {
+  if (bits != 4) return fail(IMQ_EUNSUPPORTED, "only 4-bit weights are supported");
+  if (group_size != 64) return fail(IMQ_EUNSUPPORTED, "only group size 64 is supported");
+  if (N < 1) return fail(IMQ_EINVAL, "N must be >= 1");
+  if (K < 64 || K % 64 != 0) return fail(IMQ_EINVAL, "K must be a positive multiple of 64");
+  if (K > IMQ_PROMPT_MAX_K) return fail(IMQ_EUNSUPPORTED, "K too large");
+  if (!w || !s || !b) return fail(IMQ_EINVAL, "w, scales and biases must be non-null");
+  if (!aligned(w, 16)) return fail(IMQ_EINVAL, "w must be 16-byte aligned");
+  if (!aligned(s, 2) || !aligned(b, 2)) return fail(IMQ_EINVAL, "scales/biases must be 2-byte aligned");
+  return IMQ_OK;
+}
+
+// Columns of the launch's planes: each problem's, from a multiple of four.
+int64_t plane_columns(const int32_t* N, int count) {
+  int64_t cols = 0;
+  for (int i = 0; i < count; ++i) cols += round_up(N[i], 4);
+  return cols;
+}
+
+int32_t check_product(const imq_problem* p, int32_t count, int32_t M, int32_t group_size, int32_t bits,
+                      int32_t y_dtype, const void* packed, int32_t* N, int32_t* K) {
+  if (!p || count < 1) return fail(IMQ_EINVAL, "at least one problem");
+  if (count > IMQ_PROMPT_MAX_PROBLEMS) return fail(IMQ_EUNSUPPORTED, "too many problems");
+  if (M < 1 || M > IMQ_PROMPT_MAX_ROWS) return fail(IMQ_EINVAL, "M out of range");
+  if (y_dtype != IMQ_BF16 && y_dtype != IMQ_F32) return fail(IMQ_EINVAL, "y_dtype must be bf16 or fp32");
+  if (!packed || !aligned(packed, 16)) return fail(IMQ_EINVAL, "packed rows must be non-null and 16-byte aligned");
+  for (int i = 0; i < count; ++i) {
+    const int32_t code = check_weight(p[i].w, p[i].scales, p[i].biases, p[i].N, p[i].K, group_size, bits);
+    if (code != IMQ_OK) return code;
+    if (p[i].K != p[0].K) return fail(IMQ_EINVAL, "the problems of one call share K");
+    if (!p[i].y || !aligned(p[i].y, y_dtype == IMQ_F32 ? 4 : 2)) return fail(IMQ_EINVAL, "y is null or misaligned");
+    if (p[i].ldy < p[i].N) return fail(IMQ_EINVAL, "ldy must be >= N");
+    N[i] = p[i].N;
+  }
+  *K = p[0].K;
+  return IMQ_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+size_t imq_prompt_packed_bytes(int32_t M, int32_t K) {
+  if (M < 1 || M > IMQ_PROMPT_MAX_ROWS || K < 64 || K % 64 || K > IMQ_PROMPT_MAX_K) return 0;
+  return packed_bytes(ceil_div(M, 32), K);
+}
+
+int32_t imq_prompt_pack(const uint16_t* x, int64_t ldx, int32_t M, int32_t K, void* packed, void* stream) {
+  if (!x || !packed) return fail(IMQ_EINVAL, "x and packed must be non-null");
+  if (M < 1 || M > IMQ_PROMPT_MAX_ROWS) return fail(IMQ_EINVAL, "M out of range");
+  if (K < 64 || K % 64 || K > IMQ_PROMPT_MAX_K) return fail(IMQ_EINVAL, "K must be a multiple of 64 in range");
+  if (ldx < K || ldx % 8) return fail(IMQ_EINVAL, "ldx must be >= K and a multiple of 8");
+  if (!aligned(x, 16) || !aligned(packed, 16)) return fail(IMQ_EINVAL, "x and packed must be 16-byte aligned");
+  int32_t code;
+  if (!current_device(&code)) return code;
+  pack_rows(x, ldx, nullptr, M, ceil_div(M, 32), K, packed, static_cast<hipStream_t>(stream));
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(IMQ_ELAUNCH, std::string("pack launch failed: ") + hipGetErrorString(e));
+  return ok();
+}
+
+size_t imq_prompt_product_workspace(const imq_problem* p, int32_t count, int32_t M) {
+  if (!p || count < 1 || count > IMQ_PROMPT_MAX_PROBLEMS || M < 1) return 0;
+  int32_t code, N[IMQ_PROMPT_MAX_PROBLEMS];
+  const DeviceInfo* dev = current_device(&code);
+  if (!dev) return 0;
+  for (int i = 0; i < count; ++i) N[i] = p[i].N;
+  const Plan plan = plan_product(N, count, M, p[0].K, dev->cu_count);
+  return plan.splits > 1 ? (size_t)plan.splits * M * plane_columns(N, count) * 4 : 0;
+}
+
+int32_t imq_prompt_product(const imq_problem* p, int32_t count, const void* packed, int32_t M, int32_t group_size,
+                           int32_t bits, int32_t y_dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  int32_t N[IMQ_PROMPT_MAX_PROBLEMS], K = 0;
+  int32_t code = check_product(p, count, M, group_size, bits, y_dtype, packed, N, &K);
+  if (code != IMQ_OK) return code;
+  const DeviceInfo* dev = current_device(&code);
+  if (!dev) return code;
+  const Plan plan = plan_product(N, count, M, K, dev->cu_count);
+  const int64_t cols = plane_columns(N, count);
+  const bool split = plan.splits > 1;
+  if (split && (!workspace || !aligned(workspace, 16) || workspace_bytes < (size_t)plan.splits * M * cols * 4))
+    return fail(IMQ_EINVAL, "the workspace is null, misaligned or too small");
+  ProductArgs a;
+  SumArgs sum;
+  memset(&a, 0, sizeof(a));
+  memset(&sum, 0, sizeof(sum));
+  a.count = sum.count = count;
+  int tile0 = 0, col0 = 0;
+  for (int i = 0; i < count; ++i) {
+    a.p[i] = ProductProblem{p[i].w, p[i].scales, p[i].biases, p[i].y, split ? col0 : p[i].ldy, N[i], tile0};
+    sum.p[i] = ProductProblem{nullptr, nullptr, nullptr, p[i].y, p[i].ldy, N[i], col0};
+    tile0 += ceil_div(N[i], kColumns);
+    col0 += (int)round_up(N[i], 4);
+  }
+  a.y_f32 = sum.y_f32 = y_dtype == IMQ_F32;
+  if (split) a.planes = static_cast<float*>(workspace);
+  a.plane_ld = cols;
+  a.plane_stride = cols * M;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if ((code = run_product(a, plan, packed, ceil_div(M, 32), M, K, st)) != IMQ_OK || !split) return code;
+  sum.planes = a.planes;
+  sum.plane_ld = cols;
+  sum.plane_stride = a.plane_stride;
+  sum.M = M;
+  sum.splits = plan.splits;
+  hipLaunchKernelGGL(sum_planes_kernel, dim3(ceil_div(cols * M, 4 * kThreads)), dim3(kThreads), 0, st, sum);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(IMQ_ELAUNCH, std::string("sum launch failed: ") + hipGetErrorString(e));
+  return ok();
+}
+
+size_t imq_prompt_matmul_workspace(int32_t M, int32_t N, int32_t K) {
+  const size_t packed = imq_prompt_packed_bytes(M, K);
+  if (!packed || N < 1) return 0;
+  imq_problem p;
+  memset(&p, 0, sizeof(p));
+  p.N = N;
+  p.K = K;
+  return round_up(packed, 256) + imq_prompt_product_workspace(&p, 1, M);
+}
+
+int32_t imq_prompt_matmul(const uint32_t* w, const uint16_t* scales, const uint16_t* biases, const uint16_t* x,
+                          int64_t ldx, void* y, int64_t ldy, int32_t M, int32_t N, int32_t K, int32_t group_size,
+                          int32_t bits, int32_t y_dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  const imq_problem p = {w, scales, biases, nullptr, 0, y, ldy, N, K};
+  int32_t n, k, code = check_product(&p, 1, M, group_size, bits, y_dtype, workspace, &n, &k);
+  if (code != IMQ_OK) return code;
+  const size_t packed = round_up(imq_prompt_packed_bytes(M, K), 256);
+  if (workspace_bytes < packed) return fail(IMQ_EINVAL, "the workspace is too small");
+  if ((code = imq_prompt_pack(x, ldx, M, K, workspace, stream)) != IMQ_OK) return code;
+  return imq_prompt_product(&p, 1, workspace, M, group_size, bits, y_dtype, static_cast<char*>(workspace) + packed,
+                            workspace_bytes - packed, stream);
+}
+
+}  // extern "C"

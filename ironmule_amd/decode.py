@@ -32,8 +32,8 @@ head (or one launch per stage), with every RMSNorm but the first layer's input n
 into the projections around it.
 
 `prefill` runs a whole prompt through the same model at once, the library path a prompt
-takes (ironmule/cuda_native.py:171-179): every projection of more than 32 rows is
-imq_dequant to fp16 and one GEMM, attention is causal over the prompt in fp32, the KV
+takes (ironmule/cuda_native.py:171-179): every projection of more than 32 rows is one
+product on the packed weight (include/ironmule_prompt.h), attention is causal over the prompt in fp32, the KV
 pools of the request's slot are written for positions 0..T-1, and the head is computed
 for the last position only (ironmule/cuda_native.py:271-303, `head_skip_prefill`).
 """
@@ -358,13 +358,12 @@ def _rotary(x: torch.Tensor, positions: torch.Tensor, theta: float) -> torch.Ten
 
 
 def _project(x: torch.Tensor, quant: Quant, stream=None) -> torch.Tensor:
-    """bf16 rows times a 4-bit weight: the qmv kernel up to 32 rows, else imq_dequant to
-    fp16 and one GEMM (fp16 products, fp32 accumulation), rounded to bf16."""
+    """bf16 rows times a 4-bit weight: the qmv kernel up to 32 rows, else the prompt product
+    (on the current stream, which prefill has made `stream`); fp32 sums, rounded to bf16."""
     w, s, b = quant
     if x.shape[0] <= _native.MAX_ROWS:
         return _native.qmv(w, s, b, x, stream=stream)
-    dense = _native.dequant(w, s, b, torch.float16, stream=stream)
-    return torch.matmul(x.to(torch.float16), dense.T).to(torch.bfloat16)
+    return _native.prompt_matmul(w, s, b, x)
 
 
 def prefill(weights: DecoderWeights, state: DecodeState, tokens, slot: int,

@@ -13,7 +13,8 @@ Which path a call takes (`_route`, `_gather_route`):
 call                                                  path
 ====================================================  =====================================
 bf16 x with at most MAX_ROWS (32) rows                imq_qmv, one weight sweep for all rows
-bf16 x with more rows (prefill)                       imq_dequant to fp16, one GEMM
+bf16 x with more rows (prefill)                       imq_prompt_matmul on the packed weight
+the same where autograd or a transform needs it       imq_dequant to fp16, one GEMM
 expert call, one bf16 row per (token, expert) pair,   imq_gather_qmv
 at most GATHER_MAX pairs
 anything else (fp32 x, larger expert batches)         the module's library path
@@ -60,7 +61,9 @@ _MEMORY_KEYS = ("total_memory", "memory_size", "total_memory_bytes", "memory_byt
 def _route(x: torch.Tensor, k: int) -> str:
     if x.dtype != torch.bfloat16:
         return "library"
-    return "qmv" if x.numel() // k <= MAX_ROWS else "dequant_gemm"
+    if x.numel() // k <= MAX_ROWS:
+        return "qmv"
+    return "prompt" if _native.takes_prompt(x, k) else "dequant_gemm"
 
 
 def _qmv(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
@@ -77,6 +80,9 @@ def matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor,
     route = _route(x, int(w.shape[1]) * 8)
     if route == "qmv":
         return _qmv(x, w, scales, biases)
+    if route == "prompt":
+        n, k = int(w.shape[0]), int(w.shape[1]) * 8
+        return _native.prompt_matmul(w, scales, biases, x).reshape(*x.shape[:-1], n)
     if route == "dequant_gemm":
         weight16 = _native.dequant(w, scales, biases, torch.float16)
         return torch.matmul(x.to(torch.float16), weight16.T).to(x.dtype)

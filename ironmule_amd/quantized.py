@@ -8,8 +8,9 @@ bf16 scales and biases, group size, bits), and a library path that runs on the G
 
 * up to 32 activation rows: the qmv kernel (libironmule_qmv.so, imq_qmv), as MLX's own
   `quantized_matmul` runs its qmv kernel for few rows;
-* more rows (prefill): the weight dequantised by imq_dequant, then a torch GEMM
-  (hipBLASLt), as the reference's prefill does (ironmule/cuda_native.py:177-179).
+* more rows (prefill): one product on the packed weight (imq_prompt_matmul) where the
+  reference's prefill dequantises first (ironmule/cuda_native.py:177-179); other types, and
+  calls that autograd or a transform follows, dequantise and take a torch GEMM.
 
 There is no CPU path: the forward fails loudly without a GPU and the HIP library.
 
@@ -118,7 +119,8 @@ class QuantizedEmbedding(torch.nn.Module):
 
 def library_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
                    group_size: int = GROUP_SIZE, bits: int = BITS) -> torch.Tensor:
-    """The library path: qmv for up to 32 bf16 rows, dequantise + GEMM beyond."""
+    """The library path: qmv for up to 32 bf16 rows, the prompt product beyond, and dequantise
+    + GEMM for other types and for calls autograd or a transform follows."""
     if group_size != GROUP_SIZE or bits != BITS:
         raise ValueError("only 4-bit, group-64 weights are supported")
     if not x.is_cuda:
@@ -128,6 +130,8 @@ def library_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biase
     rows = x.reshape(-1, k)
     if x.dtype == torch.bfloat16 and rows.shape[0] <= _native.MAX_ROWS:
         y = _native.qmv(w, scales, biases, rows.contiguous())
+    elif _native.takes_prompt(x, k):
+        y = _native.prompt_matmul(w, scales, biases, rows)
     else:
         dense = _native.dequant(w, scales, biases, torch.float32)
         y = (rows.to(torch.float32) @ dense.T).to(x.dtype)

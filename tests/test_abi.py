@@ -185,3 +185,38 @@ def test_workspace_keys_follow_the_current_stream(monkeypatch):
     explicit = _native._workspace_key("cuda:0", SimpleNamespace(cuda_stream=0x2000))
     assert explicit == second
     assert _native._workspace_key("cuda:1", None)[0] == 1
+
+
+def _prompt(lib, **over):
+    args = dict(w=1 << 20, s=1 << 20, b=1 << 20, x=1 << 20, ldx=2560, y=1 << 20, ldy=2560, M=64, N=2560, K=2560,
+                gs=64, bits=4, dtype=0, ws=1 << 20, nbytes=1 << 30)
+    args.update(over)
+    P = ctypes.c_void_p
+    return lib.imq_prompt_matmul(P(args["w"]), P(args["s"]), P(args["b"]), P(args["x"]), args["ldx"], P(args["y"]),
+                                 args["ldy"], args["M"], args["N"], args["K"], args["gs"], args["bits"],
+                                 args["dtype"], P(args["ws"]), args["nbytes"], None)
+
+
+@pytest.mark.parametrize("over,code", [
+    ({"bits": 8}, _native.IMQ_EUNSUPPORTED),
+    ({"gs": 128}, _native.IMQ_EUNSUPPORTED),
+    ({"K": 100}, _native.IMQ_EINVAL),
+    ({"K": (1 << 17) + 64}, _native.IMQ_EUNSUPPORTED),
+    ({"N": 0}, _native.IMQ_EINVAL),
+    ({"M": 0}, _native.IMQ_EINVAL),
+    ({"M": (1 << 20) + 1}, _native.IMQ_EINVAL),
+    ({"w": 0}, _native.IMQ_EINVAL),
+    ({"w": (1 << 20) + 4}, _native.IMQ_EINVAL),
+    ({"x": 0}, _native.IMQ_EINVAL),
+    ({"x": (1 << 20) + 2}, _native.IMQ_EINVAL),
+    ({"ldx": 2564}, _native.IMQ_EINVAL),
+    ({"ldy": 100}, _native.IMQ_EINVAL),
+    ({"y": 0}, _native.IMQ_EINVAL),
+    ({"dtype": 2}, _native.IMQ_EINVAL),
+    ({"ws": 0}, _native.IMQ_EINVAL),
+    ({"nbytes": 1024}, _native.IMQ_EINVAL),
+])
+def test_malformed_prompt_calls_are_refused_with_codes(lib, over, code):
+    assert _prompt(lib, **over) == code
+    got, msg = _native.last_error()
+    assert got == code and msg

@@ -1,0 +1,124 @@
+"""GPU parity of the product for more than 32 rows (imq_prompt_matmul, imq_prompt_product)
+through the C ABI, against the oracle's float64 product.
+
+Bars (the qmv kernels'): fp32 outputs within 2^-20 sum|w x| + 2^-23 |ref|, bf16 outputs within
+one ulp of the rounded reference plus that allowance.  Sizes: one row past a 32-row block,
+blocks that a tile of 64 or 128 rows fills in part, N off the 128 columns of a workgroup, K of
+one group, groups off the chunks of four (scales of every alignment), and K-ranges.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from tests.conftest import gpu_available
+from tests.gpu_util import announce, bf16_bits, to_device
+
+pytestmark = [pytest.mark.gpu,
+              pytest.mark.skipif(not gpu_available(), reason="needs a ROCm GPU")]
+
+
+@pytest.fixture(scope="module")
+def env():
+    import torch
+
+    from ironmule_amd import _native
+    from oracle import oracle as orc
+    code, arch, _ = _native.device_check()
+    assert code == 0, f"device {arch} is not supported"
+    orc.lib()
+    return torch, _native, orc
+
+
+SIZES = [(33, 64, 64), (40, 130, 192), (65, 1, 256), (97, 300, 320), (129, 257, 1600), (77, 512, 9728),
+         (200, 2560, 256), (512, 384, 2560), (600, 4100, 768)]
+
+
+@pytest.mark.parametrize("m,n,k", SIZES)
+def test_prompt_matmul_against_the_oracle(env, m, n, k):
+    torch, n_, orc = env
+    announce("prompt", m, n, k)
+    pr = orc.synthetic(n, k, m, seed=orc.SEED_BASE + 900 + m)
+    w, s, b, x = to_device(pr)
+    ref, mag = orc.qmv_f64(pr.w, pr.s, pr.b, pr.x)
+    verdict = orc.check_f32(n_.prompt_matmul(w, s, b, x, torch.float32).cpu().numpy(), ref, mag)
+    assert verdict.ok, verdict.detail
+    got = n_.prompt_matmul(w, s, b, x)
+    verdict = orc.check_bf16(bf16_bits(got), ref, mag)
+    assert verdict.ok, verdict.detail
+    assert torch.equal(got, n_.prompt_matmul(w, s, b, x))  # no order of arrival in any sum
+
+
+def test_rows_and_scales_of_any_alignment(env):
+    """x rows with a stride and rows off a 16-byte boundary, scales off an 8-byte boundary."""
+    torch, n_, orc = env
+    announce("prompt alignment")
+    m, n, k = 70, 200, 512
+    pr = orc.synthetic(n, k, m, seed=orc.SEED_BASE + 930)
+    w, s, b, x = to_device(pr)
+    want = n_.prompt_matmul(w, s, b, x)
+    wide = torch.zeros((m, k + 72), dtype=torch.bfloat16, device="cuda")
+    for at in (0, 8, 3):
+        wide[:, at:at + k] = x
+        assert torch.equal(n_.prompt_matmul(w, s, b, wide[:, at:at + k]), want), at
+    odd = torch.empty(s.numel() + 1, dtype=torch.bfloat16, device="cuda")[1:].view_as(s)
+    odd.copy_(s)
+    assert torch.equal(n_.prompt_matmul(w, odd, b, x), want)
+
+
+def test_infinities_nan_and_large_values_stay_in_their_rows(env):
+    """A row whose values could overflow the group sums is computed value by value: infinities
+    keep their sign, NaN stays NaN, 1e38 gives the finite result, and other rows keep their bits."""
+    torch, n_, orc = env
+    announce("prompt non-finite rows")
+    m, n, k = 100, 200, 320
+    w, s, b, x = to_device(orc.synthetic(n, k, m, seed=orc.SEED_BASE + 940))
+    clean = n_.prompt_matmul(w, s, b, x, torch.float32)
+    x[5, 7], x[50, 100], x[64, 319], x[99, 0] = float("inf"), float("nan"), -float("inf"), 1e38
+    y = n_.prompt_matmul(w, s, b, x, torch.float32).double()
+    ref = x.double() @ n_.dequant(w, s, b).double().T
+    touched = [5, 50, 64, 99]
+    others = [r for r in range(m) if r not in touched]
+    assert torch.equal(y[others], clean[others].double())
+    assert torch.equal(torch.isnan(y), torch.isnan(ref))
+    inf = torch.isinf(ref)
+    assert inf.any() and torch.equal(y[inf], ref[inf])
+    # the 1e38 row: one term dominates, fp32 rounding of 320 terms
+    assert ((y[99] - ref[99]).abs() <= 320 * 2.0**-24 * (x[99].double().abs() @ n_.dequant(w, s, b).double().abs().T)).all()
+
+
+def test_grouped_products_share_one_packing(env):
+    """Three weights of one K, N off multiples of four and of 128, over one packing."""
+    import ctypes
+    torch, n_, orc = env
+    announce("prompt grouped")
+    m, k, sizes = 161, 1024, (300, 131, 64)
+    probs = [orc.synthetic(n, k, m, seed=orc.SEED_BASE + 950 + n) for n in sizes]
+    x = to_device(probs[0])[3]
+    weights = [to_device(p)[:3] for p in probs]
+    lib = n_.lib()
+    packed = torch.empty(lib.imq_prompt_packed_bytes(m, k), dtype=torch.uint8, device="cuda")
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert lib.imq_prompt_pack(x.data_ptr(), k, m, k, packed.data_ptr(), stream) == 0
+    outs = [torch.empty((m, n), dtype=torch.float32, device="cuda") for n in sizes]
+    arr = (n_.Problem * 3)(*[n_.Problem(w.data_ptr(), s.data_ptr(), b.data_ptr(), None, 0, y.data_ptr(), n, n, k)
+                             for (w, s, b), y, n in zip(weights, outs, sizes)])
+    ws = torch.empty(lib.imq_prompt_product_workspace(arr, 3, m) + 16, dtype=torch.uint8, device="cuda")
+    assert lib.imq_prompt_product(arr, 3, packed.data_ptr(), m, 64, 4, n_.IMQ_F32, ws.data_ptr(), ws.numel(), stream) == 0
+    for p, y in zip(probs, outs):
+        ref, mag = orc.qmv_f64(p.w, p.s, p.b, probs[0].x)
+        verdict = orc.check_f32(y.cpu().numpy(), ref, mag)
+        assert verdict.ok, verdict.detail
+
+
+def test_calls_that_autograd_follows_keep_the_torch_product(env):
+    torch, n_, orc = env
+    from ironmule_amd import hip_native
+    announce("prompt autograd")
+    w, s, b, x = to_device(orc.synthetic(64, 128, 40, seed=orc.SEED_BASE + 960))
+    x.requires_grad_(True)
+    hip_native.matmul(x, w, s, b).float().sum().backward()
+    dense = n_.dequant(w, s, b)
+    want = dense.sum(dim=0).expand(40, 128)
+    assert (x.grad.float() - want).abs().max() <= 2.0**-7 * want.abs().max()  # fp16 weights, bf16 gradient
