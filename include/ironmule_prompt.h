@@ -23,6 +23,7 @@ extern "C" {
 #endif
 
 #define IMQ_PROMPT_MAX_PROBLEMS 3
+#define IMQ_PROMPT_MAX_EXPERTS 1024
 #define IMQ_PROMPT_MAX_ROWS (1 << 20)
 #define IMQ_PROMPT_MAX_K (1 << 17)
 
@@ -53,6 +54,21 @@ IMQ_API int32_t imq_prompt_matmul(const uint32_t* w, const uint16_t* scales, con
                                   const uint16_t* x, int64_t ldx, void* y, int64_t ldy, int32_t M, int32_t N,
                                   int32_t K, int32_t group_size, int32_t bits, int32_t y_dtype, void* workspace,
                                   size_t workspace_bytes, void* stream);
+
+/* Bytes of workspace imq_prompt_experts takes (0: a size out of range). */
+IMQ_API size_t imq_prompt_experts_workspace(int32_t experts, int32_t pairs, int32_t K);
+
+/* y[p] = x[p / rows_per_x] W[idx[p]]^T for `pairs` (token, expert) pairs over stacked expert
+ * weights (E, N, K/8), scales and biases (E, N, K/64): the pairs are sorted by expert on the
+ * device, each expert's rows taken together.  An index below zero counts from the last expert;
+ * a pair whose index is outside the stack gets zeros.  The workspace (16-byte aligned) needs no
+ * preparation.
+ * Replaces mx.gather_qmm beyond the gather kernel's pairs (ironmule/cuda_native.py:199-218). */
+IMQ_API int32_t imq_prompt_experts(const uint32_t* w, const uint16_t* scales, const uint16_t* biases,
+                                   int32_t experts, const uint16_t* x, int64_t ldx, int32_t rows_per_x,
+                                   const int32_t* idx, int32_t pairs, void* y, int64_t ldy, int32_t N, int32_t K,
+                                   int32_t group_size, int32_t bits, int32_t y_dtype, void* workspace,
+                                   size_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }

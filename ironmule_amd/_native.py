@@ -161,6 +161,9 @@ _SIGNATURES = {
     "imq_prompt_matmul_workspace": ([_I32, _I32, _I32], ctypes.c_size_t),
     "imq_prompt_matmul": ([_P, _P, _P, _P, _I64, _P, _I64, _I32, _I32, _I32, _I32, _I32, _I32, _P, ctypes.c_size_t,
                            _P], _I32),
+    "imq_prompt_experts_workspace": ([_I32, _I32, _I32], ctypes.c_size_t),
+    "imq_prompt_experts": ([_P, _P, _P, _I32, _P, _I64, _I32, _P, _I32, _P, _I64, _I32, _I32, _I32, _I32, _I32, _P,
+                            ctypes.c_size_t, _P], _I32),
     # persistent programs (include/ironmule_step.h)
     "imq_decode_program_create": ([ctypes.POINTER(StepDesc), ctypes.POINTER(_P)], _I32),
     "imq_qmv_program_create": ([ctypes.POINTER(QmvStage), _I32, ctypes.POINTER(_P)], _I32),
@@ -470,6 +473,7 @@ def dequant(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
 
 MAX_PROMPT_ROWS = 1 << 20
 MAX_PROMPT_K = 1 << 17
+MAX_PROMPT_EXPERTS = 1024
 
 
 def takes_prompt(x: torch.Tensor, k: int) -> bool:
@@ -509,6 +513,32 @@ def prompt_matmul(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor, x
     ws = torch.empty(nbytes, dtype=torch.uint8, device=w.device)
     _check(lib().imq_prompt_matmul(_ptr(w), _ptr(scales), _ptr(biases), _ptr(x2), ld, _ptr(out), n, m, n, k,
                                    GROUP_SIZE, BITS, _DTYPE_CODE[out_dtype], _ptr(ws), nbytes, _stream(None)))
+    return out
+
+
+def prompt_experts(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor, x: torch.Tensor,
+                   idx: torch.Tensor, rows_per_x: int = 1, out_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
+    """y[p] = x[p // rows_per_x] @ dequantize(w[idx[p]]).T for any number of (token, expert)
+    pairs (imq_prompt_experts), the pairs sorted by expert on the device; w (E, N, K/8), scales
+    and biases (E, N, K/64), x bf16 rows, idx integers on the device (negative ones count from
+    the last expert).  Returns (pairs, N), on the current stream."""
+    if w.dim() != 3 or scales.dim() != 3 or biases.dim() != 3:
+        raise ValueError("w, scales and biases must be stacked by expert")
+    e, n = int(w.shape[0]), int(w.shape[1])
+    k = check_weights(*(t.view(e * n, -1) for t in (w, scales, biases)))[1]
+    if x.dtype != torch.bfloat16 or int(x.shape[-1]) != k:
+        raise ValueError(f"x must be bf16 rows of {k} values")
+    x2, ld = _aligned_rows(x, k)
+    idx = idx.reshape(-1).to(torch.int32).contiguous()
+    pairs = int(idx.numel())
+    if pairs < 1 or rows_per_x < 1 or -(-pairs // rows_per_x) > x2.shape[0]:
+        raise ValueError("need at least one pair and ceil(pairs / rows_per_x) activation rows")
+    out = torch.empty((pairs, n), dtype=out_dtype, device=w.device)
+    nbytes = int(lib().imq_prompt_experts_workspace(e, pairs, k))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=w.device)
+    _check(lib().imq_prompt_experts(_ptr(w), _ptr(scales), _ptr(biases), e, _ptr(x2), ld, int(rows_per_x), _ptr(idx),
+                                    pairs, _ptr(out), n, n, k, GROUP_SIZE, BITS, _DTYPE_CODE[out_dtype], _ptr(ws),
+                                    nbytes, _stream(None)))
     return out
 
 

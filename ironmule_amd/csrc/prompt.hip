@@ -89,15 +89,18 @@ __device__ __forceinline__ void pack_piece(uint4 d, int piece, int row, char* im
 }
 
 // One workgroup per (chunk, block).  `src` (may be null): the x row of each packed row, -1 for
-// a row of zeros; without it packed row r is x row r, zeros past M.
+// a row of zeros, and `expert` the expert of each tile of `tm` blocks, -1 for tiles not in use;
+// without them packed row r is x row r, zeros past M.
 __global__ __launch_bounds__(kThreads) void pack_rows_kernel(const uint16_t* __restrict__ x, int64_t ldx,
-                                                             const int32_t* __restrict__ src, int M, int K,
+                                                             const int32_t* __restrict__ src,
+                                                             const int32_t* __restrict__ expert, int tm, int M, int K,
                                                              char* __restrict__ packed,
                                                              uint32_t* __restrict__ flags) {
   __shared__ __attribute__((aligned(16))) char image[kChunkBytes];
   __shared__ uint32_t flag;
   const int chunk = blockIdx.x, block = blockIdx.y, chunks = gridDim.x;
   const int tid = threadIdx.x, piece = tid & 31;
+  if (expert && expert[block / tm] < 0) return;
   if (tid == 0) flag = 0u;
   const int col = 256 * chunk + 8 * piece;
   uint4 d[4];
@@ -142,7 +145,7 @@ __global__ __launch_bounds__(kThreads) void pack_rows_kernel(const uint16_t* __r
 // LDS reads, twice the unpacking) and eight wavefronts over 256 columns measured the same;
 // 128 x 64 per wavefront 930 TFLOP/s on large launches, but its 256-column tiles leave a
 // prompt of 512 rows with too few workgroups.  Against imq_dequant and a library product (two
-// conversions of the activations besides): 1024 x 9728 x 2560 89.7 -> 79.5 us in fp16, 77 x
+// conversions of the activations besides): 1024 x 9728 x 2560 89.7 -> 81.3 us in fp16, 77 x
 // 2560 x 9728 70.9 -> 27.6 us in fp32.
 struct ProductProblem {
   const uint32_t* w;
@@ -353,13 +356,14 @@ __global__ __launch_bounds__(kThreads, 2) void product_kernel(ProductArgs a) {
         scale_unit(s[i & 1], p[at ^ 1], u - 1);
 #pragma unroll
       for (int k = u * 4 / TM; k < (u + 1) * 4 / TM; ++k) unpack(i < 3 ? wq[(i + 1) & 3] : nwq[0], k, wb[(i & 1) ^ 1]);
-      if (i == 3) {  // the chunk's group sums against its biases and scales
-        const int m = TM > 2 ? (u + 2) % TM : u;
-        const bf16x8_t u0 = __builtin_bit_cast(bf16x8_t, xsum[m * 128 + h * 32 + n]);
-        const bf16x8_t u1 = __builtin_bit_cast(bf16x8_t, xsum[m * 128 + 64 + h * 32 + n]);
+      if (i == 3) {
+        // the chunk's group sums against its biases and scales, between the tile's third and
+        // fourth groups: one order for every row, so its bits do not depend on its place
+        const bf16x8_t u0 = __builtin_bit_cast(bf16x8_t, xsum[u * 128 + h * 32 + n]);
+        const bf16x8_t u1 = __builtin_bit_cast(bf16x8_t, xsum[u * 128 + 64 + h * 32 + n]);
         const bf16x8_t c = __builtin_bit_cast(bf16x8_t, u32x4_t{bi.x, bi.y, sc.x, sc.y});
-        acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(u0, c, acc[m], 0, 0, 0);
-        acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(u1, c, acc[m], 0, 0, 0);
+        acc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(u0, c, acc[u], 0, 0, 0);
+        acc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(u1, c, acc[u], 0, 0, 0);
       }
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
@@ -504,6 +508,63 @@ __global__ __launch_bounds__(kThreads) void sum_planes_kernel(SumArgs a) {
   }
 }
 
+// ------------------------------------------------------------ rows sorted by expert
+
+// One workgroup: counts the pairs of each expert, gives every expert whole tiles of `tile`
+// packed rows, and writes each packed row's source row (pair / rows_per_x) and output row
+// (the pair), -1 for the rows that fill up a tile, and each tile's expert, -1 past the last.
+// An index below zero counts from the last expert; a pair whose index is outside the stack
+// becomes a row of zeros.  The order of an expert's pairs within its tiles is not fixed, and no
+// output depends on it: a row's sums involve no other row.  Bound by its own round trips (one
+// CU, two passes over the indices).  With it 1024 pairs of 32 experts of 2560 x 768 take 41 us in
+// place of 14.2 ms (every pair's expert dequantised to fp32 and one batched product).
+constexpr int kSortThreads = 1024;
+__global__ __launch_bounds__(kSortThreads) void sort_pairs_kernel(const int32_t* __restrict__ idx, int pairs,
+                                                                  int experts, int rows_per_x, int tile, int tiles,
+                                                                  int32_t* __restrict__ src,
+                                                                  int32_t* __restrict__ dest,
+                                                                  int32_t* __restrict__ tile_expert) {
+  __shared__ int32_t count[IMQ_PROMPT_MAX_EXPERTS];
+  __shared__ int32_t first[IMQ_PROMPT_MAX_EXPERTS];
+  __shared__ int32_t scan[kSortThreads];
+  const int tid = threadIdx.x;
+  count[tid] = 0;
+  __syncthreads();
+  for (int p = tid; p < pairs; p += kSortThreads) {
+    int e = idx[p];
+    if (e < 0) e += experts;
+    atomicAdd(&count[e >= 0 && e < experts ? e : 0], 1);
+  }
+  __syncthreads();
+  const int mine = count[tid], need = (mine + tile - 1) / tile;
+  scan[tid] = need;
+  __syncthreads();
+  for (int d = 1; d < kSortThreads; d <<= 1) {
+    const int add = tid >= d ? scan[tid - d] : 0;
+    __syncthreads();
+    scan[tid] += add;
+    __syncthreads();
+  }
+  const int tile0 = scan[tid] - need;
+  first[tid] = tile0 * tile;
+  for (int i = 0; i < need; ++i) tile_expert[tile0 + i] = tid;
+  for (int r = mine; r < need * tile; ++r) {
+    src[tile0 * tile + r] = -1;
+    dest[tile0 * tile + r] = -1;
+  }
+  const int used = scan[kSortThreads - 1];
+  for (int i = used + tid; i < tiles; i += kSortThreads) tile_expert[i] = -1;
+  __syncthreads();
+  for (int p = tid; p < pairs; p += kSortThreads) {
+    int e = idx[p];
+    if (e < 0) e += experts;
+    const bool in = e >= 0 && e < experts;
+    const int at = atomicAdd(&first[in ? e : 0], 1);
+    src[at] = in ? p / rows_per_x : -1;
+    dest[at] = p;
+  }
+}
+
 // ------------------------------------------------------------ host side
 
 int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
@@ -547,6 +608,22 @@ Plan plan_product(const int32_t* N, int count, int M, int K, int cus) {
   return plan;
 }
 
+// Tiles for rows sorted by expert: at most pairs / (32 tm) full ones and a part-full one per
+// expert.  The tile height follows the pairs an expert gets on average: short tiles while most
+// of a taller one would be rows of zeros.
+struct ExpertPlan {
+  int tm, tiles, blocks;
+};
+
+ExpertPlan plan_experts(int experts, int pairs) {
+  const int used = experts < pairs ? experts : pairs;
+  ExpertPlan p;
+  p.tm = pairs <= 40 * used ? 1 : pairs <= 160 * used ? 2 : 4;
+  p.tiles = pairs / (32 * p.tm) + used;
+  p.blocks = p.tiles * p.tm;
+  return p;
+}
+
 size_t flag_bytes(int64_t blocks, int chunks) { return round_up((size_t)blocks * chunks * 4, 256); }
 
 size_t packed_bytes(int64_t blocks, int K) {
@@ -554,11 +631,11 @@ size_t packed_bytes(int64_t blocks, int K) {
   return flag_bytes(blocks, chunks) + (size_t)blocks * chunks * kChunkBytes;
 }
 
-void pack_rows(const uint16_t* x, int64_t ldx, const int32_t* src, int M, int64_t blocks, int K, void* packed,
-               hipStream_t stream) {
+void pack_rows(const uint16_t* x, int64_t ldx, const int32_t* src, const int32_t* expert, int tm, int M,
+               int64_t blocks, int K, void* packed, hipStream_t stream) {
   const int chunks = ceil_div(K, 256);
   char* const base = static_cast<char*>(packed);
-  hipLaunchKernelGGL(pack_rows_kernel, dim3(chunks, (uint32_t)blocks), dim3(kThreads), 0, stream, x, ldx, src, M, K,
+  hipLaunchKernelGGL(pack_rows_kernel, dim3(chunks, (uint32_t)blocks), dim3(kThreads), 0, stream, x, ldx, src, expert, tm, M, K,
                      base + flag_bytes(blocks, chunks), reinterpret_cast<uint32_t*>(base));
 }
 
@@ -655,7 +732,7 @@ int32_t imq_prompt_pack(const uint16_t* x, int64_t ldx, int32_t M, int32_t K, vo
   if (!aligned(x, 16) || !aligned(packed, 16)) return fail(IMQ_EINVAL, "x and packed must be 16-byte aligned");
   int32_t code;
   if (!current_device(&code)) return code;
-  pack_rows(x, ldx, nullptr, M, ceil_div(M, 32), K, packed, static_cast<hipStream_t>(stream));
+  pack_rows(x, ldx, nullptr, nullptr, 1, M, ceil_div(M, 32), K, packed, static_cast<hipStream_t>(stream));
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(IMQ_ELAUNCH, std::string("pack launch failed: ") + hipGetErrorString(e));
   return ok();
@@ -733,6 +810,52 @@ int32_t imq_prompt_matmul(const uint32_t* w, const uint16_t* scales, const uint1
   if ((code = imq_prompt_pack(x, ldx, M, K, workspace, stream)) != IMQ_OK) return code;
   return imq_prompt_product(&p, 1, workspace, M, group_size, bits, y_dtype, static_cast<char*>(workspace) + packed,
                             workspace_bytes - packed, stream);
+}
+
+size_t imq_prompt_experts_workspace(int32_t experts, int32_t pairs, int32_t K) {
+  if (experts < 1 || experts > IMQ_PROMPT_MAX_EXPERTS || pairs < 1 || pairs > IMQ_PROMPT_MAX_ROWS || K < 64 ||
+      K % 64 || K > IMQ_PROMPT_MAX_K)
+    return 0;
+  const ExpertPlan p = plan_experts(experts, pairs);
+  return round_up((size_t)p.tiles * 4, 256) + 2 * round_up((size_t)p.blocks * 32 * 4, 256) + packed_bytes(p.blocks, K);
+}
+
+int32_t imq_prompt_experts(const uint32_t* w, const uint16_t* scales, const uint16_t* biases, int32_t experts,
+                           const uint16_t* x, int64_t ldx, int32_t rows_per_x, const int32_t* idx, int32_t pairs,
+                           void* y, int64_t ldy, int32_t N, int32_t K, int32_t group_size, int32_t bits,
+                           int32_t y_dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  const imq_problem one = {w, scales, biases, nullptr, 0, y, ldy, N, K};
+  int32_t n, k, code = check_product(&one, 1, pairs, group_size, bits, y_dtype, workspace, &n, &k);
+  if (code != IMQ_OK) return code;
+  if (experts < 1) return fail(IMQ_EINVAL, "experts must be >= 1");
+  if (experts > IMQ_PROMPT_MAX_EXPERTS) return fail(IMQ_EUNSUPPORTED, "too many experts");
+  if (!x || !idx || !aligned(x, 16) || !aligned(idx, 4)) return fail(IMQ_EINVAL, "x or idx is null or misaligned");
+  if (ldx < K || ldx % 8) return fail(IMQ_EINVAL, "ldx must be >= K and a multiple of 8");
+  if (rows_per_x < 1) return fail(IMQ_EINVAL, "rows_per_x must be >= 1");
+  if (workspace_bytes < imq_prompt_experts_workspace(experts, pairs, K))
+    return fail(IMQ_EINVAL, "the workspace is too small");
+  if (!current_device(&code)) return code;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const ExpertPlan e = plan_experts(experts, pairs);
+  char* at = static_cast<char*>(workspace);
+  int32_t* const tile_expert = reinterpret_cast<int32_t*>(at);
+  at += round_up((size_t)e.tiles * 4, 256);
+  int32_t* const src = reinterpret_cast<int32_t*>(at);
+  at += round_up((size_t)e.blocks * 32 * 4, 256);
+  int32_t* const dest = reinterpret_cast<int32_t*>(at);
+  at += round_up((size_t)e.blocks * 32 * 4, 256);
+  hipLaunchKernelGGL(sort_pairs_kernel, dim3(1), dim3(kSortThreads), 0, st, idx, pairs, experts, rows_per_x,
+                     32 * e.tm, e.tiles, src, dest, tile_expert);
+  pack_rows(x, ldx, src, tile_expert, e.tm, 0, e.blocks, K, at, st);
+  ProductArgs a;
+  memset(&a, 0, sizeof(a));
+  a.p[0] = ProductProblem{w, scales, biases, y, ldy, N, 0};
+  a.count = 1;
+  a.y_f32 = y_dtype == IMQ_F32;
+  a.expert = tile_expert;
+  a.dest = dest;
+  const Plan p = {e.tm, 1, ceil_div(K, 256), e.tiles, ceil_div(N, kColumns)};
+  return run_product(a, p, at, e.blocks, pairs, K, st);
 }
 
 }  // extern "C"

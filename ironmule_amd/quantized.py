@@ -167,14 +167,28 @@ class QuantizedSwitchLinear(torch.nn.Module):
 def library_gather_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor,
                           biases: torch.Tensor, indices: torch.Tensor,
                           group_size: int = GROUP_SIZE, bits: int = BITS) -> torch.Tensor:
-    """The library gather path: every selected expert dequantised to fp32 and one batched
-    product, (*batch, M, K) x experts -> (*batch, M, N), batch = broadcast(x.shape[:-2],
-    indices.shape)."""
+    """The library gather path, (*batch, M, K) x experts -> (*batch, M, N), batch =
+    broadcast(x.shape[:-2], indices.shape): bf16 rows sorted by expert and multiplied on the
+    packed weights (_native.prompt_experts); otherwise, and where autograd or a transform
+    follows the call, every selected expert dequantised to fp32 and one batched product."""
     if group_size != GROUP_SIZE or bits != BITS:
         raise ValueError("only 4-bit, group-64 weights are supported")
     if not x.is_cuda:
         raise _native.NativeUnavailable("the quantised layers run on the GPU only")
     batch = torch.broadcast_shapes(x.shape[:-2], indices.shape)
+    k, n, rows = int(w.shape[-1]) * 8, int(w.shape[1]), int(x.shape[-2])
+    pairs = batch.numel() * rows
+    if (_native.takes_prompt(x, k) and 1 <= pairs <= _native.MAX_PROMPT_ROWS and not indices.is_floating_point()
+            and indices.dtype != torch.bool and indices.is_cuda and x.shape[-1] == k
+            and 1 <= w.shape[0] <= _native.MAX_PROMPT_EXPERTS):
+        lead, idx, per = tuple(x.shape[:-2]), indices.expand(batch), 1
+        if rows == 1 and batch and lead == tuple(batch[:-1]) + (1,):
+            per = int(batch[-1])  # a token's row shared by its experts
+        elif lead != tuple(batch):
+            x = x.expand(*batch, *x.shape[-2:])
+        if rows > 1:
+            idx = idx.reshape(-1).repeat_interleave(rows)
+        return _native.prompt_experts(w, scales, biases, x, idx, per).reshape(*batch, rows, n)
     xb = x.expand(*batch, *x.shape[-2:]).reshape(-1, x.shape[-2], x.shape[-1])
     idx = indices.expand(batch).reshape(-1).to(torch.long)
     dense = _native.dequant(w[idx].reshape(-1, w.shape[-1]).contiguous(),

@@ -32,7 +32,7 @@ def env():
 
 
 SIZES = [(33, 64, 64), (40, 130, 192), (65, 1, 256), (97, 300, 320), (129, 257, 1600), (77, 512, 9728),
-         (200, 2560, 256), (512, 384, 2560), (600, 4100, 768)]
+         (200, 2560, 256), (512, 384, 2560), (600, 4100, 768), (2100, 2500, 128)]
 
 
 @pytest.mark.parametrize("m,n,k", SIZES)
@@ -122,3 +122,55 @@ def test_calls_that_autograd_follows_keep_the_torch_product(env):
     dense = n_.dequant(w, s, b)
     want = dense.sum(dim=0).expand(40, 128)
     assert (x.grad.float() - want).abs().max() <= 2.0**-7 * want.abs().max()  # fp16 weights, bf16 gradient
+
+
+@pytest.mark.parametrize("e,n,k,tokens,top", [(8, 130, 192, 13, 5), (32, 256, 768, 128, 8), (3, 100, 1600, 200, 2),
+                                              (64, 64, 256, 9, 8), (2, 300, 512, 400, 1)])
+@pytest.mark.parametrize("shared", [True, False])
+def test_expert_batches_against_the_oracle(env, e, n, k, tokens, top, shared):
+    """Pairs sorted by expert, tiles of 32, 64 and 128 rows, experts without pairs (64 experts,
+    72 pairs on the even ones), a token's row shared by its experts or a row per pair."""
+    torch, n_, orc = env
+    from ironmule_amd.quantized import library_gather_matmul
+    announce("experts", e, n, k, tokens, top, shared)
+    stack = [orc.synthetic(n, k, 1, seed=orc.SEED_BASE + 970 + i) for i in range(e)]
+    w, s, b = (np.stack([getattr(p, f) for p in stack]) for f in "wsb")
+    dw = torch.from_numpy(w.view(np.int32)).cuda()
+    ds, db = (torch.from_numpy(t).cuda().view(torch.bfloat16) for t in (s, b))
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(tokens)
+    x = torch.randn((tokens, 1 if shared else top, 1, k), device="cuda", generator=gen).to(torch.bfloat16)
+    idx = torch.randint(0, e, (tokens, top), device="cuda", generator=gen)
+    if e == 64:
+        idx = idx // 2 * 2
+    y = library_gather_matmul(x, dw, ds, db, idx)
+    assert tuple(y.shape) == (tokens, top, 1, n)
+    ref, mag = orc.gather_qmv_f64(w, s, b, bf16_bits(x.reshape(-1, k)), idx.reshape(-1).cpu().numpy(),
+                                  top if shared else 1)
+    verdict = orc.check_bf16(bf16_bits(y.reshape(-1, n)), ref, mag)
+    assert verdict.ok, verdict.detail
+    wrapped = torch.where(idx % 3 == 0, idx - e, idx)  # the same experts counted from the last
+    assert torch.equal(library_gather_matmul(x, dw, ds, db, wrapped), y)
+
+
+def test_expert_batch_forms(env):
+    """Several rows per pair, a broadcast index and indices outside the stack."""
+    torch, n_, orc = env
+    from ironmule_amd.quantized import library_gather_matmul
+    announce("expert forms")
+    e, n, k = 4, 96, 320
+    stack = [to_device(orc.synthetic(n, k, 1, seed=orc.SEED_BASE + 990 + i)) for i in range(e)]
+    w, s, b = (torch.stack([p[f] for p in stack]) for f in range(3))
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(5)
+    x = torch.randn((6, 1, 3, k), device="cuda", generator=gen).to(torch.bfloat16)
+    idx = torch.randint(0, e, (5,), device="cuda", generator=gen)
+    y = library_gather_matmul(x, w, s, b, idx)
+    assert tuple(y.shape) == (6, 5, 3, n)
+    for t in range(6):
+        for j in range(5):
+            i = int(idx[j])
+            want = x[t, 0].double() @ n_.dequant(w[i], s[i], b[i]).double().T
+            assert (y[t, j].double() - want).abs().max() <= 2.0**-8 * want.abs().max()
+    out = n_.prompt_experts(w, s, b, x[:, 0, 0], torch.tensor([0, 4, -5, 3, 2, 1], device="cuda"))
+    assert not out[1].any() and not out[2].any() and out[0].any() and out[3:].any(dim=1).all()
