@@ -17,6 +17,7 @@
 #include <stdint.h>
 
 #include "ironmule_qmv.h"
+#include "ironmule_step.h"
 
 #ifdef __cplusplus
 extern "C" {
@@ -69,6 +70,28 @@ IMQ_API int32_t imq_prompt_experts(const uint32_t* w, const uint16_t* scales, co
                                    const int32_t* idx, int32_t pairs, void* y, int64_t ldy, int32_t N, int32_t K,
                                    int32_t group_size, int32_t bits, int32_t y_dtype, void* workspace,
                                    size_t workspace_bytes, void* stream);
+
+/* A whole prompt of one request through decoder layers (head size 128), one call per layer:
+ *   x = rms_norm(h) ; q,k,v = x W^T ; q,k = rope(rms_norm_head(q, k)) at positions 0 .. tokens-1 ;
+ *   KV[slot][0 .. tokens-1] = k, v ; o = causal attention ; h += bf16(o Wo^T) ; x = rms_norm(h) ;
+ *   h += bf16(bf16(silu(bf16(x Wg^T)) * bf16(x Wu^T)) Wd^T)
+ * with fp32 residual stream h (tokens, hidden) and bf16 activations between the steps.  The last
+ * addition of a layer is left in the workspace for the next call (`first` of the first layer is 1,
+ * of the others 0) or for imq_prompt_finish, which
+ * adds it to the last `rows` rows; the calls of one prompt share one workspace
+ * (256-byte aligned, no preparation) and no other call may use it meanwhile.
+ * Replaces a prompt's pass through the layers (ironmule/cuda_native.py:171-179;
+ * ironmule/dense_plan.py:337-363). */
+typedef struct {
+  int32_t tokens, hidden, heads, kv_heads, intermediate, capacity, num_slots, slot;
+  float eps, theta;
+} imq_prompt_shape;
+
+IMQ_API size_t imq_prompt_layer_workspace(const imq_prompt_shape* shape);
+IMQ_API int32_t imq_prompt_layer(const imq_step_layer* layer, const imq_prompt_shape* shape, float* h, int32_t first,
+                                 void* workspace, size_t workspace_bytes, void* stream);
+IMQ_API int32_t imq_prompt_finish(const imq_prompt_shape* shape, float* h, int32_t rows, void* workspace,
+                                  size_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }

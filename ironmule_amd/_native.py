@@ -102,6 +102,14 @@ class StepDesc(ctypes.Structure):
                 ("logits", _P)]
 
 
+class PromptShape(ctypes.Structure):
+    """imq_prompt_shape: a prompt, a decoder layer's sizes and the request's KV slot."""
+
+    _fields_ = [("tokens", _I32), ("hidden", _I32), ("heads", _I32), ("kv_heads", _I32), ("intermediate", _I32),
+                ("capacity", _I32), ("num_slots", _I32), ("slot", _I32), ("eps", ctypes.c_float),
+                ("theta", ctypes.c_float)]
+
+
 class QmvStage(ctypes.Structure):
     """imq_qmv_stage: 1-3 one-row qmv problems sharing x, optionally after the previous stage."""
 
@@ -164,6 +172,10 @@ _SIGNATURES = {
     "imq_prompt_experts_workspace": ([_I32, _I32, _I32], ctypes.c_size_t),
     "imq_prompt_experts": ([_P, _P, _P, _I32, _P, _I64, _I32, _P, _I32, _P, _I64, _I32, _I32, _I32, _I32, _I32, _P,
                             ctypes.c_size_t, _P], _I32),
+    "imq_prompt_layer_workspace": ([ctypes.POINTER(PromptShape)], ctypes.c_size_t),
+    "imq_prompt_layer": ([ctypes.POINTER(StepLayer), ctypes.POINTER(PromptShape), _P, _I32, _P, ctypes.c_size_t, _P],
+                         _I32),
+    "imq_prompt_finish": ([ctypes.POINTER(PromptShape), _P, _I32, _P, ctypes.c_size_t, _P], _I32),
     # persistent programs (include/ironmule_step.h)
     "imq_decode_program_create": ([ctypes.POINTER(StepDesc), ctypes.POINTER(_P)], _I32),
     "imq_qmv_program_create": ([ctypes.POINTER(QmvStage), _I32, ctypes.POINTER(_P)], _I32),
@@ -540,6 +552,51 @@ def prompt_experts(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor, 
                                     pairs, _ptr(out), n, n, k, GROUP_SIZE, BITS, _DTYPE_CODE[out_dtype], _ptr(ws),
                                     nbytes, _stream(None)))
     return out
+
+
+class PromptLayers:
+    """A prompt's pass through decoder layers (imq_prompt_layer) on the current stream: its
+    residual stream h (tokens, hidden) fp32 and the workspace the layers share.  `layer` runs one,
+    in order; `finish` adds the last layer's output to the last row of h and returns that row."""
+
+    def __init__(self, config, h: torch.Tensor, slots: int, capacity: int, slot: int) -> None:
+        c = config
+        _require(h, torch.float32, "h")
+        if h.dim() != 2 or int(h.shape[1]) != c.hidden or c.head_dim != 128:
+            raise ValueError(f"h must be (tokens, {c.hidden}), the head size 128")
+        self.config, self.h, self.first = c, h, 1
+        self.shape = PromptShape(int(h.shape[0]), c.hidden, c.heads, c.kv_heads, c.intermediate, int(capacity),
+                                 int(slots), int(slot), float(c.eps), float(c.theta))
+        self.pool_shape = (int(slots), c.kv_heads, int(capacity), c.head_dim)
+        self.nbytes = int(lib().imq_prompt_layer_workspace(ctypes.byref(self.shape)))
+        if self.nbytes == 0:
+            raise NativeError(*last_error())
+        self.workspace = torch.empty(self.nbytes, dtype=torch.uint8, device=h.device)
+
+    def layer(self, layer: dict, k_pool: torch.Tensor, v_pool: torch.Tensor) -> None:
+        quants = []
+        for name, size in self.config.projections.items():
+            if check_weights(*layer[name]) != tuple(size):
+                raise ValueError(f"{name} must be {tuple(size)}")
+            quants.append(QWeight(*[t.data_ptr() for t in layer[name]]))
+        norms = [layer[name] for name in ("input_norm", "post_norm", "q_norm", "k_norm")]
+        for t, want in zip(norms, (self.config.hidden, self.config.hidden, 128, 128)):
+            _require(t, torch.bfloat16, "a norm weight")
+            if t.numel() != want:
+                raise ValueError(f"a norm weight must have {want} values")
+        for t in (k_pool, v_pool):
+            _require(t, torch.bfloat16, "a pool")
+            if tuple(t.shape) != self.pool_shape:
+                raise ValueError(f"a pool must be {self.pool_shape}")
+        desc = StepLayer(*quants, *[t.data_ptr() for t in norms], k_pool.data_ptr(), v_pool.data_ptr())
+        _check(lib().imq_prompt_layer(ctypes.byref(desc), ctypes.byref(self.shape), _ptr(self.h), self.first,
+                                      _ptr(self.workspace), self.nbytes, _stream(None)))
+        self.first = 0
+
+    def finish(self) -> torch.Tensor:
+        _check(lib().imq_prompt_finish(ctypes.byref(self.shape), _ptr(self.h), 1, _ptr(self.workspace), self.nbytes,
+                                       _stream(None)))
+        return self.h[-1:]
 
 
 # --------------------------------------------------------------- decode-step kernels

@@ -53,12 +53,11 @@ __device__ __forceinline__ uint32_t exponent_max(uint32_t u, uint32_t m) {
   return m > hi ? m : hi;
 }
 
-// A (block, chunk) from row-major x into its LDS image, 16 bytes (one piece) per step of a
-// thread; `piece` 0..31 of the chunk (columns 8 piece ..), `row` 0..31 of the block.  The 32
-// lanes of a half wavefront hold one row's chunk.
-__device__ __forceinline__ void pack_piece(uint4 d, int piece, int row, char* image, uint32_t* flag) {
-  const int g = piece >> 3, c = piece & 7;
-  *reinterpret_cast<uint4*>(image + g * kGroupBytes + c * 512 + row * 16) = pair_order(d);
+// One row's chunk from the 32 lanes of a half wavefront into the (block, chunk) at `to`: lane l
+// holds piece l (columns 8 l .. of the chunk) in d.  Returns whether the row is flagged.
+__device__ __forceinline__ bool emit_row_chunk(uint4 d, int l, int row, char* to) {
+  const int g = l >> 3, c = l & 7;
+  *reinterpret_cast<uint4*>(to + g * kGroupBytes + c * 512 + row * 16) = pair_order(d);
   uint32_t e = exponent_max(d.x, 0u);
   e = exponent_max(d.y, e);
   e = exponent_max(d.z, e);
@@ -69,55 +68,68 @@ __device__ __forceinline__ void pack_piece(uint4 d, int piece, int row, char* im
   s += dpp<0xB1>(s);   // lanes ^ 1
   s += dpp<0x4E>(s);   // lanes ^ 2
   s += dpp<0x141>(s);  // the other four of the eight
-  if (c != 0) return;
-  if (flagged) {
-    s = 0.0f;
-    if (g == 0) atomicOr(flag, 1u << row);
-  }
-  char* const at = image + 4 * kGroupBytes + row * 16 + g * 2;
-  float left = s;
+  if (flagged) s = 0.0f;
+  // the four groups' sums in every lane, one term at a time
+  const int first = threadIdx.x & 32;
+  float left[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) left[k] = __shfl(s, first + 8 * k);
+  uint32_t term[4][4];
 #pragma unroll
   for (int t = 0; t < 3; ++t) {
-    const uint16_t part = f32_to_bf16_bits(left);
-    const float v = bf16_bits_to_f32(part);
-    left -= v;
-    *reinterpret_cast<uint16_t*>(at + t * 512) = part;
-    *reinterpret_cast<uint16_t*>(at + t * 512 + 8) = (uint16_t)(__float_as_uint(-16.0f * v) >> 16);
+    uint32_t a[4], b[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      a[k] = f32_to_bf16_bits(left[k]);
+      const float v = bf16_bits_to_f32(a[k]);
+      left[k] -= v;
+      b[k] = __float_as_uint(-16.0f * v) >> 16;
+    }
+    term[t][0] = a[0] | (a[1] << 16);
+    term[t][1] = a[2] | (a[3] << 16);
+    term[t][2] = b[0] | (b[1] << 16);
+    term[t][3] = b[2] | (b[3] << 16);
   }
-  *reinterpret_cast<uint16_t*>(at + 3 * 512) = 0;
-  *reinterpret_cast<uint16_t*>(at + 3 * 512 + 8) = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) term[3][k] = 0u;
+  // lane t of the half writes term t (hi, mid, lo, zero)
+  if (l < 4) {
+    const uint32_t w0 = l == 0 ? term[0][0] : l == 1 ? term[1][0] : l == 2 ? term[2][0] : 0u;
+    const uint32_t w1 = l == 0 ? term[0][1] : l == 1 ? term[1][1] : l == 2 ? term[2][1] : 0u;
+    const uint32_t w2 = l == 0 ? term[0][2] : l == 1 ? term[1][2] : l == 2 ? term[2][2] : 0u;
+    const uint32_t w3 = l == 0 ? term[0][3] : l == 1 ? term[1][3] : l == 2 ? term[2][3] : 0u;
+    *reinterpret_cast<uint4*>(to + 4 * kGroupBytes + l * 512 + row * 16) = make_uint4(w0, w1, w2, w3);
+  }
+  return flagged;
 }
 
-// One workgroup per (chunk, block).  `src` (may be null): the x row of each packed row, -1 for
-// a row of zeros, and `expert` the expert of each tile of `tm` blocks, -1 for tiles not in use;
-// without them packed row r is x row r, zeros past M.
+// Flag words are written a byte, eight rows, at a time.
+__device__ __forceinline__ void store_flags(uint32_t* flags, int64_t word, int rows8, uint32_t bits) {
+  reinterpret_cast<uint8_t*>(flags + word)[rows8] = (uint8_t)bits;
+}
+
+// One workgroup per (chunk, eight rows).  `src` (may be null): the x row of each packed row, -1
+// for a row of zeros, and `expert` the expert of each tile of `tm` blocks, -1 for tiles not in
+// use; without them packed row r is x row r, zeros past M.
 __global__ __launch_bounds__(kThreads) void pack_rows_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                              const int32_t* __restrict__ src,
                                                              const int32_t* __restrict__ expert, int tm, int M, int K,
                                                              char* __restrict__ packed,
                                                              uint32_t* __restrict__ flags) {
-  __shared__ __attribute__((aligned(16))) char image[kChunkBytes];
-  __shared__ uint32_t flag;
-  const int chunk = blockIdx.x, block = blockIdx.y, chunks = gridDim.x;
-  const int tid = threadIdx.x, piece = tid & 31;
+  __shared__ uint32_t bits;
+  const int chunk = blockIdx.x, chunks = gridDim.x, block = blockIdx.y >> 2, rows8 = blockIdx.y & 3;
+  const int tid = threadIdx.x, l = tid & 31, at = tid >> 5;
   if (expert && expert[block / tm] < 0) return;
-  if (tid == 0) flag = 0u;
-  const int col = 256 * chunk + 8 * piece;
-  uint4 d[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = 32 * block + 8 * i + (tid >> 5);
-    const int64_t row = src ? src[r] : (r < M ? r : -1);
-    d[i] = make_uint4(0u, 0u, 0u, 0u);
-    if (row >= 0 && col < K) d[i] = *reinterpret_cast<const uint4*>(x + row * ldx + col);
-  }
+  if (tid == 0) bits = 0u;
+  const int col = 256 * chunk + 8 * l, r = 32 * block + 8 * rows8 + at;
+  const int64_t row = src ? src[r] : (r < M ? r : -1);
+  uint4 d = make_uint4(0u, 0u, 0u, 0u);
+  if (row >= 0 && col < K) d = *reinterpret_cast<const uint4*>(x + row * ldx + col);
   __syncthreads();
-#pragma unroll
-  for (int i = 0; i < 4; ++i) pack_piece(d[i], piece, 8 * i + (tid >> 5), image, &flag);
+  const int64_t word = (int64_t)block * chunks + chunk;
+  if (emit_row_chunk(d, l, 8 * rows8 + at, packed + word * kChunkBytes) && l == 0) atomicOr(&bits, 1u << at);
   __syncthreads();
-  uint4* const out = reinterpret_cast<uint4*>(packed + ((int64_t)block * chunks + chunk) * kChunkBytes);
-  for (int i = tid; i < kChunkBytes / 16; i += kThreads) out[i] = reinterpret_cast<const uint4*>(image)[i];
-  if (tid == 0) flags[block * chunks + chunk] = flag;
+  if (tid == 0) store_flags(flags, word, rows8, bits);
 }
 
 // ------------------------------------------------------------ the product
@@ -565,6 +577,316 @@ __global__ __launch_bounds__(kSortThreads) void sort_pairs_kernel(const int32_t*
   }
 }
 
+// ------------------------------------------------------------ a prompt through a layer
+
+constexpr int kD = 128;  // head dimension
+
+// h[row] += bf16(the planes' sum) (planes may be null); with `weight`, x = bf16(rms_norm(h) *
+// weight) packed.  A wavefront per row, eight rows per workgroup; lane l of a wavefront holds
+// the 8-column pieces l, l + 64, .. (at most NP).  Every load is issued before the first use.
+template <int NP>
+__global__ __launch_bounds__(512) void norm_pack_kernel(float* __restrict__ h, const float* __restrict__ planes,
+                                                        int splits, int64_t plane_stride,
+                                                        const uint16_t* __restrict__ weight, int M, int dim, float eps,
+                                                        int chunks, char* __restrict__ packed,
+                                                        uint32_t* __restrict__ flags) {
+  __shared__ uint32_t bits[2 * NP];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int row = 8 * blockIdx.x + wave;
+  const bool live = row < M;
+  if (threadIdx.x < 2 * NP) bits[threadIdx.x] = 0u;
+  float* const hr = h + (int64_t)min(row, M - 1) * dim;
+  const float* const pr = planes ? planes + (int64_t)min(row, M - 1) * dim : nullptr;
+  float v[NP][8];
+  uint4 wv[NP];
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    const int col = 8 * (lane + 64 * i);
+    float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f), b = a;
+    wv[i] = make_uint4(0u, 0u, 0u, 0u);
+    if (col < dim && live) {
+      a = *reinterpret_cast<const float4*>(hr + col);
+      b = *reinterpret_cast<const float4*>(hr + col + 4);
+      if (weight) wv[i] = *reinterpret_cast<const uint4*>(weight + col);
+    }
+    v[i][0] = a.x, v[i][1] = a.y, v[i][2] = a.z, v[i][3] = a.w;
+    v[i][4] = b.x, v[i][5] = b.y, v[i][6] = b.z, v[i][7] = b.w;
+  }
+  if (pr) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int col = 8 * (lane + 64 * i);
+      if (col >= dim || !live) continue;
+      float d[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+      for (int s = 0; s < splits; ++s) {
+        const float4 a = *reinterpret_cast<const float4*>(pr + s * plane_stride + col);
+        const float4 b = *reinterpret_cast<const float4*>(pr + s * plane_stride + col + 4);
+        d[0] += a.x, d[1] += a.y, d[2] += a.z, d[3] += a.w;
+        d[4] += b.x, d[5] += b.y, d[6] += b.z, d[7] += b.w;
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[i][e] += bf16_bits_to_f32(f32_to_bf16_bits(d[e]));
+      *reinterpret_cast<float4*>(hr + col) = make_float4(v[i][0], v[i][1], v[i][2], v[i][3]);
+      *reinterpret_cast<float4*>(hr + col + 4) = make_float4(v[i][4], v[i][5], v[i][6], v[i][7]);
+    }
+  }
+  if (!weight) return;
+  float ss = 0.0f;
+#pragma unroll
+  for (int i = 0; i < NP; ++i)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ss = fmaf(v[i][e], v[i][e], ss);
+  const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)dim + eps);
+  __syncthreads();
+  const int block = blockIdx.x >> 2, rows8 = blockIdx.x & 3;
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    const uint32_t w[4] = {wv[i].x, wv[i].y, wv[i].z, wv[i].w};
+    uint32_t out[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t lo = f32_to_bf16_bits(v[i][2 * e] * inv * bf16_bits_to_f32(w[e] & 0xffffu));
+      const uint32_t hi = f32_to_bf16_bits(v[i][2 * e + 1] * inv * bf16_bits_to_f32(w[e] >> 16));
+      out[e] = lo | (hi << 16);
+    }
+    const int chunk = 2 * i + (lane >> 5);
+    // columns past the row (a last part-full chunk) and rows past M are packed as zeros
+    uint4 d = make_uint4(out[0], out[1], out[2], out[3]);
+    if (!live || 8 * (lane + 64 * i) >= dim) d = make_uint4(0u, 0u, 0u, 0u);
+    if (chunk >= chunks) continue;
+    const int64_t word = (int64_t)block * chunks + chunk;
+    if (emit_row_chunk(d, lane & 31, 8 * rows8 + wave, packed + word * kChunkBytes) && (lane & 31) == 0)
+      atomicOr(&bits[chunk], 1u << wave);
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < chunks) store_flags(flags, (int64_t)block * chunks + threadIdx.x, rows8, bits[threadIdx.x]);
+}
+
+// act = bf16(silu(gate) * up), packed; one workgroup per (chunk, eight rows).
+__global__ __launch_bounds__(kThreads) void silu_pack_kernel(const uint16_t* __restrict__ gate,
+                                                             const uint16_t* __restrict__ up, int M, int K,
+                                                             char* __restrict__ packed,
+                                                             uint32_t* __restrict__ flags) {
+  __shared__ uint32_t bits;
+  const int chunk = blockIdx.x, chunks = gridDim.x, block = blockIdx.y >> 2, rows8 = blockIdx.y & 3;
+  const int tid = threadIdx.x, l = tid & 31, at = tid >> 5;
+  if (tid == 0) bits = 0u;
+  const int col = 256 * chunk + 8 * l, row = 32 * block + 8 * rows8 + at;
+  uint32_t out[4] = {0u, 0u, 0u, 0u};
+  if (row < M && col < K) {
+    const uint4 g4 = *reinterpret_cast<const uint4*>(gate + (int64_t)row * K + col);
+    const uint4 u4 = *reinterpret_cast<const uint4*>(up + (int64_t)row * K + col);
+    const uint32_t g[4] = {g4.x, g4.y, g4.z, g4.w}, u[4] = {u4.x, u4.y, u4.z, u4.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float a = bf16_bits_to_f32(g[e] & 0xffffu), b = bf16_bits_to_f32(g[e] >> 16);
+      const uint32_t lo = f32_to_bf16_bits(a / (1.0f + expf(-a)) * bf16_bits_to_f32(u[e] & 0xffffu));
+      const uint32_t hi = f32_to_bf16_bits(b / (1.0f + expf(-b)) * bf16_bits_to_f32(u[e] >> 16));
+      out[e] = lo | (hi << 16);
+    }
+  }
+  __syncthreads();
+  const int64_t word = (int64_t)block * chunks + chunk;
+  if (emit_row_chunk(make_uint4(out[0], out[1], out[2], out[3]), l, 8 * rows8 + at, packed + word * kChunkBytes) && l == 0)
+    atomicOr(&bits, 1u << at);
+  __syncthreads();
+  if (tid == 0) store_flags(flags, word, rows8, bits);
+}
+
+// Per token and head: q and k heads get the per-head RMSNorm (rounded to bf16) and the
+// non-interleaved rotary embedding at the token's position, angles in double; q in place, k and
+// v into the slot's pools.  A workgroup per token, a wavefront per head at a time; lane i holds
+// dimensions i and i + 64, the pair that turns together.
+__global__ __launch_bounds__(kThreads) void prompt_rope_kernel(uint16_t* __restrict__ q,
+                                                               const uint16_t* __restrict__ k,
+                                                               const uint16_t* __restrict__ v,
+                                                               const uint16_t* __restrict__ q_norm,
+                                                               const uint16_t* __restrict__ k_norm,
+                                                               uint16_t* __restrict__ k_pool,
+                                                               uint16_t* __restrict__ v_pool, int Hq, int Hkv,
+                                                               int capacity, double log2_theta, float eps) {
+  const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double sn, cs;
+  sincos((double)t * exp2(-(double)lane * (log2_theta / 64.0)), &sn, &cs);
+  const float s = (float)sn, c = (float)cs;
+  for (int hh = wave; hh < Hq + 2 * Hkv; hh += kThreads / 64) {
+    const bool is_q = hh < Hq, is_v = hh >= Hq + Hkv;
+    const int head = is_q ? hh : is_v ? hh - Hq - Hkv : hh - Hq;
+    const uint16_t* const src = is_q ? q + ((int64_t)t * Hq + head) * kD : (is_v ? v : k) + ((int64_t)t * Hkv + head) * kD;
+    uint16_t* const dst = is_q ? q + ((int64_t)t * Hq + head) * kD
+                               : (is_v ? v_pool : k_pool) + ((int64_t)head * capacity + t) * kD;
+    if (is_v) {
+      reinterpret_cast<uint32_t*>(dst)[lane] = reinterpret_cast<const uint32_t*>(src)[lane];
+      continue;
+    }
+    const uint16_t* const nw = is_q ? q_norm : k_norm;
+    float a = bf16_bits_to_f32(src[lane]), b = bf16_bits_to_f32(src[lane + 64]);
+    const float inv = 1.0f / sqrtf(wave_sum(fmaf(a, a, b * b)) / (float)kD + eps);
+    a = bf16_bits_to_f32(f32_to_bf16_bits(a * inv * bf16_bits_to_f32(nw[lane])));
+    b = bf16_bits_to_f32(f32_to_bf16_bits(b * inv * bf16_bits_to_f32(nw[lane + 64])));
+    dst[lane] = f32_to_bf16_bits(a * c - b * s);
+    dst[lane + 64] = f32_to_bf16_bits(a * s + b * c);
+  }
+}
+
+// Causal attention of a prompt: out[t][head] = softmax(q . K / sqrt(128)) V over positions
+// 0 .. t of one slot.
+//
+// A workgroup takes 64 queries of one head, a wavefront 16 of them, and walks the keys in
+// blocks of 64, the next block's K and V in flight in registers meanwhile.  Scores are K Q^T on
+// v_mfma_f32_16x16x32_bf16, so that a lane holds keys of one query: P^T is then the B operand
+// of V^T P^T without leaving its lane (key order 4 g .. of two 16-key tiles per 32-key step).  P
+// goes in as three bf16 terms that add up to its 24 bits, so P V keeps fp32's accuracy.  K lies
+// in LDS in rows of swizzled 16-byte pieces, V transposed with padded rows; both twice.  Heavy
+// query blocks, the last ones, start first.
+//
+// Bound by latency at a few hundred tokens (512 tokens of 32 heads: 256 workgroups, at most
+// eight key blocks each), where the same in torch operations (fp32 products, mask, softmax,
+// repeated heads) took about 300 us a layer.
+constexpr int kQ = 64, kKeys = 64, kVRow = 2 * kKeys + 8;  // V^T row bytes: 16 mod 128 banks apart
+
+__global__ __launch_bounds__(kThreads, 2) void prompt_attention_kernel(const uint16_t* __restrict__ q,
+                                                                       const uint16_t* __restrict__ k_pool,
+                                                                       const uint16_t* __restrict__ v_pool,
+                                                                       uint16_t* __restrict__ out, int T, int Hq,
+                                                                       int Hkv, int capacity) {
+  __shared__ __attribute__((aligned(16))) char kl[2][kKeys * 256];
+  __shared__ __attribute__((aligned(16))) char vl[2][kD * kVRow];
+  const int qblocks = gridDim.x / Hq;
+  const int head = blockIdx.x % Hq, qb = qblocks - 1 - (int)blockIdx.x / Hq;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4;
+  const int64_t kv = (int64_t)(head / (Hq / Hkv)) * capacity * kD;
+  const int query = qb * kQ + 16 * wave + n;
+  const int last = T - 1;
+
+  bf16x8_t qf[4];
+  {
+    const uint16_t* const src = q + ((int64_t)min(query, last) * Hq + head) * kD;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      qf[t] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(src + 32 * t + 8 * g));
+  }
+  uint4 kr[4], va[2], vb[2];
+  auto load = [&](int block) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int p = tid + kThreads * i;
+      kr[i] = *reinterpret_cast<const uint4*>(k_pool + kv + (int64_t)min(block * kKeys + (p >> 4), last) * kD + 8 * (p & 15));
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int p = tid + kThreads * i, key = block * kKeys + 2 * (p >> 4);
+      va[i] = *reinterpret_cast<const uint4*>(v_pool + kv + (int64_t)min(key, last) * kD + 8 * (p & 15));
+      vb[i] = *reinterpret_cast<const uint4*>(v_pool + kv + (int64_t)min(key + 1, last) * kD + 8 * (p & 15));
+    }
+  };
+  auto stage = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int p = tid + kThreads * i, row = p >> 4;
+      *reinterpret_cast<uint4*>(kl[b] + row * 256 + (((p & 15) ^ (row & 15)) << 4)) = kr[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int p = tid + kThreads * i;
+      char* const to = vl[b] + 8 * (p & 15) * kVRow + 4 * (p >> 4);
+      const uint32_t a[4] = {va[i].x, va[i].y, va[i].z, va[i].w}, c[4] = {vb[i].x, vb[i].y, vb[i].z, vb[i].w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        *reinterpret_cast<uint32_t*>(to + (2 * e) * kVRow) = __builtin_amdgcn_perm(c[e], a[e], 0x05040100u);
+        *reinterpret_cast<uint32_t*>(to + (2 * e + 1) * kVRow) = __builtin_amdgcn_perm(c[e], a[e], 0x07060302u);
+      }
+    }
+  };
+
+  constexpr float kLog2e = 1.44269504088896340736f, kScale = 0.08838834764831845f;  // 128^-1/2
+  f32x4_t o[8];
+#pragma unroll
+  for (int d = 0; d < 8; ++d) o[d] = f32x4_t{};
+  float top = -INFINITY, sum = 0.0f;
+  load(0);
+  stage(0);
+  __syncthreads();
+  for (int block = 0; block <= qb; ++block) {
+    if (block < qb) load(block + 1);
+    const char* const kb = kl[block & 1];
+    const char* const vt = vl[block & 1];
+    f32x4_t s[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      s[b] = f32x4_t{};
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const uint4 kf = *reinterpret_cast<const uint4*>(kb + (16 * b + n) * 256 + (((4 * t + g) ^ n) << 4));
+        s[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf), qf[t], s[b], 0, 0, 0);
+      }
+    }
+    float most = -INFINITY;
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        s[b][e] *= kScale;
+        if (block == qb && block * kKeys + 16 * b + 4 * g + e > query) s[b][e] = -INFINITY;
+        most = fmaxf(most, s[b][e]);  // (a NaN score comes back through its exponential)
+      }
+    most = fmaxf(most, top);
+    most = max_xor32(max_xor16(most));
+    const float base = most == -INFINITY ? 0.0f : most;
+    const float keep = exp2f((top - base) * kLog2e);
+    top = most;
+    sum *= keep;
+    uint32_t p0[4][2], p1[4][2], p2[4][2];  // the three terms, two keys a word
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; e += 2) {
+        uint32_t w[2][3];
+#pragma unroll
+        for (int z = 0; z < 2; ++z) {
+          const float v = exp2f((s[b][e + z] - base) * kLog2e);
+          sum += v;
+          w[z][0] = __float_as_uint(v);
+          const float r = v - __uint_as_float(w[z][0] & 0xffff0000u);
+          w[z][1] = __float_as_uint(r);
+          w[z][2] = __float_as_uint(r - __uint_as_float(w[z][1] & 0xffff0000u));
+        }
+        p0[b][e >> 1] = __builtin_amdgcn_perm(w[1][0], w[0][0], 0x07060302u);
+        p1[b][e >> 1] = __builtin_amdgcn_perm(w[1][1], w[0][1], 0x07060302u);
+        p2[b][e >> 1] = __builtin_amdgcn_perm(w[1][2], w[0][2], 0x07060302u);
+      }
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[d][e] *= keep;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const char* const at = vt + (16 * d + n) * kVRow + 64 * j + 8 * g;
+        const u32x2_t lo = *reinterpret_cast<const u32x2_t*>(at), hi = *reinterpret_cast<const u32x2_t*>(at + 32);
+        const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, u32x4_t{lo.x, lo.y, hi.x, hi.y});
+        const u32x4_t t0 = {p0[2 * j][0], p0[2 * j][1], p0[2 * j + 1][0], p0[2 * j + 1][1]};
+        const u32x4_t t1 = {p1[2 * j][0], p1[2 * j][1], p1[2 * j + 1][0], p1[2 * j + 1][1]};
+        const u32x4_t t2 = {p2[2 * j][0], p2[2 * j][1], p2[2 * j + 1][0], p2[2 * j + 1][1]};
+        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(bf16x8_t, t0), o[d], 0, 0, 0);
+        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(bf16x8_t, t1), o[d], 0, 0, 0);
+        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(bf16x8_t, t2), o[d], 0, 0, 0);
+      }
+    }
+    if (block < qb) stage((block + 1) & 1);
+    __syncthreads();
+  }
+  sum = add_xor32(add_xor16(sum));
+  if (query > last) return;
+  uint16_t* const to = out + ((int64_t)query * Hq + head) * kD + 4 * g;
+#pragma unroll
+  for (int d = 0; d < 8; ++d) {
+    uint32_t w[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w[e] = f32_to_bf16_bits(o[d][e] / sum);
+    *reinterpret_cast<u32x2_t*>(to + 16 * d) = u32x2_t{w[0] | (w[1] << 16), w[2] | (w[3] << 16)};
+  }
+}
+
 // ------------------------------------------------------------ host side
 
 int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
@@ -586,7 +908,7 @@ int column_tiles(const int32_t* N, int count) {
 // workgroup of the busiest CU 0.56 / 0.31 / 0.20 us, with tiles of 128 / 64 / 32 rows: tall
 // tiles reuse the weights, short ones fill the CUs.  K-ranges add the planes' traffic (about
 // 4 TB/s each way) and the launch that adds them.
-Plan plan_product(const int32_t* N, int count, int M, int K, int cus) {
+Plan plan_product(const int32_t* N, int count, int M, int K, int cus, int max_splits = 8) {
   const int chunks = ceil_div(K, 256), col_tiles = column_tiles(N, count);
   double columns = 0.0, best = 0.0;
   for (int i = 0; i < count; ++i) columns += N[i];
@@ -595,7 +917,7 @@ Plan plan_product(const int32_t* N, int count, int M, int K, int cus) {
   for (int tm = 4; tm >= 1; tm >>= 1) {
     const double start = tm == 4 ? 14.0 : tm == 2 ? 11.0 : 9.0, group = tm == 4 ? 0.56 : tm == 2 ? 0.31 : 0.20;
     const int row_tiles = ceil_div(M, 32 * tm);
-    for (int splits = 1; splits <= 8 && splits <= chunks; ++splits) {
+    for (int splits = 1; splits <= max_splits && splits <= chunks; ++splits) {
       const int range = ceil_div(chunks, splits);
       if (ceil_div(chunks, range) != splits) continue;
       double us = start + group * 4.0 * range * ceil_div((int64_t)row_tiles * col_tiles * splits, cus);
@@ -635,7 +957,7 @@ void pack_rows(const uint16_t* x, int64_t ldx, const int32_t* src, const int32_t
                int64_t blocks, int K, void* packed, hipStream_t stream) {
   const int chunks = ceil_div(K, 256);
   char* const base = static_cast<char*>(packed);
-  hipLaunchKernelGGL(pack_rows_kernel, dim3(chunks, (uint32_t)blocks), dim3(kThreads), 0, stream, x, ldx, src, expert, tm, M, K,
+  hipLaunchKernelGGL(pack_rows_kernel, dim3(chunks, (uint32_t)blocks * 4), dim3(kThreads), 0, stream, x, ldx, src, expert, tm, M, K,
                      base + flag_bytes(blocks, chunks), reinterpret_cast<uint32_t*>(base));
 }
 
@@ -715,9 +1037,186 @@ int32_t check_product(const imq_problem* p, int32_t count, int32_t M, int32_t gr
   return IMQ_OK;
 }
 
+// y = x W^T as the plan's fp32 planes (one where it does not split): the residual add takes them.
+int32_t product_planes(const imq_qweight& w, const void* packed, int M, int N, int K, float* planes, int cus,
+                       int* splits, hipStream_t stream) {
+  const int32_t n = N;
+  const Plan plan = plan_product(&n, 1, M, K, cus);
+  ProductArgs a;
+  memset(&a, 0, sizeof(a));
+  a.p[0] = ProductProblem{w.w, w.scales, w.biases, nullptr, 0, N, 0};
+  a.count = 1;
+  a.planes = planes;
+  a.plane_ld = N;
+  a.plane_stride = (int64_t)M * N;
+  *splits = plan.splits;
+  return run_product(a, plan, packed, ceil_div(M, 32), M, K, stream);
+}
+
+void norm_pack(float* h, const float* planes, int splits, int64_t stride, const uint16_t* weight, int M, int dim,
+               float eps, void* packed, hipStream_t stream) {
+  const int chunks = ceil_div(dim, 256), blocks = ceil_div(M, 32);
+  char* const base = static_cast<char*>(packed);
+  char* const to = base + flag_bytes(blocks, chunks);
+  uint32_t* const flags = reinterpret_cast<uint32_t*>(base);
+  const dim3 grid(4 * blocks), threads(512);
+  const int pieces = ceil_div(dim, 512);
+  if (pieces <= 2)
+    hipLaunchKernelGGL(norm_pack_kernel<2>, grid, threads, 0, stream, h, planes, splits, stride, weight, M, dim, eps, chunks, to, flags);
+  else if (pieces <= 5)
+    hipLaunchKernelGGL(norm_pack_kernel<5>, grid, threads, 0, stream, h, planes, splits, stride, weight, M, dim, eps, chunks, to, flags);
+  else if (pieces <= 8)
+    hipLaunchKernelGGL(norm_pack_kernel<8>, grid, threads, 0, stream, h, planes, splits, stride, weight, M, dim, eps, chunks, to, flags);
+  else
+    hipLaunchKernelGGL(norm_pack_kernel<16>, grid, threads, 0, stream, h, planes, splits, stride, weight, M, dim, eps, chunks, to, flags);
+}
+
+// The parts of a prompt's workspace, each 256-byte aligned.
+struct LayerSpace {
+  size_t x, attn_packed, act, q, k, v, attn, gate, up, planes, bytes;
+};
+
+int32_t check_shape(const imq_prompt_shape* s) {
+  if (!s) return fail(IMQ_EINVAL, "the shape is null");
+  if (s->tokens < 1 || s->tokens > IMQ_PROMPT_MAX_ROWS) return fail(IMQ_EINVAL, "tokens out of range");
+  if (s->heads < 1 || s->kv_heads < 1 || s->heads % s->kv_heads) return fail(IMQ_EINVAL, "need kv_heads >= 1 dividing heads");
+  if (s->heads > 1024) return fail(IMQ_EUNSUPPORTED, "too many heads");
+  if (s->hidden < 64 || s->hidden % 64 || s->intermediate < 64 || s->intermediate % 64)
+    return fail(IMQ_EINVAL, "hidden and intermediate must be positive multiples of 64");
+  if (s->hidden > 8192 || s->intermediate > IMQ_PROMPT_MAX_K) return fail(IMQ_EUNSUPPORTED, "hidden or intermediate too large");
+  if (s->capacity < s->tokens) return fail(IMQ_EINVAL, "the prompt does not fit the capacity");
+  if (s->slot < 0 || s->slot >= s->num_slots) return fail(IMQ_EINVAL, "slot out of range");
+  if (!(s->eps >= 0.0f) || !(s->theta > 1.0f)) return fail(IMQ_EINVAL, "eps must be >= 0 and theta > 1");
+  return IMQ_OK;
+}
+
+LayerSpace layer_space(const imq_prompt_shape& s, int cus) {
+  const int T = s.tokens, blocks = ceil_div(T, 32), qd = s.heads * kD, kd = s.kv_heads * kD;
+  const int32_t n = s.hidden;
+  const int so = plan_product(&n, 1, T, qd, cus).splits, sd = plan_product(&n, 1, T, s.intermediate, cus).splits;
+  LayerSpace l;
+  size_t at = 0;
+  auto take = [&](size_t bytes) {
+    const size_t here = at;
+    at += round_up(bytes, 256);
+    return here;
+  };
+  l.planes = take((size_t)(so > sd ? so : sd) * T * s.hidden * 4);
+  l.x = take(packed_bytes(blocks, s.hidden));
+  l.attn_packed = take(packed_bytes(blocks, qd));
+  l.act = take(packed_bytes(blocks, s.intermediate));
+  l.q = take((size_t)T * qd * 2);
+  l.k = take((size_t)T * kd * 2);
+  l.v = take((size_t)T * kd * 2);
+  l.attn = take((size_t)T * qd * 2);
+  l.gate = take((size_t)T * s.intermediate * 2);
+  l.up = take((size_t)T * s.intermediate * 2);
+  l.bytes = at;
+  return l;
+}
+
+int32_t launched(const char* what) {
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(IMQ_ELAUNCH, std::string(what) + " launch failed: " + hipGetErrorString(e));
+  return ok();
+}
+
 }  // namespace
 
 extern "C" {
+
+size_t imq_prompt_layer_workspace(const imq_prompt_shape* shape) {
+  int32_t code;
+  if (check_shape(shape) != IMQ_OK) return 0;
+  const DeviceInfo* dev = current_device(&code);
+  return dev ? layer_space(*shape, dev->cu_count).bytes : 0;
+}
+
+int32_t imq_prompt_layer(const imq_step_layer* layer, const imq_prompt_shape* shape, float* h, int32_t first,
+                         void* workspace, size_t workspace_bytes, void* stream) {
+  int32_t code = check_shape(shape);
+  if (code != IMQ_OK) return code;
+  if (!layer || !h || !workspace) return fail(IMQ_EINVAL, "layer, h and workspace must be non-null");
+  if (!aligned(h, 16) || !aligned(workspace, 256)) return fail(IMQ_EINVAL, "h must be 16-byte aligned, the workspace 256-byte");
+  const imq_prompt_shape& s = *shape;
+  const int T = s.tokens, blocks = ceil_div(T, 32), qd = s.heads * kD, kd = s.kv_heads * kD;
+  const imq_qweight* const ws[7] = {&layer->q, &layer->k, &layer->v, &layer->o, &layer->gate, &layer->up, &layer->down};
+  const int32_t ns[7] = {qd, kd, kd, s.hidden, s.intermediate, s.intermediate, s.hidden};
+  const int32_t ks[7] = {s.hidden, s.hidden, s.hidden, qd, s.hidden, s.hidden, s.intermediate};
+  for (int i = 0; i < 7; ++i)
+    if ((code = check_weight(ws[i]->w, ws[i]->scales, ws[i]->biases, ns[i], ks[i], 64, 4)) != IMQ_OK) return code;
+  if (!layer->input_norm || !layer->post_norm || !layer->q_norm || !layer->k_norm || !layer->k_pool || !layer->v_pool)
+    return fail(IMQ_EINVAL, "null norm weight or pool");
+  if (!aligned(layer->input_norm, 16) || !aligned(layer->post_norm, 16) || !aligned(layer->k_pool, 16) ||
+      !aligned(layer->v_pool, 16))
+    return fail(IMQ_EINVAL, "norm weights and pools must be 16-byte aligned");
+  const DeviceInfo* dev = current_device(&code);
+  if (!dev) return code;
+  const LayerSpace l = layer_space(s, dev->cu_count);
+  if (workspace_bytes < l.bytes) return fail(IMQ_EINVAL, "the workspace is too small");
+  char* const at = static_cast<char*>(workspace);
+  float* const planes = reinterpret_cast<float*>(at + l.planes);
+  uint16_t *const q = reinterpret_cast<uint16_t*>(at + l.q), *const k = reinterpret_cast<uint16_t*>(at + l.k);
+  uint16_t *const v = reinterpret_cast<uint16_t*>(at + l.v), *const attn = reinterpret_cast<uint16_t*>(at + l.attn);
+  uint16_t *const gate = reinterpret_cast<uint16_t*>(at + l.gate), *const up = reinterpret_cast<uint16_t*>(at + l.up);
+  const int64_t pool = (int64_t)s.slot * s.kv_heads * s.capacity * kD;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+
+  // several weights of one K as bf16 rows
+  auto project = [&](const imq_qweight* const* w, const int32_t* N, uint16_t* const* y, int count, int K, size_t packed) {
+    const Plan plan = plan_product(N, count, T, K, dev->cu_count, 1);
+    ProductArgs a;
+    memset(&a, 0, sizeof(a));
+    a.count = count;
+    int tile0 = 0;
+    for (int i = 0; i < count; ++i) {
+      a.p[i] = ProductProblem{w[i]->w, w[i]->scales, w[i]->biases, y[i], N[i], N[i], tile0};
+      tile0 += ceil_div(N[i], kColumns);
+    }
+    return run_product(a, plan, at + packed, blocks, T, K, st);
+  };
+
+  const int32_t n = s.hidden;
+  int splits = plan_product(&n, 1, T, s.intermediate, dev->cu_count).splits;  // of the layer before
+  norm_pack(h, first ? nullptr : planes, splits, (int64_t)T * s.hidden, layer->input_norm, T, s.hidden, s.eps, at + l.x, st);
+  uint16_t* const qkv[3] = {q, k, v};
+  if ((code = project(ws, ns, qkv, 3, s.hidden, l.x)) != IMQ_OK) return code;
+  hipLaunchKernelGGL(prompt_rope_kernel, dim3(T), dim3(kThreads), 0, st, q, k, v, layer->q_norm, layer->k_norm,
+                     layer->k_pool + pool, layer->v_pool + pool, s.heads, s.kv_heads, s.capacity,
+                     log2((double)s.theta), s.eps);
+  hipLaunchKernelGGL(prompt_attention_kernel, dim3(ceil_div(T, kQ) * s.heads), dim3(kThreads), 0, st, q,
+                     layer->k_pool + pool, layer->v_pool + pool, attn, T, s.heads, s.kv_heads, s.capacity);
+  pack_rows(attn, qd, nullptr, nullptr, 1, T, blocks, qd, at + l.attn_packed, st);
+  if ((code = product_planes(layer->o, at + l.attn_packed, T, s.hidden, qd, planes, dev->cu_count, &splits, st)) != IMQ_OK)
+    return code;
+  norm_pack(h, planes, splits, (int64_t)T * s.hidden, layer->post_norm, T, s.hidden, s.eps, at + l.x, st);
+  uint16_t* const gu[2] = {gate, up};
+  if ((code = project(ws + 4, ns + 4, gu, 2, s.hidden, l.x)) != IMQ_OK) return code;
+  const int chunks = ceil_div(s.intermediate, 256);
+  hipLaunchKernelGGL(silu_pack_kernel, dim3(chunks, 4 * blocks), dim3(kThreads), 0, st, gate, up, T, s.intermediate,
+                     at + l.act + flag_bytes(blocks, chunks), reinterpret_cast<uint32_t*>(at + l.act));
+  if ((code = product_planes(layer->down, at + l.act, T, s.hidden, s.intermediate, planes, dev->cu_count, &splits, st)) != IMQ_OK)
+    return code;
+  return launched("prompt layer");
+}
+
+int32_t imq_prompt_finish(const imq_prompt_shape* shape, float* h, int32_t rows, void* workspace,
+                          size_t workspace_bytes, void* stream) {
+  int32_t code = check_shape(shape);
+  if (code != IMQ_OK) return code;
+  if (!h || !workspace || !aligned(h, 16) || !aligned(workspace, 256)) return fail(IMQ_EINVAL, "h or workspace null or misaligned");
+  if (rows < 1 || rows > shape->tokens) return fail(IMQ_EINVAL, "rows must be 1 .. tokens");
+  const DeviceInfo* dev = current_device(&code);
+  if (!dev) return code;
+  const LayerSpace l = layer_space(*shape, dev->cu_count);
+  if (workspace_bytes < l.bytes) return fail(IMQ_EINVAL, "the workspace is too small");
+  const int32_t n = shape->hidden;
+  const int64_t stride = (int64_t)shape->tokens * n, skip = (int64_t)(shape->tokens - rows) * n;
+  const int splits = plan_product(&n, 1, shape->tokens, shape->intermediate, dev->cu_count).splits;
+  const float* const planes = reinterpret_cast<const float*>(static_cast<char*>(workspace) + l.planes);
+  norm_pack(h + skip, planes + skip, splits, stride, nullptr, rows, n, 0.0f, workspace, static_cast<hipStream_t>(stream));
+  return launched("prompt finish");
+}
 
 size_t imq_prompt_packed_bytes(int32_t M, int32_t K) {
   if (M < 1 || M > IMQ_PROMPT_MAX_ROWS || K < 64 || K % 64 || K > IMQ_PROMPT_MAX_K) return 0;

@@ -33,9 +33,9 @@ into the projections around it.
 
 `prefill` runs a whole prompt through the same model at once, the library path a prompt
 takes (ironmule/cuda_native.py:171-179): every projection of more than 32 rows is one
-product on the packed weight (include/ironmule_prompt.h), attention is causal over the prompt in fp32, the KV
-pools of the request's slot are written for positions 0..T-1, and the head is computed
-for the last position only (ironmule/cuda_native.py:271-303, `head_skip_prefill`).
+product on the packed weight (include/ironmule_prompt.h), attention is causal over the prompt
+with fp32 scores and probabilities, the KV pools of the request's slot are written for positions
+0..T-1, and the head is computed for the last position only (ironmule/cuda_native.py:271-303, `head_skip_prefill`).
 """
 
 from __future__ import annotations
@@ -366,6 +366,24 @@ def _project(x: torch.Tensor, quant: Quant, stream=None) -> torch.Tensor:
     return _native.prompt_matmul(w, s, b, x)
 
 
+def _layers_fit(weights: DecoderWeights, state: DecodeState) -> bool:
+    """Whether the prompt kernels (_native.PromptLayers) take this model and these pools: the
+    sizes and alignments of imq_prompt_layer.  Other models run the torch composition below."""
+    c = weights.config
+    if (c.head_dim != 128 or c.heads % c.kv_heads or c.heads > 1024 or c.hidden % 64 or c.hidden > 8192
+            or c.intermediate % 64 or c.intermediate > _native.MAX_PROMPT_K or not c.theta > 1.0 or c.eps < 0.0):
+        return False
+    if len(weights.layers) != c.layers or len(state.k_pool) != c.layers:
+        return False
+    shape = (state.slots, c.kv_heads, state.capacity, c.head_dim)
+    pools = (*state.k_pool, *state.v_pool)
+    norms = [layer[name] for layer in weights.layers for name in ("input_norm", "post_norm", "q_norm", "k_norm")]
+    norms.append(weights.norm)
+    return (all(tuple(t.shape) == shape for t in pools)
+            and all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.data_ptr() % 16 == 0 and t.is_cuda
+                    for t in (*pools, *norms)))
+
+
 def prefill(weights: DecoderWeights, state: DecodeState, tokens, slot: int,
             stream=None) -> torch.Tensor:
     """Runs the prompt `tokens` (positions 0..T-1) of one request through the model,
@@ -383,6 +401,13 @@ def prefill(weights: DecoderWeights, state: DecodeState, tokens, slot: int,
         ids = torch.as_tensor(list(tokens), dtype=torch.int32).to(device)
         h = torch.empty((count, c.hidden), dtype=torch.float32, device=device)
         _native.embed(*weights.embed, ids, h, stream=stream)
+        if c.layers and _layers_fit(weights, state):
+            run = _native.PromptLayers(c, h, state.slots, state.capacity, slot)
+            for layer, k_pool, v_pool in zip(weights.layers, state.k_pool, state.v_pool):
+                run.layer(layer, k_pool, v_pool)
+            last = torch.empty((1, c.hidden), dtype=torch.bfloat16, device=device)
+            _native.add_rmsnorm(run.finish(), weights.norm, last, c.eps, stream=stream)
+            return _native.qmv(*weights.embed, last, out_dtype=torch.float32, stream=stream)[0]
         positions = torch.arange(count, device=device)
         causal = torch.ones((count, count), dtype=torch.bool, device=device).tril()
         group = c.heads // c.kv_heads

@@ -174,3 +174,64 @@ def test_expert_batch_forms(env):
             assert (y[t, j].double() - want).abs().max() <= 2.0**-8 * want.abs().max()
     out = n_.prompt_experts(w, s, b, x[:, 0, 0], torch.tensor([0, 4, -5, 3, 2, 1], device="cuda"))
     assert not out[1].any() and not out[2].any() and out[0].any() and out[3:].any(dim=1).all()
+
+
+@pytest.mark.parametrize("tokens,heads,kv_heads,hidden,intermediate", [
+    (1, 4, 2, 256, 512), (16, 4, 2, 256, 512), (33, 6, 3, 320, 448), (63, 8, 1, 192, 256), (64, 4, 4, 256, 512),
+    (65, 4, 2, 256, 512), (130, 8, 2, 576, 1088), (257, 16, 2, 1024, 768)])
+def test_prompt_layers_against_the_torch_composition(env, monkeypatch, tokens, heads, kv_heads, hidden, intermediate):
+    """A prompt through imq_prompt_layer and through the same steps in torch operations: both
+    round to bf16 at the same places, so keys and values differ by a rounding (an ulp is 2^-8 of a
+    value, and a layer's differences pass through the next) and nothing outside the prompt's rows
+    is written.  Query blocks of 64 in part and in full, grouped heads, K off the chunks."""
+    torch, n_, orc = env
+    from ironmule_amd import decode
+    announce("prompt layers", tokens, heads, kv_heads, hidden, intermediate)
+    cfg = decode.DecoderConfig(hidden=hidden, layers=3, heads=heads, kv_heads=kv_heads, head_dim=128,
+                               intermediate=intermediate, vocab=512)
+    weights = decode.random_weights(cfg, "cuda", seed=tokens)
+    for layer in weights.layers:  # zero-mean weights: the layers' outputs do not line up
+        for name in cfg.projections:
+            layer[name][2].copy_(layer[name][1] * -7.5)
+    ids = np.random.default_rng(tokens).integers(0, cfg.vocab, tokens).tolist()
+    states = [decode.DecodeState(cfg, batch=1, slots=3, capacity=tokens + 5, max_len=tokens + 5, device="cuda")
+              for _ in range(2)]
+    got = decode.prefill(weights, states[0], ids, 1)
+    monkeypatch.setattr(decode, "_layers_fit", lambda *a: False)
+    want = decode.prefill(weights, states[1], ids, 1)
+    assert (got - want).abs().max() <= 2.0**-6 * want.abs().max()
+    for mine, theirs in zip(states[0].k_pool + states[0].v_pool, states[1].k_pool + states[1].v_pool):
+        assert not mine[0].any() and not mine[2].any() and not mine[1, :, tokens:].any()
+        assert (mine.float() - theirs.float()).abs().max() <= 2.0**-6 * theirs.float().abs().max()
+
+
+def test_prompt_layers_replay_in_a_graph(env):
+    """A captured prompt (the layers alone: the embedding is set before) gives the eager bits on
+    every replay, with eager work between the replays."""
+    torch, n_, orc = env
+    from ironmule_amd import decode
+    announce("prompt layers graph")
+    cfg = decode.DecoderConfig(hidden=256, layers=2, heads=4, kv_heads=2, head_dim=128, intermediate=512, vocab=512)
+    weights = decode.random_weights(cfg, "cuda", seed=3)
+    state = decode.DecodeState(cfg, batch=1, slots=1, capacity=80, max_len=80, device="cuda")
+    start = torch.randn((70, 256), device="cuda")
+    h, out = torch.empty_like(start), torch.empty((1, 256), device="cuda")
+
+    def go():
+        h.copy_(start)
+        run = n_.PromptLayers(cfg, h, 1, 80, 0)
+        for layer, k, v in zip(weights.layers, state.k_pool, state.v_pool):
+            run.layer(layer, k, v)
+        out.copy_(run.finish())
+
+    go()
+    want = out.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        go()
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        torch.randn(1 << 16, device="cuda").sum().item()
