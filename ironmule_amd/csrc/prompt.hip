@@ -39,9 +39,8 @@ constexpr int kThreads = 256;
 //            (X of groups 0..3, then -16 X of groups 0..3), of hi for (0, 0), mid for (0, 1),
 //            lo for (1, 0) and zero for (1, 1): the A operands of two k-steps against
 //            (biases of the four groups, scales of the four groups).
-// A row holding a value that could overflow fp32 sums (|x| >= 2^96, infinities, NaN) has its
-// bit set in the (block, chunk)'s flag word and zeros for sums: its outputs are
-// computed value by value.
+// A group holding a value that could overflow fp32 sums (|x| >= 2^96, infinities, NaN) has NaN
+// for its sums: the product finds the row's outputs NaN and computes them value by value.
 constexpr int kGroupBytes = 4096;
 constexpr int kSumBytes = 2048;
 constexpr int kChunkBytes = 4 * kGroupBytes + kSumBytes;
@@ -53,59 +52,29 @@ __device__ __forceinline__ uint32_t exponent_max(uint32_t u, uint32_t m) {
   return m > hi ? m : hi;
 }
 
-// One row's chunk from the 32 lanes of a half wavefront into the (block, chunk) at `to`: lane l
-// holds piece l (columns 8 l .. of the chunk) in d.  Returns whether the row is flagged.
-__device__ __forceinline__ bool emit_row_chunk(uint4 d, int l, int row, char* to) {
-  const int g = l >> 3, c = l & 7;
+// One row's group g (0..3 of its chunk) from eight lanes into the (block, chunk) at `to`: lane c
+// (0..7) holds columns 8 c .. of the group in d.
+__device__ __forceinline__ void emit_group(uint4 d, int c, int g, int row, char* to) {
   *reinterpret_cast<uint4*>(to + g * kGroupBytes + c * 512 + row * 16) = pair_order(d);
   uint32_t e = exponent_max(d.x, 0u);
   e = exponent_max(d.y, e);
   e = exponent_max(d.z, e);
   e = exponent_max(d.w, e);
-  const uint64_t huge = __ballot(e >= kHuge);
-  const bool flagged = (uint32_t)(huge >> (threadIdx.x & 32)) != 0u;
-  float s = sum8(d);
+  float s = e >= kHuge ? __uint_as_float(0x7fc00000u) : sum8(d);
   s += dpp<0xB1>(s);   // lanes ^ 1
   s += dpp<0x4E>(s);   // lanes ^ 2
   s += dpp<0x141>(s);  // the other four of the eight
-  if (flagged) s = 0.0f;
-  // the four groups' sums in every lane, one term at a time
-  const int first = threadIdx.x & 32;
-  float left[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) left[k] = __shfl(s, first + 8 * k);
-  uint32_t term[4][4];
-#pragma unroll
-  for (int t = 0; t < 3; ++t) {
-    uint32_t a[4], b[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      a[k] = f32_to_bf16_bits(left[k]);
-      const float v = bf16_bits_to_f32(a[k]);
-      left[k] -= v;
-      b[k] = __float_as_uint(-16.0f * v) >> 16;
-    }
-    term[t][0] = a[0] | (a[1] << 16);
-    term[t][1] = a[2] | (a[3] << 16);
-    term[t][2] = b[0] | (b[1] << 16);
-    term[t][3] = b[2] | (b[3] << 16);
+  // lane t of the eight writes term t (hi, mid, lo, zero)
+  const uint32_t hi = f32_to_bf16_bits(s);
+  const float s1 = s - bf16_bits_to_f32(hi);
+  const uint32_t mid = f32_to_bf16_bits(s1);
+  const uint32_t lo = f32_to_bf16_bits(s1 - bf16_bits_to_f32(mid));
+  const uint32_t term = c == 0 ? hi : c == 1 ? mid : c == 2 ? lo : 0u;
+  if (c < 4) {
+    uint16_t* const at = reinterpret_cast<uint16_t*>(to + 4 * kGroupBytes + c * 512 + row * 16) + g;
+    at[0] = (uint16_t)term;
+    at[4] = (uint16_t)(__float_as_uint(-16.0f * bf16_bits_to_f32(term)) >> 16);
   }
-#pragma unroll
-  for (int k = 0; k < 4; ++k) term[3][k] = 0u;
-  // lane t of the half writes term t (hi, mid, lo, zero)
-  if (l < 4) {
-    const uint32_t w0 = l == 0 ? term[0][0] : l == 1 ? term[1][0] : l == 2 ? term[2][0] : 0u;
-    const uint32_t w1 = l == 0 ? term[0][1] : l == 1 ? term[1][1] : l == 2 ? term[2][1] : 0u;
-    const uint32_t w2 = l == 0 ? term[0][2] : l == 1 ? term[1][2] : l == 2 ? term[2][2] : 0u;
-    const uint32_t w3 = l == 0 ? term[0][3] : l == 1 ? term[1][3] : l == 2 ? term[2][3] : 0u;
-    *reinterpret_cast<uint4*>(to + 4 * kGroupBytes + l * 512 + row * 16) = make_uint4(w0, w1, w2, w3);
-  }
-  return flagged;
-}
-
-// Flag words are written a byte, eight rows, at a time.
-__device__ __forceinline__ void store_flags(uint32_t* flags, int64_t word, int rows8, uint32_t bits) {
-  reinterpret_cast<uint8_t*>(flags + word)[rows8] = (uint8_t)bits;
 }
 
 // One workgroup per (chunk, eight rows).  `src` (may be null): the x row of each packed row, -1
@@ -114,22 +83,15 @@ __device__ __forceinline__ void store_flags(uint32_t* flags, int64_t word, int r
 __global__ __launch_bounds__(kThreads) void pack_rows_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                              const int32_t* __restrict__ src,
                                                              const int32_t* __restrict__ expert, int tm, int M, int K,
-                                                             char* __restrict__ packed,
-                                                             uint32_t* __restrict__ flags) {
-  __shared__ uint32_t bits;
-  const int chunk = blockIdx.x, chunks = gridDim.x, block = blockIdx.y >> 2, rows8 = blockIdx.y & 3;
-  const int tid = threadIdx.x, l = tid & 31, at = tid >> 5;
+                                                             char* __restrict__ packed) {
+  const int chunk = blockIdx.x, chunks = gridDim.x, block = blockIdx.y >> 2;
+  const int l = threadIdx.x & 31, in = 8 * (blockIdx.y & 3) + (threadIdx.x >> 5);  // row of the block
   if (expert && expert[block / tm] < 0) return;
-  if (tid == 0) bits = 0u;
-  const int col = 256 * chunk + 8 * l, r = 32 * block + 8 * rows8 + at;
+  const int col = 256 * chunk + 8 * l, r = 32 * block + in;
   const int64_t row = src ? src[r] : (r < M ? r : -1);
   uint4 d = make_uint4(0u, 0u, 0u, 0u);
   if (row >= 0 && col < K) d = *reinterpret_cast<const uint4*>(x + row * ldx + col);
-  __syncthreads();
-  const int64_t word = (int64_t)block * chunks + chunk;
-  if (emit_row_chunk(d, l, 8 * rows8 + at, packed + word * kChunkBytes) && l == 0) atomicOr(&bits, 1u << at);
-  __syncthreads();
-  if (tid == 0) store_flags(flags, word, rows8, bits);
+  emit_group(d, l & 7, l >> 3, in, packed + ((int64_t)block * chunks + chunk) * kChunkBytes);
 }
 
 // ------------------------------------------------------------ the product
@@ -172,7 +134,6 @@ struct ProductProblem {
 struct ProductArgs {
   ProductProblem p[IMQ_PROMPT_MAX_PROBLEMS];
   const char* packed;
-  const uint32_t* flags;
   float* planes;          // fp32 partials (split, row, column of the launch), or null
   const int32_t* expert;  // per row tile: the expert of its rows, -1 none; null: one weight
   const int32_t* dest;    // per packed row: the output row, -1 none (with expert)
@@ -181,6 +142,7 @@ struct ProductArgs {
   int32_t count, M, G, chunks, blocks;
   int32_t row_tiles, col_tiles, splits, range;  // range: chunks per split
   int32_t y_f32;
+  char* act;              // PAIR: the packed rows of silu(gate) * up
 };
 
 // A value every lane holds, in a scalar register.
@@ -199,7 +161,11 @@ __device__ __forceinline__ bf16x8_t nibbles16(uint32_t u, uint32_t magic) {
 
 constexpr int kColumns = 128;  // of a workgroup
 
-template <int TM, bool AL>  // AL: G % 4 == 0 and 8-byte aligned scales and biases
+// AL: G % 4 == 0 and 8-byte aligned scales and biases.  PAIR: the launch's two weights are gate
+// and up; a workgroup takes the same 64 columns of both and writes bf16(silu(bf16(gate)) *
+// bf16(up)) as packed rows, the operand of the down projection, in place of two outputs that
+// another launch would read (512 x 2 x 9728: 20 MB written and read, and 12 us of that launch).
+template <int TM, bool AL, bool PAIR>
 __global__ __launch_bounds__(kThreads, 2) void product_kernel(ProductArgs a) {
   constexpr int kXB = TM;                      // row loads per wavefront and group
   constexpr int kSB = TM > 1 ? TM / 2 : 1;     // sum loads per wavefront and chunk
@@ -224,19 +190,20 @@ __global__ __launch_bounds__(kThreads, 2) void product_kernel(ProductArgs a) {
     expert = __builtin_amdgcn_readfirstlane(a.expert[rt]);
     if (expert < 0) return;
   }
-  int pi = 0;
-#pragma unroll
-  for (int i = 1; i < IMQ_PROMPT_MAX_PROBLEMS; ++i)
-    if (i < a.count && ct >= a.p[i].tile0) pi = i;
-  const ProductProblem P = pi == 0 ? a.p[0] : pi == 1 ? a.p[1] : a.p[2];
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int pi = PAIR ? wave >> 1 : 0;
+  if (!PAIR)
+#pragma unroll
+    for (int i = 1; i < IMQ_PROMPT_MAX_PROBLEMS; ++i)
+      if (i < a.count && ct >= a.p[i].tile0) pi = i;
+  const ProductProblem P = pi == 0 ? a.p[0] : pi == 1 ? a.p[1] : a.p[2];
   const int G = a.G, chunks = a.chunks, N = P.N;
   const int q0 = split * a.range, q1 = min(chunks, q0 + a.range);
 
   // this wavefront's columns: the problem's rows col0 .. of W.  Every load stays inside its
   // tensor: lanes past the last row read the last one, groups and blocks past the end the last.
-  const int col0 = (ct - P.tile0) * kColumns + wave * 32;
+  const int col0 = PAIR ? ct * (kColumns / 2) + (wave & 1) * 32 : (ct - P.tile0) * kColumns + wave * 32;
   const int rows = min(32, max(1, N - col0));
   const int64_t wrow = (int64_t)expert * N + min(col0, N - 1);
   const __amdgpu_buffer_rsrc_t wr = buffer_rsrc(P.w + wrow * (8 * G), (uint32_t)rows * (uint32_t)(32 * G));
@@ -270,13 +237,10 @@ __global__ __launch_bounds__(kThreads, 2) void product_kernel(ProductArgs a) {
   const uint32_t magic = in_vgpr(0x41804180u);
 
   // a chunk's weights: the four loads of a lane share a cache line
-  auto load_w = [&](int q) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t at = uniform(32u * (uint32_t)min(4 * q + i, G - 1));
-      const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(wr, woff, at, 0);
-      nwq[i] = make_uint4(v.x, v.y, v.z, v.w);
-    }
+  auto load_w = [&](int q, int i) {
+    const uint32_t at = uniform(32u * (uint32_t)min(4 * q + i, G - 1));
+    const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(wr, woff, at, 0);
+    nwq[i] = make_uint4(v.x, v.y, v.z, v.w);
   };
   auto load_scales = [&](int q) {
     const int c = min(q, chunks - 1);
@@ -295,14 +259,11 @@ __global__ __launch_bounds__(kThreads, 2) void product_kernel(ProductArgs a) {
       nbi = u32x2_t{b4[0] | (b4[1] << 16), b4[2] | (b4[3] << 16)};
     }
   };
-  auto load_x = [&](int q, int i, uint4* dst) {
-    const uint32_t base = (uint32_t)min(q, q1 - 1) * kChunkBytes + (uint32_t)i * kGroupBytes;
-#pragma unroll
-    for (int e = 0; e < kXB; ++e) {
-      const uint32_t at = uniform(piece[e] + base);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          xr, (__attribute__((address_space(3))) void*)(dst + (wave * kXB + e) * 64), 16, xoff, at, 0, 0);
-    }
+  auto load_x = [&](int q, int i, int e, uint4* dst) {
+    const uint32_t at =
+        uniform(piece[e] + (uint32_t)min(q, q1 - 1) * kChunkBytes + (uint32_t)i * kGroupBytes);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        xr, (__attribute__((address_space(3))) void*)(dst + (wave * kXB + e) * 64), 16, xoff, at, 0, 0);
   };
   auto load_sums = [&](int q) {
 #pragma unroll
@@ -343,18 +304,21 @@ __global__ __launch_bounds__(kThreads, 2) void product_kernel(ProductArgs a) {
       __builtin_amdgcn_s_waitcnt(vmcnt_imm(kXB + kSN));
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    load_x(q + (i + 3) / 4, (i + 3) % 4, xfree);
-    if (i == 0) {
-      load_sums(q);
-      load_w(q + 1);
-    }
+    if (i == 0) load_sums(q);
     if (i == 1) load_scales(q + 1);
-    __builtin_amdgcn_sched_barrier(0);
     const uint32_t two = i < 2 ? sc.x : sc.y;
     s[i & 1] = __uint_as_float((i & 1) ? (two & 0xffff0000u) : (two << 16));
 #pragma unroll
     for (int u = 0; u < TM; ++u) {
       const int at = (i * TM + u) & 1;
+      // this unit's share of the loads, between the units' MFMAs: issued all at once they
+      // held the wavefronts at the start of the group
+      __builtin_amdgcn_sched_barrier(0);
+      load_x(q + (i + 3) / 4, (i + 3) % 4, u, xfree);
+      if (i == 0)
+#pragma unroll
+        for (int k = u * 4 / TM; k < (u + 1) * 4 / TM; ++k) load_w(q + 1, k);
+      __builtin_amdgcn_sched_barrier(0);
       if (u + 1 < TM)
         read_unit(xs, u + 1, xa[at ^ 1]);
       else
@@ -393,13 +357,17 @@ __global__ __launch_bounds__(kThreads, 2) void product_kernel(ProductArgs a) {
   };
 
   load_scales(q0);
-  load_w(q0);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) load_w(q0, k);
   __builtin_amdgcn_sched_barrier(0);
-  load_x(q0, 0, x0);
+#pragma unroll
+  for (int e = 0; e < kXB; ++e) load_x(q0, 0, e, x0);
   __builtin_amdgcn_sched_barrier(0);
-  load_x(q0, 1, x1);
+#pragma unroll
+  for (int e = 0; e < kXB; ++e) load_x(q0, 1, e, x1);
   __builtin_amdgcn_sched_barrier(0);
-  load_x(q0, 2, x2);
+#pragma unroll
+  for (int e = 0; e < kXB; ++e) load_x(q0, 2, e, x2);
   __builtin_amdgcn_sched_barrier(0);
   __builtin_amdgcn_s_waitcnt(vmcnt_imm(kXB));
   __builtin_amdgcn_s_barrier();
@@ -423,22 +391,27 @@ __global__ __launch_bounds__(kThreads, 2) void product_kernel(ProductArgs a) {
   scale_unit(s[1], p[1], TM - 1);  // the range's last unit (4 TM is even)
   wait_vmem();  // the loads past the range's end, before the LDS is given up
 
-  // rows with values too large for the sums above: every output by itself
+  // Rows with values too large for the sums came out NaN: every output of the range by itself.
   const int col = col0 + n;
 #pragma unroll
   for (int m = 0; m < TM; ++m) {
-    const int block = rt * TM + m;
-    uint32_t mask = 0u;
-    if (block < a.blocks)
-      for (int q = lane; q < chunks; q += 64) mask |= a.flags[(int64_t)block * chunks + q];
-    if (__ballot(mask != 0u) == 0) continue;
+    bool nan = false;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) nan = nan || acc[m][e] != acc[m][e];
+    if (__ballot(nan) == 0) continue;
+    if (rt * TM + m >= a.blocks) continue;
+#pragma unroll 1
     for (int r = 0; r < 32; ++r) {
-      if (__ballot((mask >> r) & 1u) == 0) continue;
-      const char* const xrow = a.packed + (int64_t)block * block_bytes + r * 16;
+      bool mine = false;
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        mine = mine || (8 * (e >> 2) + 4 * h + (e & 3) == r && acc[m][e] != acc[m][e]);
+      if (__ballot(mine) == 0) continue;
+      const char* const xrow = a.packed + (int64_t)(rt * TM + m) * block_bytes + r * 16;
       float v = 0.0f;
-      if (split == 0 && col < N) {
+      if (col < N) {
         const int64_t row = wrow + n;
-        for (int g = 0; g < G; ++g) {
+        for (int g = 4 * q0; g < min(4 * q1, G); ++g) {
           const float sg = bf16_bits_to_f32(P.s[row * G + g]), bg = bf16_bits_to_f32(P.b[row * G + g]);
           const char* const xg = xrow + (int64_t)(g >> 2) * kChunkBytes + (g & 3) * kGroupBytes;
           for (int k = 0; k < 4; ++k) {
@@ -458,6 +431,41 @@ __global__ __launch_bounds__(kThreads, 2) void product_kernel(ProductArgs a) {
       for (int e = 0; e < 16; ++e)
         if (8 * (e >> 2) + 4 * h + (e & 3) == r) acc[m][e] = v;
     }
+  }
+
+  if (PAIR) {
+    // up to the gate's wavefront through x0 and x1, the products as rows of 64 columns in x2,
+    // then eight columns a lane into the packed rows
+    __syncthreads();
+    float* const half = reinterpret_cast<float*>((wave & 1) ? x1 : x0);
+    if (wave >= 2) {
+#pragma unroll
+      for (int m = 0; m < TM; ++m)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) half[(m * 16 + e) * 64 + lane] = acc[m][e];
+    }
+    __syncthreads();
+    if (wave < 2) {
+#pragma unroll
+      for (int m = 0; m < TM; ++m)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const float gate = bf16_bits_to_f32(f32_to_bf16_bits(acc[m][e]));
+          const float up = bf16_bits_to_f32(f32_to_bf16_bits(half[(m * 16 + e) * 64 + lane]));
+          const int r = m * 32 + 8 * (e >> 2) + 4 * h + (e & 3);
+          reinterpret_cast<uint16_t*>(x2)[r * 64 + wave * 32 + n] =
+              col < N ? f32_to_bf16_bits(gate / (1.0f + expf(-gate)) * up) : (uint16_t)0;
+        }
+    }
+    __syncthreads();
+    const int act_chunks = (N + 255) >> 8;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int block = rt * TM + i, r = tid >> 3, c = tid & 7;
+      if (block >= a.blocks) break;
+      emit_group(x2[(i * 32 + r) * 8 + c], c, ct & 3, r, a.act + ((int64_t)block * act_chunks + (ct >> 2)) * kChunkBytes);
+    }
+    return;
   }
 
   // lane (n, h) holds column n of rows 8 (e / 4) + 4 h + e % 4
@@ -582,47 +590,58 @@ __global__ __launch_bounds__(kSortThreads) void sort_pairs_kernel(const int32_t*
 constexpr int kD = 128;  // head dimension
 
 // h[row] += bf16(the planes' sum) (planes may be null); with `weight`, x = bf16(rms_norm(h) *
-// weight) packed.  A wavefront per row, eight rows per workgroup; lane l of a wavefront holds
-// the 8-column pieces l, l + 64, .. (at most NP).  Every load is issued before the first use.
+// weight) packed.  A workgroup per packed row, thread t holding the 8-column pieces t, t + 256, ..
+// (at most NP); rows past M are packed as zeros.  Consecutive workgroups go to the XCDs in turn:
+// eight consecutive rows, which share the packed lines, go to one.  A wavefront per row and
+// eight rows per workgroup took 14.5 us at 512 x 2560 with three planes, on 64 CUs.
 template <int NP>
-__global__ __launch_bounds__(512) void norm_pack_kernel(float* __restrict__ h, const float* __restrict__ planes,
-                                                        int splits, int64_t plane_stride,
-                                                        const uint16_t* __restrict__ weight, int M, int dim, float eps,
-                                                        int chunks, char* __restrict__ packed,
-                                                        uint32_t* __restrict__ flags) {
-  __shared__ uint32_t bits[2 * NP];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int row = 8 * blockIdx.x + wave;
+__global__ __launch_bounds__(kThreads) void norm_pack_kernel(float* __restrict__ h, const float* __restrict__ planes,
+                                                             int splits, int64_t plane_stride,
+                                                             const uint16_t* __restrict__ weight, int M, int dim,
+                                                             float eps, int chunks, char* __restrict__ packed) {
+  __shared__ float part[kThreads / 64];
+  const int tid = threadIdx.x, b = blockIdx.x & 63;
+  const int row = ((int)blockIdx.x & ~63) + (b & 7) * 8 + (b >> 3);
+  if (row >= (M + 31) / 32 * 32) return;
   const bool live = row < M;
-  if (threadIdx.x < 2 * NP) bits[threadIdx.x] = 0u;
-  float* const hr = h + (int64_t)min(row, M - 1) * dim;
-  const float* const pr = planes ? planes + (int64_t)min(row, M - 1) * dim : nullptr;
+  float* const hr = h + (int64_t)row * dim;
   float v[NP][8];
   uint4 wv[NP];
 #pragma unroll
   for (int i = 0; i < NP; ++i) {
-    const int col = 8 * (lane + 64 * i);
-    float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f), b = a;
+    const int col = 8 * (tid + kThreads * i);
+    float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f), c = a;
     wv[i] = make_uint4(0u, 0u, 0u, 0u);
     if (col < dim && live) {
       a = *reinterpret_cast<const float4*>(hr + col);
-      b = *reinterpret_cast<const float4*>(hr + col + 4);
+      c = *reinterpret_cast<const float4*>(hr + col + 4);
       if (weight) wv[i] = *reinterpret_cast<const uint4*>(weight + col);
     }
     v[i][0] = a.x, v[i][1] = a.y, v[i][2] = a.z, v[i][3] = a.w;
-    v[i][4] = b.x, v[i][5] = b.y, v[i][6] = b.z, v[i][7] = b.w;
+    v[i][4] = c.x, v[i][5] = c.y, v[i][6] = c.z, v[i][7] = c.w;
   }
-  if (pr) {
+  if (planes && live) {
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
-      const int col = 8 * (lane + 64 * i);
-      if (col >= dim || !live) continue;
+      const int col = 8 * (tid + kThreads * i);
+      if (col >= dim) continue;
+      const float* const pr = planes + (int64_t)row * dim + col;
       float d[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-      for (int s = 0; s < splits; ++s) {
-        const float4 a = *reinterpret_cast<const float4*>(pr + s * plane_stride + col);
-        const float4 b = *reinterpret_cast<const float4*>(pr + s * plane_stride + col + 4);
-        d[0] += a.x, d[1] += a.y, d[2] += a.z, d[3] += a.w;
-        d[4] += b.x, d[5] += b.y, d[6] += b.z, d[7] += b.w;
+      for (int s0 = 0; s0 < splits; s0 += 4) {
+        float4 p[4][2];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          p[s][0] = p[s][1] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+          if (s0 + s < splits) {
+            p[s][0] = *reinterpret_cast<const float4*>(pr + (s0 + s) * plane_stride);
+            p[s][1] = *reinterpret_cast<const float4*>(pr + (s0 + s) * plane_stride + 4);
+          }
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          d[0] += p[s][0].x, d[1] += p[s][0].y, d[2] += p[s][0].z, d[3] += p[s][0].w;
+          d[4] += p[s][1].x, d[5] += p[s][1].y, d[6] += p[s][1].z, d[7] += p[s][1].w;
+        }
       }
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[i][e] += bf16_bits_to_f32(f32_to_bf16_bits(d[e]));
@@ -636,11 +655,14 @@ __global__ __launch_bounds__(512) void norm_pack_kernel(float* __restrict__ h, c
   for (int i = 0; i < NP; ++i)
 #pragma unroll
     for (int e = 0; e < 8; ++e) ss = fmaf(v[i][e], v[i][e], ss);
-  const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)dim + eps);
+  ss = wave_sum(ss);
+  if ((tid & 63) == 0) part[tid >> 6] = ss;
   __syncthreads();
-  const int block = blockIdx.x >> 2, rows8 = blockIdx.x & 3;
+  const float inv = 1.0f / sqrtf(((part[0] + part[1]) + (part[2] + part[3])) / (float)dim + eps);
 #pragma unroll
   for (int i = 0; i < NP; ++i) {
+    const int piece = tid + kThreads * i;
+    if (piece >= 32 * chunks) break;  // (whole groups of eight lanes)
     const uint32_t w[4] = {wv[i].x, wv[i].y, wv[i].z, wv[i].w};
     uint32_t out[4];
 #pragma unroll
@@ -649,67 +671,40 @@ __global__ __launch_bounds__(512) void norm_pack_kernel(float* __restrict__ h, c
       const uint32_t hi = f32_to_bf16_bits(v[i][2 * e + 1] * inv * bf16_bits_to_f32(w[e] >> 16));
       out[e] = lo | (hi << 16);
     }
-    const int chunk = 2 * i + (lane >> 5);
-    // columns past the row (a last part-full chunk) and rows past M are packed as zeros
     uint4 d = make_uint4(out[0], out[1], out[2], out[3]);
-    if (!live || 8 * (lane + 64 * i) >= dim) d = make_uint4(0u, 0u, 0u, 0u);
-    if (chunk >= chunks) continue;
-    const int64_t word = (int64_t)block * chunks + chunk;
-    if (emit_row_chunk(d, lane & 31, 8 * rows8 + wave, packed + word * kChunkBytes) && (lane & 31) == 0)
-      atomicOr(&bits[chunk], 1u << wave);
+    if (!live || 8 * piece >= dim) d = make_uint4(0u, 0u, 0u, 0u);
+    emit_group(d, piece & 7, (piece >> 3) & 3, row & 31,
+               packed + ((int64_t)(row >> 5) * chunks + (piece >> 5)) * kChunkBytes);
   }
-  __syncthreads();
-  if ((int)threadIdx.x < chunks) store_flags(flags, (int64_t)block * chunks + threadIdx.x, rows8, bits[threadIdx.x]);
-}
-
-// act = bf16(silu(gate) * up), packed; one workgroup per (chunk, eight rows).
-__global__ __launch_bounds__(kThreads) void silu_pack_kernel(const uint16_t* __restrict__ gate,
-                                                             const uint16_t* __restrict__ up, int M, int K,
-                                                             char* __restrict__ packed,
-                                                             uint32_t* __restrict__ flags) {
-  __shared__ uint32_t bits;
-  const int chunk = blockIdx.x, chunks = gridDim.x, block = blockIdx.y >> 2, rows8 = blockIdx.y & 3;
-  const int tid = threadIdx.x, l = tid & 31, at = tid >> 5;
-  if (tid == 0) bits = 0u;
-  const int col = 256 * chunk + 8 * l, row = 32 * block + 8 * rows8 + at;
-  uint32_t out[4] = {0u, 0u, 0u, 0u};
-  if (row < M && col < K) {
-    const uint4 g4 = *reinterpret_cast<const uint4*>(gate + (int64_t)row * K + col);
-    const uint4 u4 = *reinterpret_cast<const uint4*>(up + (int64_t)row * K + col);
-    const uint32_t g[4] = {g4.x, g4.y, g4.z, g4.w}, u[4] = {u4.x, u4.y, u4.z, u4.w};
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float a = bf16_bits_to_f32(g[e] & 0xffffu), b = bf16_bits_to_f32(g[e] >> 16);
-      const uint32_t lo = f32_to_bf16_bits(a / (1.0f + expf(-a)) * bf16_bits_to_f32(u[e] & 0xffffu));
-      const uint32_t hi = f32_to_bf16_bits(b / (1.0f + expf(-b)) * bf16_bits_to_f32(u[e] >> 16));
-      out[e] = lo | (hi << 16);
-    }
-  }
-  __syncthreads();
-  const int64_t word = (int64_t)block * chunks + chunk;
-  if (emit_row_chunk(make_uint4(out[0], out[1], out[2], out[3]), l, 8 * rows8 + at, packed + word * kChunkBytes) && l == 0)
-    atomicOr(&bits, 1u << at);
-  __syncthreads();
-  if (tid == 0) store_flags(flags, word, rows8, bits);
 }
 
 // Per token and head: q and k heads get the per-head RMSNorm (rounded to bf16) and the
 // non-interleaved rotary embedding at the token's position, angles in double; q in place, k and
 // v into the slot's pools.  A workgroup per token, a wavefront per head at a time; lane i holds
-// dimensions i and i + 64, the pair that turns together.
-__global__ __launch_bounds__(kThreads) void prompt_rope_kernel(uint16_t* __restrict__ q,
-                                                               const uint16_t* __restrict__ k,
-                                                               const uint16_t* __restrict__ v,
-                                                               const uint16_t* __restrict__ q_norm,
-                                                               const uint16_t* __restrict__ k_norm,
-                                                               uint16_t* __restrict__ k_pool,
-                                                               uint16_t* __restrict__ v_pool, int Hq, int Hkv,
-                                                               int capacity, double log2_theta, float eps) {
+// dimensions i and i + 64, the pair that turns together.  Four wavefronts, each with its own
+// angles, took 10.9 us at 512 tokens of 48 heads.
+constexpr int kRopeThreads = 1024;
+__global__ __launch_bounds__(kRopeThreads) void prompt_rope_kernel(uint16_t* __restrict__ q,
+                                                                   const uint16_t* __restrict__ k,
+                                                                   const uint16_t* __restrict__ v,
+                                                                   const uint16_t* __restrict__ q_norm,
+                                                                   const uint16_t* __restrict__ k_norm,
+                                                                   uint16_t* __restrict__ k_pool,
+                                                                   uint16_t* __restrict__ v_pool, int Hq, int Hkv,
+                                                                   int capacity, double log2_theta, float eps) {
+  __shared__ float turn[2][64];
   const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  double sn, cs;
-  sincos((double)t * exp2(-(double)lane * (log2_theta / 64.0)), &sn, &cs);
-  const float s = (float)sn, c = (float)cs;
-  for (int hh = wave; hh < Hq + 2 * Hkv; hh += kThreads / 64) {
+  if (wave == 0) {
+    double sn, cs;
+    sincos((double)t * exp2(-(double)lane * (log2_theta / 64.0)), &sn, &cs);
+    turn[0][lane] = (float)sn;
+    turn[1][lane] = (float)cs;
+  }
+  const float qw[2] = {bf16_bits_to_f32(q_norm[lane]), bf16_bits_to_f32(q_norm[lane + 64])};
+  const float kw[2] = {bf16_bits_to_f32(k_norm[lane]), bf16_bits_to_f32(k_norm[lane + 64])};
+  __syncthreads();
+  const float s = turn[0][lane], c = turn[1][lane];
+  for (int hh = wave; hh < Hq + 2 * Hkv; hh += kRopeThreads / 64) {
     const bool is_q = hh < Hq, is_v = hh >= Hq + Hkv;
     const int head = is_q ? hh : is_v ? hh - Hq - Hkv : hh - Hq;
     const uint16_t* const src = is_q ? q + ((int64_t)t * Hq + head) * kD : (is_v ? v : k) + ((int64_t)t * Hkv + head) * kD;
@@ -719,11 +714,10 @@ __global__ __launch_bounds__(kThreads) void prompt_rope_kernel(uint16_t* __restr
       reinterpret_cast<uint32_t*>(dst)[lane] = reinterpret_cast<const uint32_t*>(src)[lane];
       continue;
     }
-    const uint16_t* const nw = is_q ? q_norm : k_norm;
     float a = bf16_bits_to_f32(src[lane]), b = bf16_bits_to_f32(src[lane + 64]);
     const float inv = 1.0f / sqrtf(wave_sum(fmaf(a, a, b * b)) / (float)kD + eps);
-    a = bf16_bits_to_f32(f32_to_bf16_bits(a * inv * bf16_bits_to_f32(nw[lane])));
-    b = bf16_bits_to_f32(f32_to_bf16_bits(b * inv * bf16_bits_to_f32(nw[lane + 64])));
+    a = bf16_bits_to_f32(f32_to_bf16_bits(a * inv * (is_q ? qw[0] : kw[0])));
+    b = bf16_bits_to_f32(f32_to_bf16_bits(b * inv * (is_q ? qw[1] : kw[1])));
     dst[lane] = f32_to_bf16_bits(a * c - b * s);
     dst[lane + 64] = f32_to_bf16_bits(a * s + b * c);
   }
@@ -732,29 +726,32 @@ __global__ __launch_bounds__(kThreads) void prompt_rope_kernel(uint16_t* __restr
 // Causal attention of a prompt: out[t][head] = softmax(q . K / sqrt(128)) V over positions
 // 0 .. t of one slot.
 //
-// A workgroup takes 64 queries of one head, a wavefront 16 of them, and walks the keys in
-// blocks of 64, the next block's K and V in flight in registers meanwhile.  Scores are K Q^T on
+// A workgroup takes 64 queries of one head, a wavefront 16 of them; four wavefronts walk the even
+// blocks of 64 keys and four the odd ones, each with the next block's K and V in flight in
+// registers, and the two halves are merged at the end.  Scores are K Q^T on
 // v_mfma_f32_16x16x32_bf16, so that a lane holds keys of one query: P^T is then the B operand
 // of V^T P^T without leaving its lane (key order 4 g .. of two 16-key tiles per 32-key step).  P
 // goes in as three bf16 terms that add up to its 24 bits, so P V keeps fp32's accuracy.  K lies
 // in LDS in rows of swizzled 16-byte pieces, V transposed with padded rows; both twice.  Heavy
-// query blocks, the last ones, start first.
+// query blocks, the last ones, start first.  The output goes out as packed rows, the operand of
+// the o projection, zeros past T (and past an odd last head).
 //
-// Bound by latency at a few hundred tokens (512 tokens of 32 heads: 256 workgroups, at most
-// eight key blocks each), where the same in torch operations (fp32 products, mask, softmax,
-// repeated heads) took about 300 us a layer.
+// Bound by the chain of key blocks at a few hundred tokens: 512 tokens of 32 heads are 256
+// workgroups of at most eight blocks (25.8 us with four wavefronts on all of them, and 5.3 us of
+// packing behind it).
 constexpr int kQ = 64, kKeys = 64, kVRow = 2 * kKeys + 8;  // V^T row bytes: 16 mod 128 banks apart
 
-__global__ __launch_bounds__(kThreads, 2) void prompt_attention_kernel(const uint16_t* __restrict__ q,
-                                                                       const uint16_t* __restrict__ k_pool,
-                                                                       const uint16_t* __restrict__ v_pool,
-                                                                       uint16_t* __restrict__ out, int T, int Hq,
-                                                                       int Hkv, int capacity) {
-  __shared__ __attribute__((aligned(16))) char kl[2][kKeys * 256];
-  __shared__ __attribute__((aligned(16))) char vl[2][kD * kVRow];
+__global__ __launch_bounds__(2 * kThreads) void prompt_attention_kernel(const uint16_t* __restrict__ q,
+                                                                        const uint16_t* __restrict__ k_pool,
+                                                                        const uint16_t* __restrict__ v_pool,
+                                                                        char* __restrict__ packed, int T, int Hq,
+                                                                        int Hkv, int capacity) {
+  __shared__ __attribute__((aligned(16))) char kl[2][2][kKeys * 256];
+  __shared__ __attribute__((aligned(16))) char vl[2][2][kD * kVRow];
   const int qblocks = gridDim.x / Hq;
   const int head = blockIdx.x % Hq, qb = qblocks - 1 - (int)blockIdx.x / Hq;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4;
+  const int half = threadIdx.x >> 8, tid = threadIdx.x & (kThreads - 1);
+  const int lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4;
   const int64_t kv = (int64_t)(head / (Hq / Hkv)) * capacity * kD;
   const int query = qb * kQ + 16 * wave + n;
   const int last = T - 1;
@@ -784,12 +781,12 @@ __global__ __launch_bounds__(kThreads, 2) void prompt_attention_kernel(const uin
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int p = tid + kThreads * i, row = p >> 4;
-      *reinterpret_cast<uint4*>(kl[b] + row * 256 + (((p & 15) ^ (row & 15)) << 4)) = kr[i];
+      *reinterpret_cast<uint4*>(kl[half][b] + row * 256 + (((p & 15) ^ (row & 15)) << 4)) = kr[i];
     }
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int p = tid + kThreads * i;
-      char* const to = vl[b] + 8 * (p & 15) * kVRow + 4 * (p >> 4);
+      char* const to = vl[half][b] + 8 * (p & 15) * kVRow + 4 * (p >> 4);
       const uint32_t a[4] = {va[i].x, va[i].y, va[i].z, va[i].w}, c[4] = {vb[i].x, vb[i].y, vb[i].z, vb[i].w};
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -804,13 +801,17 @@ __global__ __launch_bounds__(kThreads, 2) void prompt_attention_kernel(const uin
 #pragma unroll
   for (int d = 0; d < 8; ++d) o[d] = f32x4_t{};
   float top = -INFINITY, sum = 0.0f;
-  load(0);
+  // (a half without blocks of its own loads rows it does not use)
+  load(half);
   stage(0);
   __syncthreads();
-  for (int block = 0; block <= qb; ++block) {
-    if (block < qb) load(block + 1);
-    const char* const kb = kl[block & 1];
-    const char* const vt = vl[block & 1];
+  for (int at = 0; 2 * at <= qb; ++at) {
+    const int block = 2 * at + half;
+    const bool more = block + 2 <= qb;
+    if (more) load(block + 2);
+    if (block <= qb) {
+    const char* const kb = kl[half][at & 1];
+    const char* const vt = vl[half][at & 1];
     f32x4_t s[4];
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
@@ -872,18 +873,48 @@ __global__ __launch_bounds__(kThreads, 2) void prompt_attention_kernel(const uin
         o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(bf16x8_t, t2), o[d], 0, 0, 0);
       }
     }
-    if (block < qb) stage((block + 1) & 1);
+    }
+    if (more) stage((at + 1) & 1);
     __syncthreads();
   }
   sum = add_xor32(add_xor16(sum));
-  if (query > last) return;
-  uint16_t* const to = out + ((int64_t)query * Hq + head) * kD + 4 * g;
+
+  // the odd half's state to the even half's lanes
+  float* const state = reinterpret_cast<float*>(vl[0][0]);  // 34 floats a lane, 34 KB of the 68
+  if (half) {
+    state[tid] = top;
+    state[kThreads + tid] = sum;
 #pragma unroll
-  for (int d = 0; d < 8; ++d) {
-    uint32_t w[4];
+    for (int d = 0; d < 8; ++d)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) w[e] = f32_to_bf16_bits(o[d][e] / sum);
-    *reinterpret_cast<u32x2_t*>(to + 16 * d) = u32x2_t{w[0] | (w[1] << 16), w[2] | (w[3] << 16)};
+      for (int e = 0; e < 4; ++e) state[(2 + 4 * d + e) * kThreads + tid] = o[d][e];
+  }
+  __syncthreads();
+  uint16_t* const rows = reinterpret_cast<uint16_t*>(kl[0][0]);  // 64 x 128
+  if (!half) {
+    const float other = state[tid], most = fmaxf(top, other), base = most == -INFINITY ? 0.0f : most;
+    const float mine = exp2f((top - base) * kLog2e), theirs = exp2f((other - base) * kLog2e);
+    const float total = sum * mine + state[kThreads + tid] * theirs;
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+      uint32_t w[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        w[e] = f32_to_bf16_bits((o[d][e] * mine + state[(2 + 4 * d + e) * kThreads + tid] * theirs) / total);
+      const u32x2_t four = {w[0] | (w[1] << 16), w[2] | (w[3] << 16)};
+      *reinterpret_cast<u32x2_t*>(rows + (16 * wave + n) * kD + 16 * d + 4 * g) = query <= last ? four : u32x2_t{};
+    }
+  }
+  __syncthreads();
+  const int chunks = (Hq + 1) >> 1, blocks = (T + 31) >> 5;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int p = threadIdx.x + 2 * kThreads * i, r = p >> 4, c = p & 15, row = qb * kQ + r;
+    if (row >= 32 * blocks) continue;  // (whole groups of eight lanes)
+    char* const to = packed + ((int64_t)(row >> 5) * chunks + (head >> 1)) * kChunkBytes;
+    const uint4 d = *reinterpret_cast<const uint4*>(rows + r * kD + 8 * c);
+    emit_group(d, c & 7, 2 * (head & 1) + (c >> 3), row & 31, to);
+    if (head == Hq - 1 && !(head & 1)) emit_group(make_uint4(0u, 0u, 0u, 0u), c & 7, 2 + (c >> 3), row & 31, to);
   }
 }
 
@@ -946,36 +977,31 @@ ExpertPlan plan_experts(int experts, int pairs) {
   return p;
 }
 
-size_t flag_bytes(int64_t blocks, int chunks) { return round_up((size_t)blocks * chunks * 4, 256); }
-
-size_t packed_bytes(int64_t blocks, int K) {
-  const int chunks = ceil_div(K, 256);
-  return flag_bytes(blocks, chunks) + (size_t)blocks * chunks * kChunkBytes;
-}
+size_t packed_bytes(int64_t blocks, int K) { return (size_t)blocks * ceil_div(K, 256) * kChunkBytes; }
 
 void pack_rows(const uint16_t* x, int64_t ldx, const int32_t* src, const int32_t* expert, int tm, int M,
                int64_t blocks, int K, void* packed, hipStream_t stream) {
-  const int chunks = ceil_div(K, 256);
-  char* const base = static_cast<char*>(packed);
-  hipLaunchKernelGGL(pack_rows_kernel, dim3(chunks, (uint32_t)blocks * 4), dim3(kThreads), 0, stream, x, ldx, src, expert, tm, M, K,
-                     base + flag_bytes(blocks, chunks), reinterpret_cast<uint32_t*>(base));
+  hipLaunchKernelGGL(pack_rows_kernel, dim3(ceil_div(K, 256), (uint32_t)blocks * 4), dim3(kThreads), 0, stream, x, ldx,
+                     src, expert, tm, M, K, static_cast<char*>(packed));
 }
 
 template <int TM>
 void launch_product(const ProductArgs& a, bool al, uint32_t grid, hipStream_t stream) {
-  if (al)
-    hipLaunchKernelGGL((product_kernel<TM, true>), dim3(grid), dim3(kThreads), 0, stream, a);
+  if (a.act && al)
+    hipLaunchKernelGGL((product_kernel<TM, true, true>), dim3(grid), dim3(kThreads), 0, stream, a);
+  else if (a.act)
+    hipLaunchKernelGGL((product_kernel<TM, false, true>), dim3(grid), dim3(kThreads), 0, stream, a);
+  else if (al)
+    hipLaunchKernelGGL((product_kernel<TM, true, false>), dim3(grid), dim3(kThreads), 0, stream, a);
   else
-    hipLaunchKernelGGL((product_kernel<TM, false>), dim3(grid), dim3(kThreads), 0, stream, a);
+    hipLaunchKernelGGL((product_kernel<TM, false, false>), dim3(grid), dim3(kThreads), 0, stream, a);
 }
 
 // Fills the shape fields and launches; p[], planes and the expert tables are the caller's.
 int32_t run_product(ProductArgs& a, const Plan& p, const void* packed, int64_t blocks, int M, int K,
                     hipStream_t stream) {
   const int chunks = ceil_div(K, 256);
-  const char* base = static_cast<const char*>(packed);
-  a.flags = reinterpret_cast<const uint32_t*>(base);
-  a.packed = base + flag_bytes(blocks, chunks);
+  a.packed = static_cast<const char*>(packed);
   a.M = M;
   a.G = K / 64;
   a.chunks = chunks;
@@ -1055,25 +1081,21 @@ int32_t product_planes(const imq_qweight& w, const void* packed, int M, int N, i
 
 void norm_pack(float* h, const float* planes, int splits, int64_t stride, const uint16_t* weight, int M, int dim,
                float eps, void* packed, hipStream_t stream) {
-  const int chunks = ceil_div(dim, 256), blocks = ceil_div(M, 32);
-  char* const base = static_cast<char*>(packed);
-  char* const to = base + flag_bytes(blocks, chunks);
-  uint32_t* const flags = reinterpret_cast<uint32_t*>(base);
-  const dim3 grid(4 * blocks), threads(512);
-  const int pieces = ceil_div(dim, 512);
-  if (pieces <= 2)
-    hipLaunchKernelGGL(norm_pack_kernel<2>, grid, threads, 0, stream, h, planes, splits, stride, weight, M, dim, eps, chunks, to, flags);
-  else if (pieces <= 5)
-    hipLaunchKernelGGL(norm_pack_kernel<5>, grid, threads, 0, stream, h, planes, splits, stride, weight, M, dim, eps, chunks, to, flags);
-  else if (pieces <= 8)
-    hipLaunchKernelGGL(norm_pack_kernel<8>, grid, threads, 0, stream, h, planes, splits, stride, weight, M, dim, eps, chunks, to, flags);
+  const int chunks = ceil_div(dim, 256);
+  char* const to = static_cast<char*>(packed);
+  const dim3 grid(64 * ceil_div(M, 64)), threads(kThreads);
+  const int pieces = ceil_div(32 * chunks, kThreads);
+  if (pieces <= 1)
+    hipLaunchKernelGGL(norm_pack_kernel<1>, grid, threads, 0, stream, h, planes, splits, stride, weight, M, dim, eps, chunks, to);
+  else if (pieces <= 2)
+    hipLaunchKernelGGL(norm_pack_kernel<2>, grid, threads, 0, stream, h, planes, splits, stride, weight, M, dim, eps, chunks, to);
   else
-    hipLaunchKernelGGL(norm_pack_kernel<16>, grid, threads, 0, stream, h, planes, splits, stride, weight, M, dim, eps, chunks, to, flags);
+    hipLaunchKernelGGL(norm_pack_kernel<4>, grid, threads, 0, stream, h, planes, splits, stride, weight, M, dim, eps, chunks, to);
 }
 
 // The parts of a prompt's workspace, each 256-byte aligned.
 struct LayerSpace {
-  size_t x, attn_packed, act, q, k, v, attn, gate, up, planes, bytes;
+  size_t x, attn, act, q, k, v, planes, bytes;
 };
 
 int32_t check_shape(const imq_prompt_shape* s) {
@@ -1103,14 +1125,11 @@ LayerSpace layer_space(const imq_prompt_shape& s, int cus) {
   };
   l.planes = take((size_t)(so > sd ? so : sd) * T * s.hidden * 4);
   l.x = take(packed_bytes(blocks, s.hidden));
-  l.attn_packed = take(packed_bytes(blocks, qd));
+  l.attn = take(packed_bytes(blocks, qd));
   l.act = take(packed_bytes(blocks, s.intermediate));
   l.q = take((size_t)T * qd * 2);
   l.k = take((size_t)T * kd * 2);
   l.v = take((size_t)T * kd * 2);
-  l.attn = take((size_t)T * qd * 2);
-  l.gate = take((size_t)T * s.intermediate * 2);
-  l.up = take((size_t)T * s.intermediate * 2);
   l.bytes = at;
   return l;
 }
@@ -1157,44 +1176,41 @@ int32_t imq_prompt_layer(const imq_step_layer* layer, const imq_prompt_shape* sh
   char* const at = static_cast<char*>(workspace);
   float* const planes = reinterpret_cast<float*>(at + l.planes);
   uint16_t *const q = reinterpret_cast<uint16_t*>(at + l.q), *const k = reinterpret_cast<uint16_t*>(at + l.k);
-  uint16_t *const v = reinterpret_cast<uint16_t*>(at + l.v), *const attn = reinterpret_cast<uint16_t*>(at + l.attn);
-  uint16_t *const gate = reinterpret_cast<uint16_t*>(at + l.gate), *const up = reinterpret_cast<uint16_t*>(at + l.up);
+  uint16_t* const v = reinterpret_cast<uint16_t*>(at + l.v);
   const int64_t pool = (int64_t)s.slot * s.kv_heads * s.capacity * kD;
   hipStream_t st = static_cast<hipStream_t>(stream);
-
-  // several weights of one K as bf16 rows
-  auto project = [&](const imq_qweight* const* w, const int32_t* N, uint16_t* const* y, int count, int K, size_t packed) {
-    const Plan plan = plan_product(N, count, T, K, dev->cu_count, 1);
-    ProductArgs a;
-    memset(&a, 0, sizeof(a));
-    a.count = count;
-    int tile0 = 0;
-    for (int i = 0; i < count; ++i) {
-      a.p[i] = ProductProblem{w[i]->w, w[i]->scales, w[i]->biases, y[i], N[i], N[i], tile0};
-      tile0 += ceil_div(N[i], kColumns);
-    }
-    return run_product(a, plan, at + packed, blocks, T, K, st);
-  };
 
   const int32_t n = s.hidden;
   int splits = plan_product(&n, 1, T, s.intermediate, dev->cu_count).splits;  // of the layer before
   norm_pack(h, first ? nullptr : planes, splits, (int64_t)T * s.hidden, layer->input_norm, T, s.hidden, s.eps, at + l.x, st);
+  ProductArgs a;
+  memset(&a, 0, sizeof(a));
   uint16_t* const qkv[3] = {q, k, v};
-  if ((code = project(ws, ns, qkv, 3, s.hidden, l.x)) != IMQ_OK) return code;
-  hipLaunchKernelGGL(prompt_rope_kernel, dim3(T), dim3(kThreads), 0, st, q, k, v, layer->q_norm, layer->k_norm,
+  int tile0 = 0;
+  for (int i = 0; i < 3; ++i) {
+    a.p[i] = ProductProblem{ws[i]->w, ws[i]->scales, ws[i]->biases, qkv[i], ns[i], ns[i], tile0};
+    tile0 += ceil_div(ns[i], kColumns);
+  }
+  a.count = 3;
+  const Plan three = plan_product(ns, 3, T, s.hidden, dev->cu_count, 1);
+  if ((code = run_product(a, three, at + l.x, blocks, T, s.hidden, st)) != IMQ_OK) return code;
+  hipLaunchKernelGGL(prompt_rope_kernel, dim3(T), dim3(kRopeThreads), 0, st, q, k, v, layer->q_norm, layer->k_norm,
                      layer->k_pool + pool, layer->v_pool + pool, s.heads, s.kv_heads, s.capacity,
                      log2((double)s.theta), s.eps);
-  hipLaunchKernelGGL(prompt_attention_kernel, dim3(ceil_div(T, kQ) * s.heads), dim3(kThreads), 0, st, q,
-                     layer->k_pool + pool, layer->v_pool + pool, attn, T, s.heads, s.kv_heads, s.capacity);
-  pack_rows(attn, qd, nullptr, nullptr, 1, T, blocks, qd, at + l.attn_packed, st);
-  if ((code = product_planes(layer->o, at + l.attn_packed, T, s.hidden, qd, planes, dev->cu_count, &splits, st)) != IMQ_OK)
+  hipLaunchKernelGGL(prompt_attention_kernel, dim3(ceil_div(T, kQ) * s.heads), dim3(2 * kThreads), 0, st, q,
+                     layer->k_pool + pool, layer->v_pool + pool, at + l.attn, T, s.heads, s.kv_heads, s.capacity);
+  if ((code = product_planes(layer->o, at + l.attn, T, s.hidden, qd, planes, dev->cu_count, &splits, st)) != IMQ_OK)
     return code;
   norm_pack(h, planes, splits, (int64_t)T * s.hidden, layer->post_norm, T, s.hidden, s.eps, at + l.x, st);
-  uint16_t* const gu[2] = {gate, up};
-  if ((code = project(ws + 4, ns + 4, gu, 2, s.hidden, l.x)) != IMQ_OK) return code;
-  const int chunks = ceil_div(s.intermediate, 256);
-  hipLaunchKernelGGL(silu_pack_kernel, dim3(chunks, 4 * blocks), dim3(kThreads), 0, st, gate, up, T, s.intermediate,
-                     at + l.act + flag_bytes(blocks, chunks), reinterpret_cast<uint32_t*>(at + l.act));
+  memset(&a, 0, sizeof(a));
+  for (int i = 0; i < 2; ++i)
+    a.p[i] = ProductProblem{ws[4 + i]->w, ws[4 + i]->scales, ws[4 + i]->biases, nullptr, 0, s.intermediate, 0};
+  a.count = 2;
+  a.act = at + l.act;
+  // a column tile per group of act, up to whole chunks (the last ones, past N, are zeros)
+  Plan two = plan_product(ns + 4, 2, T, s.hidden, dev->cu_count, 1);
+  two.col_tiles = 4 * ceil_div(s.intermediate, 256);
+  if ((code = run_product(a, two, at + l.x, blocks, T, s.hidden, st)) != IMQ_OK) return code;
   if ((code = product_planes(layer->down, at + l.act, T, s.hidden, s.intermediate, planes, dev->cu_count, &splits, st)) != IMQ_OK)
     return code;
   return launched("prompt layer");
