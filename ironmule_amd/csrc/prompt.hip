@@ -737,8 +737,8 @@ __global__ __launch_bounds__(kRopeThreads) void prompt_rope_kernel(uint16_t* __r
 // the o projection, zeros past T (and past an odd last head).
 //
 // Bound by the chain of key blocks at a few hundred tokens: 512 tokens of 32 heads are 256
-// workgroups of at most eight blocks (25.8 us with four wavefronts on all of them, and 5.3 us of
-// packing behind it).
+// workgroups of at most eight blocks (21.7 us; 25.8 with four wavefronts on all of them and the
+// next block's loads waited for in every turn, and 5.3 us of packing behind it).
 constexpr int kQ = 64, kKeys = 64, kVRow = 2 * kKeys + 8;  // V^T row bytes: 16 mod 128 banks apart
 
 __global__ __launch_bounds__(2 * kThreads) void prompt_attention_kernel(const uint16_t* __restrict__ q,
@@ -750,44 +750,37 @@ __global__ __launch_bounds__(2 * kThreads) void prompt_attention_kernel(const ui
   __shared__ __attribute__((aligned(16))) char vl[2][2][kD * kVRow];
   const int qblocks = gridDim.x / Hq;
   const int head = blockIdx.x % Hq, qb = qblocks - 1 - (int)blockIdx.x / Hq;
-  const int half = threadIdx.x >> 8, tid = threadIdx.x & (kThreads - 1);
+  const int half = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), tid = threadIdx.x & (kThreads - 1);
   const int lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4;
   const int64_t kv = (int64_t)(head / (Hq / Hkv)) * capacity * kD;
   const int query = qb * kQ + 16 * wave + n;
   const int last = T - 1;
 
-  bf16x8_t qf[4];
-  {
-    const uint16_t* const src = q + ((int64_t)min(query, last) * Hq + head) * kD;
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-      qf[t] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(src + 32 * t + 8 * g));
-  }
-  uint4 kr[4], va[2], vb[2];
+  u32x4_t kr[4], va[2], vb[2];
   auto load = [&](int block) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int p = tid + kThreads * i;
-      kr[i] = *reinterpret_cast<const uint4*>(k_pool + kv + (int64_t)min(block * kKeys + (p >> 4), last) * kD + 8 * (p & 15));
+      kr[i] = *reinterpret_cast<const u32x4_t*>(k_pool + kv + (int64_t)min(block * kKeys + (p >> 4), last) * kD + 8 * (p & 15));
     }
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int p = tid + kThreads * i, key = block * kKeys + 2 * (p >> 4);
-      va[i] = *reinterpret_cast<const uint4*>(v_pool + kv + (int64_t)min(key, last) * kD + 8 * (p & 15));
-      vb[i] = *reinterpret_cast<const uint4*>(v_pool + kv + (int64_t)min(key + 1, last) * kD + 8 * (p & 15));
+      va[i] = *reinterpret_cast<const u32x4_t*>(v_pool + kv + (int64_t)min(key, last) * kD + 8 * (p & 15));
+      vb[i] = *reinterpret_cast<const u32x4_t*>(v_pool + kv + (int64_t)min(key + 1, last) * kD + 8 * (p & 15));
     }
   };
   auto stage = [&](int b) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int p = tid + kThreads * i, row = p >> 4;
-      *reinterpret_cast<uint4*>(kl[half][b] + row * 256 + (((p & 15) ^ (row & 15)) << 4)) = kr[i];
+      *reinterpret_cast<u32x4_t*>(kl[half][b] + row * 256 + (((p & 15) ^ (row & 15)) << 4)) = kr[i];
     }
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int p = tid + kThreads * i;
       char* const to = vl[half][b] + 8 * (p & 15) * kVRow + 4 * (p >> 4);
-      const uint32_t a[4] = {va[i].x, va[i].y, va[i].z, va[i].w}, c[4] = {vb[i].x, vb[i].y, vb[i].z, vb[i].w};
+      const u32x4_t a = va[i], c = vb[i];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         *reinterpret_cast<uint32_t*>(to + (2 * e) * kVRow) = __builtin_amdgcn_perm(c[e], a[e], 0x05040100u);
@@ -801,80 +794,92 @@ __global__ __launch_bounds__(2 * kThreads) void prompt_attention_kernel(const ui
 #pragma unroll
   for (int d = 0; d < 8; ++d) o[d] = f32x4_t{};
   float top = -INFINITY, sum = 0.0f;
-  // (a half without blocks of its own loads rows it does not use)
+  u32x4_t qr[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+    qr[t] = *reinterpret_cast<const u32x4_t*>(q + ((int64_t)min(query, last) * Hq + head) * kD + 32 * t + 8 * g);
   load(half);
   stage(0);
+  bf16x8_t qf[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    // the queries are waited for here: a wait at their first use inside the loop would cover
+    // the next block's loads, in every turn
+    asm volatile("" : "+v"(qr[t]));
+    qf[t] = __builtin_bit_cast(bf16x8_t, qr[t]);
+  }
   __syncthreads();
+  // Every turn loads and stages a block, past the last one rows that nothing uses: without
+  // branches around them the loads stay in flight over the turn.
   for (int at = 0; 2 * at <= qb; ++at) {
     const int block = 2 * at + half;
-    const bool more = block + 2 <= qb;
-    if (more) load(block + 2);
+    load(block + 2);
     if (block <= qb) {
-    const char* const kb = kl[half][at & 1];
-    const char* const vt = vl[half][at & 1];
-    f32x4_t s[4];
+      const char* const kb = kl[half][at & 1];
+      const char* const vt = vl[half][at & 1];
+      f32x4_t s[4];
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      s[b] = f32x4_t{};
+      for (int b = 0; b < 4; ++b) {
+        s[b] = f32x4_t{};
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const uint4 kf = *reinterpret_cast<const uint4*>(kb + (16 * b + n) * 256 + (((4 * t + g) ^ n) << 4));
-        s[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf), qf[t], s[b], 0, 0, 0);
-      }
-    }
-    float most = -INFINITY;
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        s[b][e] *= kScale;
-        if (block == qb && block * kKeys + 16 * b + 4 * g + e > query) s[b][e] = -INFINITY;
-        most = fmaxf(most, s[b][e]);  // (a NaN score comes back through its exponential)
-      }
-    most = fmaxf(most, top);
-    most = max_xor32(max_xor16(most));
-    const float base = most == -INFINITY ? 0.0f : most;
-    const float keep = exp2f((top - base) * kLog2e);
-    top = most;
-    sum *= keep;
-    uint32_t p0[4][2], p1[4][2], p2[4][2];  // the three terms, two keys a word
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-      for (int e = 0; e < 4; e += 2) {
-        uint32_t w[2][3];
-#pragma unroll
-        for (int z = 0; z < 2; ++z) {
-          const float v = exp2f((s[b][e + z] - base) * kLog2e);
-          sum += v;
-          w[z][0] = __float_as_uint(v);
-          const float r = v - __uint_as_float(w[z][0] & 0xffff0000u);
-          w[z][1] = __float_as_uint(r);
-          w[z][2] = __float_as_uint(r - __uint_as_float(w[z][1] & 0xffff0000u));
+        for (int t = 0; t < 4; ++t) {
+          const uint4 kf = *reinterpret_cast<const uint4*>(kb + (16 * b + n) * 256 + (((4 * t + g) ^ n) << 4));
+          s[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf), qf[t], s[b], 0, 0, 0);
         }
-        p0[b][e >> 1] = __builtin_amdgcn_perm(w[1][0], w[0][0], 0x07060302u);
-        p1[b][e >> 1] = __builtin_amdgcn_perm(w[1][1], w[0][1], 0x07060302u);
-        p2[b][e >> 1] = __builtin_amdgcn_perm(w[1][2], w[0][2], 0x07060302u);
       }
+      float most = -INFINITY;
 #pragma unroll
-    for (int d = 0; d < 8; ++d) {
+      for (int b = 0; b < 4; ++b)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) o[d][e] *= keep;
+        for (int e = 0; e < 4; ++e) {
+          s[b][e] *= kScale;
+          if (block == qb && block * kKeys + 16 * b + 4 * g + e > query) s[b][e] = -INFINITY;
+          most = fmaxf(most, s[b][e]);  // (a NaN score comes back through its exponential)
+        }
+      most = fmaxf(most, top);
+      most = max_xor32(max_xor16(most));
+      const float base = most == -INFINITY ? 0.0f : most;
+      const float keep = exp2f((top - base) * kLog2e);
+      top = most;
+      sum *= keep;
+      uint32_t p0[4][2], p1[4][2], p2[4][2];  // the three terms, two keys a word
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const char* const at = vt + (16 * d + n) * kVRow + 64 * j + 8 * g;
-        const u32x2_t lo = *reinterpret_cast<const u32x2_t*>(at), hi = *reinterpret_cast<const u32x2_t*>(at + 32);
-        const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, u32x4_t{lo.x, lo.y, hi.x, hi.y});
-        const u32x4_t t0 = {p0[2 * j][0], p0[2 * j][1], p0[2 * j + 1][0], p0[2 * j + 1][1]};
-        const u32x4_t t1 = {p1[2 * j][0], p1[2 * j][1], p1[2 * j + 1][0], p1[2 * j + 1][1]};
-        const u32x4_t t2 = {p2[2 * j][0], p2[2 * j][1], p2[2 * j + 1][0], p2[2 * j + 1][1]};
-        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(bf16x8_t, t0), o[d], 0, 0, 0);
-        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(bf16x8_t, t1), o[d], 0, 0, 0);
-        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(bf16x8_t, t2), o[d], 0, 0, 0);
+      for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; e += 2) {
+          uint32_t w[2][3];
+#pragma unroll
+          for (int z = 0; z < 2; ++z) {
+            const float v = exp2f((s[b][e + z] - base) * kLog2e);
+            sum += v;
+            w[z][0] = __float_as_uint(v);
+            const float r = v - __uint_as_float(w[z][0] & 0xffff0000u);
+            w[z][1] = __float_as_uint(r);
+            w[z][2] = __float_as_uint(r - __uint_as_float(w[z][1] & 0xffff0000u));
+          }
+          p0[b][e >> 1] = __builtin_amdgcn_perm(w[1][0], w[0][0], 0x07060302u);
+          p1[b][e >> 1] = __builtin_amdgcn_perm(w[1][1], w[0][1], 0x07060302u);
+          p2[b][e >> 1] = __builtin_amdgcn_perm(w[1][2], w[0][2], 0x07060302u);
+        }
+#pragma unroll
+      for (int d = 0; d < 8; ++d) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[d][e] *= keep;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const char* const at = vt + (16 * d + n) * kVRow + 64 * j + 8 * g;
+          const u32x2_t lo = *reinterpret_cast<const u32x2_t*>(at), hi = *reinterpret_cast<const u32x2_t*>(at + 32);
+          const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, u32x4_t{lo.x, lo.y, hi.x, hi.y});
+          const u32x4_t t0 = {p0[2 * j][0], p0[2 * j][1], p0[2 * j + 1][0], p0[2 * j + 1][1]};
+          const u32x4_t t1 = {p1[2 * j][0], p1[2 * j][1], p1[2 * j + 1][0], p1[2 * j + 1][1]};
+          const u32x4_t t2 = {p2[2 * j][0], p2[2 * j][1], p2[2 * j + 1][0], p2[2 * j + 1][1]};
+          o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(bf16x8_t, t0), o[d], 0, 0, 0);
+          o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(bf16x8_t, t1), o[d], 0, 0, 0);
+          o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(bf16x8_t, t2), o[d], 0, 0, 0);
+        }
       }
     }
-    }
-    if (more) stage((at + 1) & 1);
+    stage((at + 1) & 1);
     __syncthreads();
   }
   sum = add_xor32(add_xor16(sum));
