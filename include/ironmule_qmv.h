@@ -294,6 +294,13 @@ IMQ_API int32_t imq_qmv_grouped_ws(const imq_problem* problems, int32_t count, i
                                    int32_t group_size, int32_t bits, int32_t y_dtype,
                                    float* workspace, size_t workspace_bytes, void* stream);
 
+/* imq_qmv_grouped_workspace (contiguous x rows) and imq_qmv_grouped_ws for one weight, without
+ * the problem array. */
+IMQ_API size_t imq_qmv_workspace(int32_t M, int32_t N, int32_t K);
+IMQ_API int32_t imq_qmv_ws(const uint32_t* w, const uint16_t* scales, const uint16_t* biases, const uint16_t* x,
+                           int64_t ldx, void* y, int64_t ldy, int32_t M, int32_t N, int32_t K, int32_t group_size,
+                           int32_t bits, int32_t y_dtype, float* workspace, size_t workspace_bytes, void* stream);
+
 /* Bytes of the library's static split scratch (one per device, held until the process
  * ends), the largest split workspace imq_qmv_grouped_noalloc serves. */
 #define IMQ_NOALLOC_SCRATCH_BYTES (8u << 20)

@@ -125,6 +125,8 @@ _SIGNATURES = {
     "imq_qmv_grouped_workspace": ([ctypes.POINTER(Problem), _I32, _I32], ctypes.c_size_t),
     "imq_qmv_grouped_ws": ([ctypes.POINTER(Problem), _I32, _I32, _I32, _I32, _I32, _P,
                             ctypes.c_size_t, _P], _I32),
+    "imq_qmv_workspace": ([_I32, _I32, _I32], ctypes.c_size_t),
+    "imq_qmv_ws": ([_P, _P, _P, _P, _I64, _P, _I64, _I32, _I32, _I32, _I32, _I32, _I32, _P, ctypes.c_size_t, _P], _I32),
     "imq_qmv_grouped_noalloc": ([ctypes.POINTER(Problem), _I32, _I32, _I32, _I32, _I32, _P],
                                 _I32),
     "imq_qmv_gate_up_silu": ([_P, _P, _P, _P, _P, _P, _P, _I64, _P, _I64, _I32, _I32, _I32, _I32,
@@ -248,18 +250,29 @@ def device_check() -> tuple[int, str, int]:
     return int(code), arch.value.decode(), int(cus.value)
 
 
-def _stream(stream) -> ctypes.c_void_p:
-    if stream is None:
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(int(stream.cuda_stream))
+def _stream(stream) -> int:
+    """The handle of a torch stream, or of the current device's current stream."""
+    if stream is None:  # torch.cuda.current_stream().cuda_stream without the Stream object (1.5 us of a call's 12)
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    return int(stream.cuda_stream)
 
 
-def _ptr(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(t.data_ptr())
+def _ptr(t: torch.Tensor) -> int:
+    return t.data_ptr()
 
 
 def check_weights(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor) -> tuple[int, int]:
     """(N, K) of a well-formed 4-bit group-64 weight on a GPU, else ValueError."""
+    shape = w.shape
+    if len(shape) == 2:  # one pass for a well-formed weight; the messages are below
+        n, words = shape
+        groups = (n, words >> 3)
+        if (words & 7 == 0 and (w.dtype is torch.int32 or w.dtype is torch.uint32)
+                and scales.dtype is torch.bfloat16 and biases.dtype is torch.bfloat16
+                and scales.shape == groups and biases.shape == groups
+                and w.is_cuda and scales.is_cuda and biases.is_cuda
+                and w.is_contiguous() and scales.is_contiguous() and biases.is_contiguous()):
+            return n, words * 8
     if w.dtype not in (torch.int32, torch.uint32):
         raise ValueError(f"w must be int32/uint32 packed words, got {w.dtype}")
     if w.dim() != 2:
@@ -287,11 +300,11 @@ def qmv(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor, x: torch.Te
     sweep.  x is bf16 (K,) or (M, K); y is bf16 (default) or fp32, shape (M, N)."""
     n, k = check_weights(w, scales, biases)
     x2 = x.reshape(1, -1) if x.dim() == 1 else x
-    if x2.dim() != 2 or int(x2.shape[1]) != k:
+    if x2.dim() != 2 or x2.shape[1] != k:
         raise ValueError(f"x must be (M, {k}), got {tuple(x.shape)}")
-    if x2.dtype != torch.bfloat16:
+    if x2.dtype is not torch.bfloat16:
         raise ValueError(f"x must be bfloat16, got {x2.dtype}")
-    m = int(x2.shape[0])
+    m = x2.shape[0]
     if not 1 <= m <= MAX_ROWS:
         raise ValueError(f"the qmv kernels take 1 to {MAX_ROWS} rows, got {m}")
     if not x2.is_contiguous():
@@ -301,16 +314,19 @@ def qmv(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor, x: torch.Te
         raise ValueError(f"output must be bfloat16 or float32, got {dtype}")
     if out is None:
         out = torch.empty((m, n), dtype=dtype, device=w.device)
-    elif tuple(out.shape) != (m, n) or out.dtype != dtype or not out.is_contiguous():
+    elif out.shape != (m, n) or out.dtype != dtype or not out.is_contiguous():
         raise ValueError("out must be a contiguous (M, N) tensor of the output dtype")
+    code = _DTYPE_CODE[dtype]
+    library = _lib or lib()
     if m >= 3:  # the shared-weight MFMA path, with a workspace for split groups
-        probs = (Problem * 1)()
-        probs[0] = Problem(w.data_ptr(), scales.data_ptr(), biases.data_ptr(), x2.data_ptr(), k,
-                           out.data_ptr(), n, n, k)
-        _grouped_launch(probs, 1, m, dtype, w.device, stream)
+        nbytes = library.imq_qmv_workspace(m, n, k)
+        ws = _workspace(nbytes, w.device, stream) if nbytes else None
+        _check(library.imq_qmv_ws(w.data_ptr(), scales.data_ptr(), biases.data_ptr(), x2.data_ptr(), k,
+                                  out.data_ptr(), n, m, n, k, GROUP_SIZE, BITS, code,
+                                  ws.data_ptr() if nbytes else None, ws.numel() * 4 if nbytes else 0, _stream(stream)))
         return out
-    _check(lib().imq_qmv(_ptr(w), _ptr(scales), _ptr(biases), _ptr(x2), k, _ptr(out), n,
-                         m, n, k, GROUP_SIZE, BITS, _DTYPE_CODE[dtype], _stream(stream)))
+    _check(library.imq_qmv(w.data_ptr(), scales.data_ptr(), biases.data_ptr(), x2.data_ptr(), k, out.data_ptr(), n,
+                           m, n, k, GROUP_SIZE, BITS, code, _stream(stream)))
     return out
 
 
@@ -438,12 +454,14 @@ def gather_qmv(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor, x: t
     """MoE gather (imq_gather_qmv): y[p] = x[p // rows_per_x] @ dequant(w[idx[p]]).T for the
     P = idx.numel() pairs; w (E, N, K/8) int32, scales/biases (E, N, K/64) bf16, x (R, K)
     bf16 contiguous rows, idx int32 on the device.  Returns (P, N)."""
-    if w.dim() != 3 or w.dtype != torch.int32:
+    if w.dim() != 3 or w.dtype is not torch.int32:
         raise ValueError("w must be an (experts, N, K/8) int32 tensor")
-    e, n, k = int(w.shape[0]), int(w.shape[1]), int(w.shape[2]) * 8
+    e, n, words = w.shape
+    k = words * 8
+    groups = (e, n, k // GROUP_SIZE)
     for name, t in (("scales", scales), ("biases", biases)):
-        if tuple(t.shape) != (e, n, k // GROUP_SIZE) or t.dtype != torch.bfloat16:
-            raise ValueError(f"{name} must be a bf16 tensor of shape {(e, n, k // GROUP_SIZE)}")
+        if t.shape != groups or t.dtype is not torch.bfloat16:
+            raise ValueError(f"{name} must be a bf16 tensor of shape {groups}")
         if not t.is_contiguous():
             raise ValueError(f"{name} must be contiguous")
     if not w.is_contiguous():
@@ -452,8 +470,9 @@ def gather_qmv(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor, x: t
         raise ValueError(f"x must be a contiguous bf16 (rows, {k}) tensor")
     if idx.dtype != torch.int32 or idx.device != w.device:
         raise ValueError("idx must be an int32 tensor on the weights' device")
-    idx = idx.reshape(-1).contiguous()
-    pairs = int(idx.numel())
+    if idx.dim() != 1 or not idx.is_contiguous():
+        idx = idx.reshape(-1).contiguous()
+    pairs = idx.shape[0]
     if pairs < 1 or rows_per_x < 1 or -(-pairs // rows_per_x) > x.shape[0]:
         raise ValueError("need at least one pair and ceil(pairs / rows_per_x) activation rows")
     if out is None:

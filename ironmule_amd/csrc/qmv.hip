@@ -3739,6 +3739,22 @@ int32_t imq_qmv_grouped_ws(const imq_problem* problems, int32_t count, int32_t M
   return launch(a, dev, static_cast<hipStream_t>(stream), workspace, workspace_bytes);
 }
 
+size_t imq_qmv_workspace(int32_t M, int32_t N, int32_t K) {
+  imq_problem p;
+  memset(&p, 0, sizeof(p));
+  p.N = N;
+  p.K = K;
+  p.ldx = K;
+  return imq_qmv_grouped_workspace(&p, 1, M);
+}
+
+int32_t imq_qmv_ws(const uint32_t* w, const uint16_t* scales, const uint16_t* biases, const uint16_t* x, int64_t ldx,
+                   void* y, int64_t ldy, int32_t M, int32_t N, int32_t K, int32_t group_size, int32_t bits,
+                   int32_t y_dtype, float* workspace, size_t workspace_bytes, void* stream) {
+  const imq_problem p = {w, scales, biases, x, ldx, y, ldy, N, K};
+  return imq_qmv_grouped_ws(&p, 1, M, group_size, bits, y_dtype, workspace, workspace_bytes, stream);
+}
+
 int32_t imq_qmv_grouped_noalloc(const imq_problem* problems, int32_t count, int32_t M,
                                 int32_t group_size, int32_t bits, int32_t y_dtype, void* stream) {
   LaunchArgs a;

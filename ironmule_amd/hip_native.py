@@ -31,6 +31,7 @@ within PROBE_TOLERANCE.
 
 from __future__ import annotations
 
+import math
 import time
 from typing import Any
 
@@ -68,6 +69,8 @@ def _route(x: torch.Tensor, k: int) -> str:
 
 def _qmv(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
          out_dtype: torch.dtype | None = None) -> torch.Tensor:
+    if x.dim() == 2:
+        return _native.qmv(w, scales, biases, x, out_dtype=out_dtype or x.dtype)
     n, k = int(w.shape[0]), int(w.shape[1]) * 8
     y = _native.qmv(w, scales, biases, x.reshape(-1, k).contiguous(),
                     out_dtype=out_dtype or x.dtype)
@@ -98,10 +101,11 @@ def _gather_route(x: torch.Tensor, indices: torch.Tensor):
     Any other broadcast is expanded to one row per pair first."""
     if x.dtype != torch.bfloat16 or x.shape[-2] != 1:
         return None
-    pairs = tuple(torch.broadcast_shapes(x.shape[:-2], indices.shape))
-    if torch.Size(pairs).numel() > GATHER_MAX:
+    lead, pairs = tuple(x.shape[:-2]), tuple(indices.shape)
+    if lead != pairs and not (pairs and lead == pairs[:-1] + (1,)):
+        pairs = tuple(torch.broadcast_shapes(lead, pairs))
+    if math.prod(pairs) > GATHER_MAX:
         return None
-    lead = tuple(x.shape[:-2])
     if lead == pairs:
         return pairs, 1
     if pairs and lead == pairs[:-1] + (1,):
@@ -120,8 +124,12 @@ def gather_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases
     pairs, rows_per_x = route
     if rows_per_x == 0:
         x, rows_per_x = x.expand(*pairs, *x.shape[-2:]), 1
-    experts = indices.expand(pairs).reshape(-1).to(torch.int32).contiguous()
-    rows = x.reshape(-1, x.shape[-1]).contiguous()
+    experts = (indices if indices.shape == pairs else indices.expand(pairs)).reshape(-1)
+    if experts.dtype is not torch.int32:
+        experts = experts.to(torch.int32)
+    rows = x.reshape(-1, x.shape[-1])
+    if not rows.is_contiguous():
+        rows = rows.contiguous()
     y = _native.gather_qmv(w, scales, biases, rows, experts, rows_per_x=rows_per_x)
     return y.reshape(*pairs, 1, int(w.shape[1]))
 
