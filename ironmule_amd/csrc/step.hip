@@ -1317,9 +1317,12 @@ void attention_split(int B, int Hkv, int span, int* splits, int* cps) {
 #ifndef IMQ_ATTN_WIDE_WAVES
 #define IMQ_ATTN_WIDE_WAVES 12
 #endif
-// From 64 (request, KV head) pairs (8 requests over 8 KV heads): at 8 requests the fused
-// launch took 12.0 us against 13.5 with 4 wavefronts per workgroup, at 4 requests 11.7
-// against 10.6.
+// From 64 (request, KV head) pairs (8 requests over 8 KV heads): at 8 requests over 512 keys the
+// fused launch took 12.0 us against 13.5 with 4 wavefronts per workgroup, at 4 requests 11.7
+// against 10.6.  And for any pairs whose keys are more chunks than a merge loads at once, where
+// the narrow plan's splits pass a second merge round: one request over 1010 / 1080 / 2048 / 8192
+// keys 9.5 / 12.7 / 15.7 / 32.3 us narrow and 11.8 / 11.6 / 12.3 / 19.3 wide, four over 1010 /
+// 1080 / 8192 13.3 / 16.8 / 41.0 and 12.6 / 12.5 / 28.8.
 #ifndef IMQ_ATTN_WIDE_PAIRS
 #define IMQ_ATTN_WIDE_PAIRS 64
 #endif
@@ -1328,16 +1331,17 @@ void attention_split(int B, int Hkv, int span, int* splits, int* cps) {
 #endif
 constexpr int kWideWaves = IMQ_ATTN_WIDE_WAVES;
 
-// The wide plan, from IMQ_ATTN_WIDE_PAIRS (request, KV head) pairs: a workgroup of
-// kWideWaves wavefronts takes a split of at least one unit per wavefront, and the splits
-// target one workgroup per CU.  Never more splits than attention_split's plan, so its
-// workspace size holds.
+// The wide plan: a workgroup of kWideWaves wavefronts takes a split of at least one unit per
+// wavefront, and the splits fill at most one workgroup per CU: a few more than 256 workgroups
+// are a second round of whole splits (20 requests over 512 keys: 320 workgroups 25.5 us, 160
+// of them 14.3; 14 requests 336: 19.2, 224: 14.1).  Never more splits than attention_split's
+// plan, so its workspace size holds.
 bool attention_wide_split(int B, int Hkv, int span, int* splits, int* cps) {
   const int pairs = B * Hkv;
-  if (pairs < IMQ_ATTN_WIDE_PAIRS) return false;
   const int chunks = (span + kChunk - 1) / kChunk;
+  if (pairs < IMQ_ATTN_WIDE_PAIRS && chunks <= kMergeBatch) return false;
   const int min_c = (kWideWaves * kUnit + kChunk - 1) / kChunk;
-  int sp = (IMQ_ATTN_WIDE_WORKGROUPS + pairs - 1) / pairs;
+  int sp = IMQ_ATTN_WIDE_WORKGROUPS / pairs;
   sp = sp < chunks ? sp : chunks;
   sp = sp > 1 ? sp : 1;
   int c = (chunks + sp - 1) / sp;

@@ -230,6 +230,32 @@ def test_attention_fused_matches_the_oracle_and_writes_the_same_pools(env, B, po
     assert np.array_equal(bf16_bits(b[0]), first)
 
 
+@pytest.mark.parametrize("B,positions,cap", [(1, [1023], 1024), (1, [1024], 1025), (1, [2099], 2100),
+                                             (4, [0, 1087, 640, 1500], 1600), (6, [5, 1279, 64, 1200, 1, 900], 1280),
+                                             (14, [37 * r for r in range(14)], 520),
+                                             (20, [26 * r for r in range(20)], 520)])
+def test_attention_fused_long_contexts_and_split_counts(env, B, positions, cap):
+    """The wide plan below 64 (request, KV head) pairs, from 17 chunks of 64 keys (16 keep the
+    narrow one), and request counts whose pairs do not divide 256: as the test above."""
+    torch, n, do, orc = env
+    announce("attention fused long", B, cap)
+    slots = list(RNG.permutation(B + 1)[:B].astype(int))
+    a, b, fused, counters = _fused_pair(torch, n, B, positions, slots, B + 1, cap=cap, max_len=cap, seed=B + cap)
+    got = _fused_against_oracle(a, b, positions, slots, B + 1, cap)
+    q_rot = _vals(fused_q_rot(torch, n, fused))
+    kp, vp = _vals(a[1]), _vals(a[2])
+    for r in range(B):
+        L = positions[r] + 1
+        ref = do.attention(q_rot[r].reshape(32, 128), kp[slots[r], :, :L], vp[slots[r], :, :L], 128 ** -0.5)
+        err = np.abs(got[r].reshape(32, 128) - ref)
+        assert (err <= _ulp(ref) + 1e-5 * np.abs(vp[slots[r], :, :L]).max()).all(), (r, err.max())
+    assert not counters.any()
+    first = bf16_bits(b[0]).copy()
+    n.attention_fused(*fused)
+    torch.cuda.synchronize()
+    assert np.array_equal(bf16_bits(b[0]), first)
+
+
 def fused_q_rot(torch, n, fused):
     """The rotated q of the fused call's inputs, by imq_qk_norm_rope on fresh pools."""
     q, k, v, qn, kn, pos, sl, kp, vp, out, max_len, theta, eps, ws, counters = fused
