@@ -111,16 +111,17 @@ __global__ __launch_bounds__(kThreads) void pack_rows_kernel(const uint16_t* __r
 // One barrier per group.  Within a wavefront the scaling of one tile, the LDS reads of the
 // next and the unpacking of the next group's weights are issued between a tile's MFMAs.
 //
-// What bounds it (K = 2560, 512 workgroups of TM = 4, two per CU; a group takes 1.03 us):
-// MFMA busy 33% of the launch and the VALU about as long (16 FMAs and 8 unpackings per four
-// MFMAs), and the two overlap only in part: without any load or LDS read a group takes 0.61
-// us, the row loads add 0.29 and the weights 0.10.  About 1.04 PFLOP/s marginal, 750-870 TFLOP/s
-// with a launch's start and end.  128 columns x 64 rows as 2 x 2 tiles per wavefront (half the
-// LDS reads, twice the unpacking) and eight wavefronts over 256 columns measured the same;
-// 128 x 64 per wavefront 930 TFLOP/s on large launches, but its 256-column tiles leave a
-// prompt of 512 rows with too few workgroups.  Against imq_dequant and a library product (two
-// conversions of the activations besides): 1024 x 9728 x 2560 89.7 -> 81.3 us in fp16, 77 x
-// 2560 x 9728 70.9 -> 27.6 us in fp32.
+// What bounds it (K = 2560, 512 workgroups of TM = 4, two per CU; a group takes 1.0 us): the
+// MFMAs (half of that time) and the 16 FMAs and 8 unpackings per four of them, which overlap only
+// in part.  Without loads and LDS reads, on constant data, a group takes 0.61 us; taking out the
+// waits, the barriers or the distance to memory (every load from one line) changes it by 3% or
+// less.  860 TFLOP/s on large launches, 755 at 512 workgroups with a launch's start and end.
+// Not faster: 64 x 64 per wavefront (half the LDS reads, twice the unpacking), eight wavefronts
+// over 256 columns, one wait for a unit's four operands in place of one each (large launches 4%
+// faster, 1024 x 9728 2% slower); 128 x 64 per wavefront took 930 TFLOP/s in an earlier form, but
+// its 256-column tiles leave a prompt of 512 rows with too few workgroups.  Against imq_dequant and a library product (two conversions of the
+// activations besides): 1024 x 9728 x 2560 90 -> 80 us in fp16, 77 x 2560 x 9728 70.9 -> 26 us in
+// fp32.
 struct ProductProblem {
   const uint32_t* w;
   const uint16_t* s;
@@ -434,29 +435,30 @@ __global__ __launch_bounds__(kThreads, 2) void product_kernel(ProductArgs a) {
   }
 
   if (PAIR) {
-    // up to the gate's wavefront through x0 and x1, the products as rows of 64 columns in x2,
-    // then eight columns a lane into the packed rows
+    // The gate's and the up's wavefront of the same columns exchange half their values through
+    // x0 or x1, so that both apply the activation; the products as rows of 64 columns in x2, then
+    // eight columns a lane into the packed rows.
     __syncthreads();
-    float* const half = reinterpret_cast<float*>((wave & 1) ? x1 : x0);
-    if (wave >= 2) {
+    float* const shared = reinterpret_cast<float*>((wave & 1) ? x1 : x0);
+    const int keep = wave < 2 ? 0 : 8;  // the half of each tile's 16 values this wavefront computes
 #pragma unroll
-      for (int m = 0; m < TM; ++m)
+    for (int m = 0; m < TM; ++m)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) half[(m * 16 + e) * 64 + lane] = acc[m][e];
-    }
+      for (int e = 0; e < 8; ++e)
+        shared[((m * 2 + (wave < 2 ? 1 : 0)) * 8 + e) * 64 + lane] = wave < 2 ? acc[m][8 + e] : acc[m][e];
     __syncthreads();
-    if (wave < 2) {
 #pragma unroll
-      for (int m = 0; m < TM; ++m)
+    for (int m = 0; m < TM; ++m)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const float gate = bf16_bits_to_f32(f32_to_bf16_bits(acc[m][e]));
-          const float up = bf16_bits_to_f32(f32_to_bf16_bits(half[(m * 16 + e) * 64 + lane]));
-          const int r = m * 32 + 8 * (e >> 2) + 4 * h + (e & 3);
-          reinterpret_cast<uint16_t*>(x2)[r * 64 + wave * 32 + n] =
-              col < N ? f32_to_bf16_bits(gate / (1.0f + expf(-gate)) * up) : (uint16_t)0;
-        }
-    }
+      for (int e = 0; e < 8; ++e) {
+        const float mine = bf16_bits_to_f32(f32_to_bf16_bits(wave < 2 ? acc[m][e] : acc[m][8 + e]));
+        const float other =
+            bf16_bits_to_f32(f32_to_bf16_bits(shared[((m * 2 + (wave < 2 ? 0 : 1)) * 8 + e) * 64 + lane]));
+        const float gate = wave < 2 ? mine : other, up = wave < 2 ? other : mine;
+        const int at = keep + e, r = m * 32 + 8 * (at >> 2) + 4 * h + (at & 3);
+        reinterpret_cast<uint16_t*>(x2)[r * 64 + (wave & 1) * 32 + n] =
+            col < N ? f32_to_bf16_bits(gate / (1.0f + expf(-gate)) * up) : (uint16_t)0;
+      }
     __syncthreads();
     const int act_chunks = (N + 255) >> 8;
 #pragma unroll
@@ -817,16 +819,27 @@ __global__ __launch_bounds__(2 * kThreads) void prompt_attention_kernel(const ui
     if (block <= qb) {
       const char* const kb = kl[half][at & 1];
       const char* const vt = vl[half][at & 1];
+      // four independent chains over the dimensions, and the first half of V on its way
       f32x4_t s[4];
 #pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        s[b] = f32x4_t{};
+      for (int b = 0; b < 4; ++b) s[b] = f32x4_t{};
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const uint4 kf = *reinterpret_cast<const uint4*>(kb + (16 * b + n) * 256 + (((4 * t + g) ^ n) << 4));
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const u32x4_t kf = *reinterpret_cast<const u32x4_t*>(kb + (16 * b + n) * 256 + (((4 * t + g) ^ n) << 4));
           s[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf), qf[t], s[b], 0, 0, 0);
         }
-      }
+      bf16x8_t vf[8];
+      auto read_v = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+        for (int d = 0; d < 8; ++d) {
+          const char* const from = vt + (16 * d + n) * kVRow + 64 * j + 8 * g;
+          const u32x2_t lo = *reinterpret_cast<const u32x2_t*>(from), hi = *reinterpret_cast<const u32x2_t*>(from + 32);
+          vf[d] = __builtin_bit_cast(bf16x8_t, u32x4_t{lo.x, lo.y, hi.x, hi.y});
+        }
+      };
+      read_v(0);
       float most = -INFINITY;
 #pragma unroll
       for (int b = 0; b < 4; ++b)
@@ -862,21 +875,20 @@ __global__ __launch_bounds__(2 * kThreads) void prompt_attention_kernel(const ui
           p2[b][e >> 1] = __builtin_amdgcn_perm(w[1][2], w[0][2], 0x07060302u);
         }
 #pragma unroll
-      for (int d = 0; d < 8; ++d) {
+      for (int d = 0; d < 8; ++d)
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[d][e] *= keep;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const char* const at = vt + (16 * d + n) * kVRow + 64 * j + 8 * g;
-          const u32x2_t lo = *reinterpret_cast<const u32x2_t*>(at), hi = *reinterpret_cast<const u32x2_t*>(at + 32);
-          const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, u32x4_t{lo.x, lo.y, hi.x, hi.y});
-          const u32x4_t t0 = {p0[2 * j][0], p0[2 * j][1], p0[2 * j + 1][0], p0[2 * j + 1][1]};
-          const u32x4_t t1 = {p1[2 * j][0], p1[2 * j][1], p1[2 * j + 1][0], p1[2 * j + 1][1]};
-          const u32x4_t t2 = {p2[2 * j][0], p2[2 * j][1], p2[2 * j + 1][0], p2[2 * j + 1][1]};
-          o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(bf16x8_t, t0), o[d], 0, 0, 0);
-          o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(bf16x8_t, t1), o[d], 0, 0, 0);
-          o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(bf16x8_t, t2), o[d], 0, 0, 0);
-        }
+      for (int j = 0; j < 2; ++j) {
+        if (j) read_v(1);
+        const u32x4_t term[3] = {{p0[2 * j][0], p0[2 * j][1], p0[2 * j + 1][0], p0[2 * j + 1][1]},
+                                 {p1[2 * j][0], p1[2 * j][1], p1[2 * j + 1][0], p1[2 * j + 1][1]},
+                                 {p2[2 * j][0], p2[2 * j][1], p2[2 * j + 1][0], p2[2 * j + 1][1]}};
+#pragma unroll
+        for (int t = 0; t < 3; ++t)  // eight independent chains over the terms
+#pragma unroll
+          for (int d = 0; d < 8; ++d)
+            o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[d], __builtin_bit_cast(bf16x8_t, term[t]), o[d], 0, 0, 0);
       }
     }
     stage((at + 1) & 1);
@@ -968,7 +980,8 @@ Plan plan_product(const int32_t* N, int count, int M, int K, int cus, int max_sp
 
 // Tiles for rows sorted by expert: at most pairs / (32 tm) full ones and a part-full one per
 // expert.  The tile height follows the pairs an expert gets on average: short tiles while most
-// of a taller one would be rows of zeros.
+// of a taller one would be rows of zeros (1024 pairs of 32 experts: 38.7 us with tiles of 32 rows,
+// half of them a second tile for a few rows, 37.2 with 64).
 struct ExpertPlan {
   int tm, tiles, blocks;
 };
@@ -976,7 +989,7 @@ struct ExpertPlan {
 ExpertPlan plan_experts(int experts, int pairs) {
   const int used = experts < pairs ? experts : pairs;
   ExpertPlan p;
-  p.tm = pairs <= 40 * used ? 1 : pairs <= 160 * used ? 2 : 4;
+  p.tm = pairs <= 24 * used ? 1 : pairs <= 160 * used ? 2 : 4;
   p.tiles = pairs / (32 * p.tm) + used;
   p.blocks = p.tiles * p.tm;
   return p;
