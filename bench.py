@@ -394,8 +394,8 @@ def bench_prefill(torch, weights, device, gen, count: int = CONTEXT, repeats: in
     sec = sorted(times)[len(times) // 2]
     return {"tokens": count, "ms": round(sec * 1e3, 3), "ns": int(sec * 1e9),
             "tokens_per_s": round(count / sec, 1),
-            "path": "imq_dequant to fp16 + GEMM per projection, fp32 causal attention, "
-                    "head at the last position only"}
+            "path": "imq_prompt_layer per layer (products on the packed weights, causal attention "
+                    "kernel), head at the last position only"}
 
 
 def _epilogue_launches(weights, batch: int) -> int:

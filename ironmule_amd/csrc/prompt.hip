@@ -77,15 +77,15 @@ __device__ __forceinline__ void emit_group(uint4 d, int c, int g, int row, char*
   }
 }
 
-// One workgroup per (chunk, eight rows).  `src` (may be null): the x row of each packed row, -1
+// One workgroup per (eight rows, chunk).  `src` (may be null): the x row of each packed row, -1
 // for a row of zeros, and `expert` the expert of each tile of `tm` blocks, -1 for tiles not in
 // use; without them packed row r is x row r, zeros past M.
 __global__ __launch_bounds__(kThreads) void pack_rows_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                              const int32_t* __restrict__ src,
                                                              const int32_t* __restrict__ expert, int tm, int M, int K,
                                                              char* __restrict__ packed) {
-  const int chunk = blockIdx.x, chunks = gridDim.x, block = blockIdx.y >> 2;
-  const int l = threadIdx.x & 31, in = 8 * (blockIdx.y & 3) + (threadIdx.x >> 5);  // row of the block
+  const int chunk = blockIdx.y, chunks = gridDim.y, block = blockIdx.x >> 2;
+  const int l = threadIdx.x & 31, in = 8 * (blockIdx.x & 3) + (threadIdx.x >> 5);  // row of the block
   if (expert && expert[block / tm] < 0) return;
   const int col = 256 * chunk + 8 * l, r = 32 * block + in;
   const int64_t row = src ? src[r] : (r < M ? r : -1);
@@ -999,7 +999,7 @@ size_t packed_bytes(int64_t blocks, int K) { return (size_t)blocks * ceil_div(K,
 
 void pack_rows(const uint16_t* x, int64_t ldx, const int32_t* src, const int32_t* expert, int tm, int M,
                int64_t blocks, int K, void* packed, hipStream_t stream) {
-  hipLaunchKernelGGL(pack_rows_kernel, dim3(ceil_div(K, 256), (uint32_t)blocks * 4), dim3(kThreads), 0, stream, x, ldx,
+  hipLaunchKernelGGL(pack_rows_kernel, dim3((uint32_t)blocks * 4, ceil_div(K, 256)), dim3(kThreads), 0, stream, x, ldx,
                      src, expert, tm, M, K, static_cast<char*>(packed));
 }
 

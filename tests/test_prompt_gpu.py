@@ -88,6 +88,18 @@ def test_infinities_nan_and_large_values_stay_in_their_rows(env):
     assert ((y[99] - ref[99]).abs() <= 320 * 2.0**-24 * (x[99].double().abs() @ n_.dequant(w, s, b).double().abs().T)).all()
 
 
+def test_more_rows_than_a_launch_dimension(env):
+    """600,000 rows (150,000 workgroups of eight rows): first, middle and last rows against a
+    product of those rows alone."""
+    torch, n_, orc = env
+    announce("prompt many rows")
+    w, s, b, _ = to_device(orc.synthetic(48, 64, 1, seed=orc.SEED_BASE + 945))
+    x = torch.randn((600_000, 64), device="cuda").to(torch.bfloat16)
+    y = n_.prompt_matmul(w, s, b, x)
+    for at in (0, 299_990, 599_960):
+        assert torch.equal(y[at:at + 40], n_.prompt_matmul(w, s, b, x[at:at + 40]))
+
+
 def test_grouped_products_share_one_packing(env):
     """Three weights of one K, N off multiples of four and of 128, over one packing."""
     import ctypes
