@@ -84,7 +84,8 @@ IMQ_API int32_t imq_prompt_experts(const uint32_t* w, const uint16_t* scales, co
  * ironmule/dense_plan.py:337-363). */
 typedef struct {
   int32_t tokens, hidden, heads, kv_heads, intermediate, capacity, num_slots, slot;
-  float eps, theta;
+  float eps;
+  double theta; /* the rotary base: angles are computed in double */
 } imq_prompt_shape;
 
 IMQ_API size_t imq_prompt_layer_workspace(const imq_prompt_shape* shape);

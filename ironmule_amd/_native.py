@@ -107,7 +107,7 @@ class PromptShape(ctypes.Structure):
 
     _fields_ = [("tokens", _I32), ("hidden", _I32), ("heads", _I32), ("kv_heads", _I32), ("intermediate", _I32),
                 ("capacity", _I32), ("num_slots", _I32), ("slot", _I32), ("eps", ctypes.c_float),
-                ("theta", ctypes.c_float)]
+                ("theta", ctypes.c_double)]
 
 
 class QmvStage(ctypes.Structure):

@@ -1126,7 +1126,7 @@ int32_t check_shape(const imq_prompt_shape* s) {
   if (s->hidden > 8192 || s->intermediate > IMQ_PROMPT_MAX_K) return fail(IMQ_EUNSUPPORTED, "hidden or intermediate too large");
   if (s->capacity < s->tokens) return fail(IMQ_EINVAL, "the prompt does not fit the capacity");
   if (s->slot < 0 || s->slot >= s->num_slots) return fail(IMQ_EINVAL, "slot out of range");
-  if (!(s->eps >= 0.0f) || !(s->theta > 1.0f)) return fail(IMQ_EINVAL, "eps must be >= 0 and theta > 1");
+  if (!(s->eps >= 0.0f) || !(s->theta > 1.0)) return fail(IMQ_EINVAL, "eps must be >= 0 and theta > 1");
   return IMQ_OK;
 }
 
@@ -1214,7 +1214,7 @@ int32_t imq_prompt_layer(const imq_step_layer* layer, const imq_prompt_shape* sh
   if ((code = run_product(a, three, at + l.x, blocks, T, s.hidden, st)) != IMQ_OK) return code;
   hipLaunchKernelGGL(prompt_rope_kernel, dim3(T), dim3(kRopeThreads), 0, st, q, k, v, layer->q_norm, layer->k_norm,
                      layer->k_pool + pool, layer->v_pool + pool, s.heads, s.kv_heads, s.capacity,
-                     log2((double)s.theta), s.eps);
+                     log2(s.theta), s.eps);
   hipLaunchKernelGGL(prompt_attention_kernel, dim3(ceil_div(T, kQ) * s.heads), dim3(2 * kThreads), 0, st, q,
                      layer->k_pool + pool, layer->v_pool + pool, at + l.attn, T, s.heads, s.kv_heads, s.capacity);
   if ((code = product_planes(layer->o, at + l.attn, T, s.hidden, qd, planes, dev->cu_count, &splits, st)) != IMQ_OK)

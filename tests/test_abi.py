@@ -220,3 +220,30 @@ def test_malformed_prompt_calls_are_refused_with_codes(lib, over, code):
     assert _prompt(lib, **over) == code
     got, msg = _native.last_error()
     assert got == code and msg
+
+
+@pytest.mark.parametrize("over", [{"tokens": 0}, {"tokens": 65}, {"kv_heads": 3}, {"hidden": 100}, {"hidden": 8256},
+                                  {"intermediate": 96}, {"slot": 2}, {"slot": -1}, {"theta": 1.0}])
+def test_malformed_prompt_shapes_are_refused(lib, over):
+    fields = dict(tokens=64, hidden=256, heads=4, kv_heads=2, intermediate=512, capacity=64, num_slots=2, slot=0,
+                  eps=1e-6, theta=1e6)
+    fields.update(over)
+    shape = _native.PromptShape(**fields)
+    layer = _native.StepLayer()
+    P = ctypes.c_void_p
+    assert lib.imq_prompt_layer_workspace(ctypes.byref(shape)) == 0
+    for code in (lib.imq_prompt_layer(ctypes.byref(layer), ctypes.byref(shape), P(1 << 20), 1, P(1 << 20), 1 << 30, None),
+                 lib.imq_prompt_finish(ctypes.byref(shape), P(1 << 20), 1, P(1 << 20), 1 << 30, None)):
+        assert code in (_native.IMQ_EINVAL, _native.IMQ_EUNSUPPORTED)
+
+
+@pytest.mark.parametrize("over,code", [({"experts": 0}, _native.IMQ_EINVAL), ({"experts": 1025}, _native.IMQ_EUNSUPPORTED),
+                                       ({"pairs": 0}, _native.IMQ_EINVAL), ({"idx": 0}, _native.IMQ_EINVAL),
+                                       ({"per": 0}, _native.IMQ_EINVAL), ({"nbytes": 64}, _native.IMQ_EINVAL),
+                                       ({"ldx": 60}, _native.IMQ_EINVAL)])
+def test_malformed_expert_calls_are_refused(lib, over, code):
+    a = dict(experts=8, per=1, pairs=100, idx=1 << 20, nbytes=1 << 30, ldx=128)
+    a.update(over)
+    P = ctypes.c_void_p(1 << 20)
+    assert lib.imq_prompt_experts(P, P, P, a["experts"], P, a["ldx"], a["per"], ctypes.c_void_p(a["idx"]), a["pairs"], P,
+                                  64, 64, 128, 64, 4, 0, P, a["nbytes"], None) == code
