@@ -520,6 +520,14 @@ def takes_prompt(x: torch.Tensor, k: int) -> bool:
             and torch._C._len_torch_dispatch_stack() == 0)
 
 
+def _same_device(w: torch.Tensor, **others: torch.Tensor) -> None:
+    """The kernels read every operand through its address: one on the host or on another GPU would
+    be a stray access there, or one that its own device's streams do not order."""
+    for name, t in others.items():
+        if t.device != w.device:
+            raise ValueError(f"{name} is on {t.device}, expected {w.device}")
+
+
 def _aligned_rows(x: torch.Tensor, k: int) -> tuple[torch.Tensor, int]:
     """x as (rows, k) bf16 rows the kernels can load 16 bytes at a time, and their stride."""
     x2 = x.reshape(-1, k)
@@ -537,6 +545,7 @@ def prompt_matmul(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor, x
     n, k = check_weights(w, scales, biases)
     if x.dtype != torch.bfloat16 or x.dim() < 1 or int(x.shape[-1]) != k:
         raise ValueError(f"x must be bf16 rows of {k} values")
+    _same_device(w, scales=scales, biases=biases, x=x)
     x2, ld = _aligned_rows(x, k)
     m = int(x2.shape[0])
     out = torch.empty((m, n), dtype=out_dtype, device=w.device)
@@ -559,6 +568,7 @@ def prompt_experts(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor, 
     k = check_weights(*(t.view(e * n, -1) for t in (w, scales, biases)))[1]
     if x.dtype != torch.bfloat16 or int(x.shape[-1]) != k:
         raise ValueError(f"x must be bf16 rows of {k} values")
+    _same_device(w, scales=scales, biases=biases, x=x, idx=idx)
     x2, ld = _aligned_rows(x, k)
     idx = idx.reshape(-1).to(torch.int32).contiguous()
     pairs = int(idx.numel())
@@ -583,6 +593,8 @@ class PromptLayers:
         _require(h, torch.float32, "h")
         if h.dim() != 2 or int(h.shape[1]) != c.hidden or c.head_dim != 128:
             raise ValueError(f"h must be (tokens, {c.hidden}), the head size 128")
+        if not h.is_cuda:
+            raise ValueError("h must be on a GPU")
         self.config, self.h, self.first = c, h, 1
         self.shape = PromptShape(int(h.shape[0]), c.hidden, c.heads, c.kv_heads, c.intermediate, int(capacity),
                                  int(slots), int(slot), float(c.eps), float(c.theta))
@@ -597,7 +609,9 @@ class PromptLayers:
         for name, size in self.config.projections.items():
             if check_weights(*layer[name]) != tuple(size):
                 raise ValueError(f"{name} must be {tuple(size)}")
-            quants.append(QWeight(*[t.data_ptr() for t in layer[name]]))
+            w, scales, biases = layer[name]
+            _same_device(self.h, **{name: w, f"{name} scales": scales, f"{name} biases": biases})
+            quants.append(QWeight(w.data_ptr(), scales.data_ptr(), biases.data_ptr()))
         norms = [layer[name] for name in ("input_norm", "post_norm", "q_norm", "k_norm")]
         for t, want in zip(norms, (self.config.hidden, self.config.hidden, 128, 128)):
             _require(t, torch.bfloat16, "a norm weight")
@@ -607,6 +621,8 @@ class PromptLayers:
             _require(t, torch.bfloat16, "a pool")
             if tuple(t.shape) != self.pool_shape:
                 raise ValueError(f"a pool must be {self.pool_shape}")
+        for t in (*norms, k_pool, v_pool):
+            _same_device(self.h, **{"a norm weight or pool": t})
         desc = StepLayer(*quants, *[t.data_ptr() for t in norms], k_pool.data_ptr(), v_pool.data_ptr())
         _check(lib().imq_prompt_layer(ctypes.byref(desc), ctypes.byref(self.shape), _ptr(self.h), self.first,
                                       _ptr(self.workspace), self.nbytes, _stream(None)))

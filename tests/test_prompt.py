@@ -1,0 +1,76 @@
+"""Host-side rules of the calls for more than 32 rows: what they refuse before a kernel is
+launched.  No GPU: meta tensors stand for the device's, and a launch fails the test."""
+
+from __future__ import annotations
+
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from ironmule_amd import _native
+
+N, K = 64, 128
+
+
+@pytest.fixture
+def no_launch(monkeypatch):
+    def refuse(*args):
+        raise AssertionError("a kernel would be launched")
+
+    monkeypatch.setattr(_native, "lib", lambda: SimpleNamespace(
+        imq_prompt_matmul_workspace=lambda *a: 256, imq_prompt_experts_workspace=lambda *a: 256,
+        imq_prompt_layer_workspace=lambda *a: 256, imq_prompt_matmul=refuse, imq_prompt_experts=refuse,
+        imq_prompt_layer=refuse))
+    # the check that weights are on a GPU; meta tensors stand for those
+    monkeypatch.setattr(_native, "check_weights", lambda w, s, b: (int(w.shape[0]), int(w.shape[1]) * 8))
+    monkeypatch.setattr(_native, "_stream", lambda stream: 0)
+
+
+def _quant(device, lead=()):
+    return (torch.empty((*lead, N, K // 8), dtype=torch.int32, device=device),
+            torch.empty((*lead, N, K // 64), dtype=torch.bfloat16, device=device),
+            torch.empty((*lead, N, K // 64), dtype=torch.bfloat16, device=device))
+
+
+def _move(tensors, which):
+    return [torch.zeros_like(t, device="cpu") if i == which else t for i, t in enumerate(tensors)]
+
+
+@pytest.mark.parametrize("which", [1, 2, 3])
+def test_products_refuse_operands_of_another_device(no_launch, which):
+    w, s, b, x = _move([*_quant("meta"), torch.empty((40, K), dtype=torch.bfloat16, device="meta")], which)
+    with pytest.raises(ValueError, match="is on cpu"):
+        _native.prompt_matmul(w, s, b, x)
+
+
+@pytest.mark.parametrize("which", [1, 2, 3, 4])
+def test_expert_batches_refuse_operands_of_another_device(no_launch, which):
+    w, s, b, x, idx = _move([*_quant("meta", (4,)), torch.empty((40, K), dtype=torch.bfloat16, device="meta"),
+                             torch.empty(40, dtype=torch.int32, device="meta")], which)
+    with pytest.raises(ValueError, match="is on cpu"):
+        _native.prompt_experts(w, s, b, x, idx)
+
+
+@pytest.mark.parametrize("where", ["up", "post_norm", "k_pool", "v_pool", "h"])
+def test_prompt_layers_refuse_operands_of_another_device(no_launch, where):
+    projections = {name: (N, K) for name in ("q", "k", "v", "o", "gate", "up", "down")}
+    config = SimpleNamespace(hidden=K, heads=1, kv_heads=1, head_dim=128, intermediate=N, eps=1e-6, theta=1e6,
+                             projections=projections)
+    h = torch.empty((40, K), device="cpu" if where == "h" else "meta")
+    if where == "h":
+        with pytest.raises(ValueError, match="GPU"):
+            _native.PromptLayers(config, h, 1, 64, 0)
+        return
+    run = object.__new__(_native.PromptLayers)
+    run.config, run.h, run.first, run.pool_shape, run.nbytes = config, h, 1, (1, 1, 64, 128), 256
+    run.shape, run.workspace = _native.PromptShape(), torch.empty(256, dtype=torch.uint8, device="meta")
+
+    def made(name, *shape):
+        return torch.empty(shape, dtype=torch.bfloat16, device="cpu" if name == where else "meta")
+
+    layer = {name: _quant("cpu" if name == where else "meta") for name in projections}
+    layer.update(input_norm=made("input_norm", K), post_norm=made("post_norm", K), q_norm=made("q_norm", 128),
+                 k_norm=made("k_norm", 128))
+    with pytest.raises(ValueError, match="is on cpu"):
+        run.layer(layer, made("k_pool", 1, 1, 64, 128), made("v_pool", 1, 1, 64, 128))
