@@ -304,6 +304,8 @@ def qmv(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor, x: torch.Te
         raise ValueError(f"x must be (M, {k}), got {tuple(x.shape)}")
     if x2.dtype is not torch.bfloat16:
         raise ValueError(f"x must be bfloat16, got {x2.dtype}")
+    if x2.device != w.device:
+        raise ValueError(f"x is on {x2.device}, the weights on {w.device}")
     m = x2.shape[0]
     if not 1 <= m <= MAX_ROWS:
         raise ValueError(f"the qmv kernels take 1 to {MAX_ROWS} rows, got {m}")
@@ -468,6 +470,8 @@ def gather_qmv(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor, x: t
         raise ValueError("w must be contiguous")
     if x.dtype != torch.bfloat16 or x.dim() != 2 or x.shape[1] != k or not x.is_contiguous():
         raise ValueError(f"x must be a contiguous bf16 (rows, {k}) tensor")
+    if x.device != w.device:
+        raise ValueError(f"x is on {x.device}, the weights on {w.device}")
     if idx.dtype != torch.int32 or idx.device != w.device:
         raise ValueError("idx must be an int32 tensor on the weights' device")
     if idx.dim() != 1 or not idx.is_contiguous():

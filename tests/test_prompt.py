@@ -1,5 +1,6 @@
-"""Host-side rules of the calls for more than 32 rows: what they refuse before a kernel is
-launched.  No GPU: meta tensors stand for the device's, and a launch fails the test."""
+"""Host-side rules of the calls through `_native`, above all those for more than 32 rows: what
+they refuse before a kernel is launched.  No GPU: meta tensors stand for the device's, and a
+launch fails the test."""
 
 from __future__ import annotations
 
@@ -21,7 +22,9 @@ def no_launch(monkeypatch):
     monkeypatch.setattr(_native, "lib", lambda: SimpleNamespace(
         imq_prompt_matmul_workspace=lambda *a: 256, imq_prompt_experts_workspace=lambda *a: 256,
         imq_prompt_layer_workspace=lambda *a: 256, imq_prompt_matmul=refuse, imq_prompt_experts=refuse,
-        imq_prompt_layer=refuse))
+        imq_prompt_layer=refuse, imq_qmv=refuse, imq_qmv_ws=refuse, imq_qmv_workspace=lambda *a: 0,
+        imq_gather_qmv=refuse))
+    monkeypatch.setattr(_native, "_lib", None)
     # the check that weights are on a GPU; meta tensors stand for those
     monkeypatch.setattr(_native, "check_weights", lambda w, s, b: (int(w.shape[0]), int(w.shape[1]) * 8))
     monkeypatch.setattr(_native, "_stream", lambda stream: 0)
@@ -74,3 +77,15 @@ def test_prompt_layers_refuse_operands_of_another_device(no_launch, where):
                  k_norm=made("k_norm", 128))
     with pytest.raises(ValueError, match="is on cpu"):
         run.layer(layer, made("k_pool", 1, 1, 64, 128), made("v_pool", 1, 1, 64, 128))
+
+
+@pytest.mark.parametrize("rows", [1, 3])
+def test_up_to_32_rows_refuse_x_of_another_device(no_launch, rows):
+    with pytest.raises(ValueError, match="x is on cpu"):
+        _native.qmv(*_quant("meta"), torch.zeros((rows, K), dtype=torch.bfloat16))
+
+
+def test_gathered_rows_refuse_x_of_another_device(no_launch):
+    with pytest.raises(ValueError, match="x is on cpu"):
+        _native.gather_qmv(*_quant("meta", (4,)), torch.zeros((3, K), dtype=torch.bfloat16),
+                           torch.empty(3, dtype=torch.int32, device="meta"))
