@@ -164,13 +164,21 @@ class QuantizedSwitchLinear(torch.nn.Module):
         return y + self.bias[indices].unsqueeze(-2) if self.bias is not None else y
 
 
+def _stack_as_stored(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor) -> bool:
+    """Whether the kernels can read an expert stack where it lies: whole, in order, 16-byte
+    aligned.  A slice of a fused stack, every other expert or a view off that alignment is copied
+    expert by expert instead."""
+    return (w.dim() == scales.dim() == biases.dim() == 3 and w.is_contiguous() and scales.is_contiguous()
+            and biases.is_contiguous() and w.data_ptr() % 16 == 0)
+
+
 def library_gather_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor,
                           biases: torch.Tensor, indices: torch.Tensor,
                           group_size: int = GROUP_SIZE, bits: int = BITS) -> torch.Tensor:
     """The library gather path, (*batch, M, K) x experts -> (*batch, M, N), batch =
     broadcast(x.shape[:-2], indices.shape): bf16 rows sorted by expert and multiplied on the
-    packed weights (_native.prompt_experts); otherwise, and where autograd or a transform
-    follows the call, every selected expert dequantised to fp32 and one batched product."""
+    packed weights (_native.prompt_experts); otherwise, for stacks of other strides, and where
+    autograd or a transform follows the call, every selected expert dequantised to fp32 and one batched product."""
     if group_size != GROUP_SIZE or bits != BITS:
         raise ValueError("only 4-bit, group-64 weights are supported")
     if not x.is_cuda:
@@ -180,7 +188,7 @@ def library_gather_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor
     pairs = batch.numel() * rows
     if (_native.takes_prompt(x, k) and 1 <= pairs <= _native.MAX_PROMPT_ROWS and not indices.is_floating_point()
             and indices.dtype != torch.bool and indices.is_cuda and x.shape[-1] == k
-            and 1 <= w.shape[0] <= _native.MAX_PROMPT_EXPERTS):
+            and 1 <= w.shape[0] <= _native.MAX_PROMPT_EXPERTS and _stack_as_stored(w, scales, biases)):
         lead, idx, per = tuple(x.shape[:-2]), indices.expand(batch), 1
         if rows == 1 and batch and lead == tuple(batch[:-1]) + (1,):
             per = int(batch[-1])  # a token's row shared by its experts

@@ -89,3 +89,20 @@ def test_gathered_rows_refuse_x_of_another_device(no_launch):
     with pytest.raises(ValueError, match="x is on cpu"):
         _native.gather_qmv(*_quant("meta", (4,)), torch.zeros((3, K), dtype=torch.bfloat16),
                            torch.empty(3, dtype=torch.int32, device="meta"))
+
+
+def test_only_whole_aligned_expert_stacks_are_read_in_place():
+    from ironmule_amd.quantized import _stack_as_stored
+
+    def stack(e, n):
+        return (torch.zeros((e, n, K // 8), dtype=torch.int32), torch.zeros((e, n, K // 64), dtype=torch.bfloat16),
+                torch.zeros((e, n, K // 64), dtype=torch.bfloat16))
+
+    assert _stack_as_stored(*stack(4, N))
+    assert _stack_as_stored(*(t[1:3] for t in stack(4, N)))
+    assert not _stack_as_stored(*(t[:, :N // 2] for t in stack(4, N)))
+    assert not _stack_as_stored(*(t[::2] for t in stack(4, N)))
+    w, s, b = stack(4, N)
+    assert not _stack_as_stored(w, s.transpose(0, 1).contiguous().transpose(0, 1), b)
+    off = torch.zeros(w.numel() + 1, dtype=torch.int32)[1:].view_as(w)
+    assert not _stack_as_stored(off, s, b)

@@ -188,6 +188,33 @@ def test_expert_batch_forms(env):
     assert not out[1].any() and not out[2].any() and out[0].any() and out[3:].any(dim=1).all()
 
 
+def test_expert_stacks_of_any_stride_and_alignment(env):
+    """One half of a fused gate/up stack, every other expert, scales of another order and words off a
+    16-byte boundary: the same products as a stack copied whole, through both entry points."""
+    torch, n_, orc = env
+    from ironmule_amd import hip_native
+    from ironmule_amd.quantized import library_gather_matmul
+    announce("expert stack strides")
+    e, n, k, tokens, top = 8, 128, 256, 20, 4
+    stack = [to_device(orc.synthetic(n, k, 1, seed=orc.SEED_BASE + 1000 + i)) for i in range(e)]
+    whole = tuple(torch.stack([p[f] for p in stack]) for f in range(3))
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(7)
+    x = torch.randn((tokens, 1, 1, k), device="cuda", generator=gen).to(torch.bfloat16)
+    off = torch.empty(whole[0].numel() + 1, dtype=torch.int32, device="cuda")[1:].view_as(whole[0]).copy_(whole[0])
+    turned = whole[1].transpose(0, 1).contiguous().transpose(0, 1)
+    for w, s, b in (tuple(t[:, n // 2:] for t in whole), tuple(t[::2] for t in whole), (off, *whole[1:]),
+                    (whole[0], turned, whole[2])):
+        idx = torch.randint(0, w.shape[0], (tokens, top), device="cuda", generator=gen)
+        copied = [t.clone(memory_format=torch.contiguous_format) for t in (w, s, b)]
+        want = library_gather_matmul(x, *copied, idx).float()
+        for call in (library_gather_matmul, hip_native.gather_matmul):
+            got = call(x, w, s, b, idx).float()
+            # two fp32 sums, each within 2^-20 sum|w x| (at most 16 times the outputs' root mean square
+            # at K = 256) and rounded to bf16: one ulp, at most 2^-7 of the value, and that much
+            assert ((got - want).abs() <= 2.0**-7 * want.abs() + 2.0**-15 * want.abs().max()).all()
+
+
 @pytest.mark.parametrize("tokens,heads,kv_heads,hidden,intermediate", [
     (1, 4, 2, 256, 512), (16, 4, 2, 256, 512), (33, 6, 3, 320, 448), (63, 8, 1, 192, 256), (64, 4, 4, 256, 512),
     (65, 4, 2, 256, 512), (130, 8, 2, 576, 1088), (257, 16, 2, 1024, 768)])
