@@ -99,10 +99,10 @@ IMQ_API int32_t imq_attention_decode(const uint16_t* q, const uint16_t* k_pool,
  * of q (B, Hq, 128) and k (B, Hkv, 128); this step's k and v written into the pools at
  * row positions[b] of slot slots[b]; then out[b][h] = softmax(q . K / sqrt(128)) V over
  * rows 0 .. positions[b] of the slot (clamped to max_len and capacity), split over 64-key
- * chunks with the split plan of imq_attention_decode and merged in split order by the
- * last split of each (request, KV head); from 64 (request, KV head) pairs, and for fewer over
- * more than 1024 keys, a workgroup of 12 wavefronts per task, split so that at most about 256
- * tasks run (never more splits than that plan; none from 129 pairs).  The KV pools get the same bits as
+ * chunks (imq_attention_fused_plan: by B, Hkv and max_len the workgroups and splits, by each
+ * request's own length the chunks of its splits; never more splits than imq_attention_decode's
+ * plan, none from 129 pairs) and merged in split order by the last split of each (request, KV
+ * head).  The KV pools get the same bits as
  * imq_qk_norm_rope followed by imq_attention_decode with lengths = positions + 1 for every
  * valid request, and the output agrees with theirs to the attention's oracle bar (the
  * scores and P.V run on MFMA, in another summation order); a request with
@@ -121,6 +121,12 @@ IMQ_API int32_t imq_attention_fused(const uint16_t* q, const uint16_t* k, const 
                                     int32_t Hq, int32_t Hkv, int32_t capacity, int32_t num_slots,
                                     int32_t max_len, float theta, float eps, float* workspace,
                                     uint32_t* counters, void* stream);
+
+/* The plan of imq_attention_fused under min(max_len, capacity) = max_len: wavefronts per workgroup,
+ * splits launched per (request, KV head) pair, and the 64-key chunks of a split of a request that
+ * attends over `keys` keys (its splits in use are the quotient, rounded up). */
+IMQ_API int32_t imq_attention_fused_plan(int32_t B, int32_t Hkv, int32_t max_len, int32_t keys, int32_t* wavefronts,
+                                         int32_t* splits, int32_t* chunks);
 
 /* imq_attention_fused with q, k and v given as the fp32 output planes of a split projection
  * (imq_qmv_norm_planes over the q, k and v weights, ironmule_qmv.h) instead of bf16 rows:

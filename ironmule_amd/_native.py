@@ -158,6 +158,7 @@ _SIGNATURES = {
                               ctypes.c_float, _P, _P], _I32),
     "imq_attention_fused": ([_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I32, _I32, _I32, _I32,
                              _I32, _I32, ctypes.c_float, ctypes.c_float, _P, _P, _P], _I32),
+    "imq_attention_fused_plan": ([_I32, _I32, _I32, _I32] + [ctypes.POINTER(_I32)] * 3, _I32),
     "imq_attention_fused_planes": ([_P, _I64, _I32, _P, _P, _P, _P, _P, _P, _P, _I64, _I32, _I32, _I32,
                                     _I32, _I32, _I32, ctypes.c_float, ctypes.c_float, _P, _P, _P],
                                    _I32),

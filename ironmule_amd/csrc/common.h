@@ -153,9 +153,10 @@ __host__ __device__ inline int m1_lane_shift(int K) {
 
 // Decode attention's split of each (request, KV head) pair's keys: whole 64-key chunks per
 // split, as many splits as it takes to give the launch about IMQ_ATTN_WORKGROUPS
-// workgroups (at most one split per chunk).  Shared by every attention path so that they
-// merge the same partials in the same order.  At 32 requests x 8 KV heads over 512 keys
-// the fused attention launch measured 31.5 us at 4096 workgroups (one chunk per split),
+// workgroups (at most one split per chunk): the per-kernel path, the decode programs, and the
+// fused launch for few pairs over short caches (its other plans have fewer splits and merge other
+// partials).  At 32 requests x 8 KV heads over 512 keys the fused attention launch, while it
+// followed this plan, measured 31.5 us at 4096 workgroups (one chunk per split),
 // 28.1 at 2048, 22.6 at 1024 (three chunks per split) and 25.3 at 512; one request keeps
 // a split per chunk at any of these.
 #ifndef IMQ_ATTN_WORKGROUPS

@@ -113,6 +113,7 @@ struct Stage {
   float* ml;
   uint32_t* combine;  // one counter per (request, KV head)
   int32_t Hq, Hkv, capacity, num_slots, max_len, splits, cps;
+  uint32_t per_split;  // ceil(2^32 / splits) where the kernel shares the request's chunks out
   int32_t out_tiled;  // 1: the attention output in the 32-row tile layout (else rows Hq * 128 apart)
   // q, k and v as fp32 output planes of a split projection instead (staged launches only):
   // problem i (q, k, v), plane s, request b at qkv + i * qkv_pstride + (s * qkv_rows + b) * N_i
@@ -557,10 +558,23 @@ __device__ __forceinline__ uint16_t ld16_sc1(const uint16_t* base, uint32_t byte
   return (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(buffer_rsrc(base, bytes), off, 0, kSc1);
 }
 
+// Chunks per split of a request that holds `held` chunks: its own chunks shared out over the pair's
+// splits (per_split = ceil(2^32 / splits), the quotient exact for held below 2^23), at least `fewest`
+// each, and over no more splits than a merge loads at once while that leaves a split at most 8.
+// With the share of max_len instead, a short request in a roomy cache left most of its splits
+// without keys: four requests of 512 / 1000 keys under max_len 8192 took 14.7 / 22.2 us, 12.5 /
+// 13.2 so; fourteen of 2000 under 4096 40.8, 28.2 so.
+__host__ __device__ inline int shared_chunks(int held, int splits, uint32_t per_split, int fewest) {
+  const int even = (int)(((uint64_t)(uint32_t)(held + splits - 1) * per_split) >> 32);
+  const int merged = held <= 8 * kMergeBatch ? (held + kMergeBatch - 1) / kMergeBatch : 0;
+  const int most = even > merged ? even : merged;
+  return most > fewest ? most : fewest;
+}
+
 // kPlanes (staged launches only): q, k and v arrive as the fp32 K-range planes of the q/k/v
 // launch (Stage::qkv) rather than as bf16 rows; one instantiation per form, so that each has
 // one sequence of loads and its waits count them exactly.
-template <bool kStaged, typename SRef, int W = kAttnWaves, bool kPlanes = false>
+template <bool kStaged, typename SRef, int W = kAttnWaves, bool kPlanes = false, bool kShare = false>
 __device__ __forceinline__ bool attention_task(SRef S, int task, const StepArgs& a, uint4* smem) {
   AttnLdsT<W>& L = *reinterpret_cast<AttnLdsT<W>*>(smem);
   constexpr int kRounds = (8 + W - 1) / W;  // query heads (at most 8) per wavefront
@@ -654,12 +668,14 @@ __device__ __forceinline__ bool attention_task(SRef S, int task, const StepArgs&
   len = len < S.max_len ? len : S.max_len;
   len = len < S.capacity ? len : S.capacity;
   if (!write_ok || len < 0) len = 0;
-  const int span = S.cps * kChunk;
+  const int cps = kShare ? shared_chunks((len + kChunk - 1) / kChunk, splits, S.per_split, S.cps) : S.cps;
+  const int span = cps * kChunk;
   const int first = s * span;
   const int last = min(len, first + span);
   const int used = (len + span - 1) / span;
   const int newrow = write_ok && pos < len ? pos : -1;
-  const int writer = write_ok ? min(pos / span, splits - 1) : -1;
+  // the split that holds position `pos` (the last one for a position past max_len)
+  const bool writer = write_ok && pos >= first && (pos < first + span || s == splits - 1);
   const size_t base = (((size_t)(slot_ok ? slot : 0) * Hkv + kvh) * S.capacity) * kD;
 
   // This wavefront's keys: units of 16, units wave, wave + W, ... of the split's keys
@@ -763,7 +779,7 @@ __device__ __forceinline__ bool attention_task(SRef S, int task, const StepArgs&
     rotate(kx[0], kx[1], kn0, kn1, kn);
     vn[lane] = (uint16_t)vx[0];
     vn[lane + 64] = (uint16_t)vx[1];
-    if (s == writer) {  // this step's key and value into the pools (read by later launches)
+    if (writer) {  // this step's key and value into the pools (read by later launches)
       uint16_t* kd = S.k_pool + base + (size_t)pos * kD;
       uint16_t* vd = S.v_pool + base + (size_t)pos * kD;
       kd[lane] = kn[lane];
@@ -1126,10 +1142,10 @@ __global__ __launch_bounds__(kThreads) void qmv_stage_kernel(const Stage S, Step
   qmv_task<NCH, XR, XSRC, EPI, true, const Stage&>(S, blockIdx.x, a, smem);
 }
 
-template <int W, bool kPlanes>
+template <int W, bool kPlanes, bool kShare>
 __global__ __launch_bounds__(64 * W) void attention_stage_kernel(const Stage S, StepArgs a) {
   extern __shared__ uint4 smem[];
-  attention_task<true, const Stage&, W, kPlanes>(S, blockIdx.x, a, smem);
+  attention_task<true, const Stage&, W, kPlanes, kShare>(S, blockIdx.x, a, smem);
 }
 
 #undef IMQ_QMV_SHAPES_X2
@@ -1307,51 +1323,82 @@ int32_t finish_program(imq_program* prog) {
   return ok();
 }
 
-// Attention splits: the per-kernel path's plan (attention_splits, common.h): a split's
-// chunks of 64 keys are shared by the workgroup's four wavefronts, 16 keys each.
+// The persistent form's splits: the per-kernel path's plan (attention_splits, common.h): a
+// split's chunks of 64 keys are shared by the workgroup's four wavefronts, 16 keys each.
 void attention_split(int B, int Hkv, int span, int* splits, int* cps) {
   static_assert(kChunk == kAttnWaves * kUnit, "a chunk is one unit per wavefront");
   attention_splits(B, Hkv, span, splits, cps);
 }
 
-#ifndef IMQ_ATTN_WIDE_WAVES
-#define IMQ_ATTN_WIDE_WAVES 12
-#endif
-// From 64 (request, KV head) pairs (8 requests over 8 KV heads): at 8 requests over 512 keys the
-// fused launch took 12.0 us against 13.5 with 4 wavefronts per workgroup, at 4 requests 11.7
-// against 10.6.  And for any pairs whose keys are more chunks than a merge loads at once, where
-// the narrow plan's splits pass a second merge round: one request over 1010 / 1080 / 2048 / 8192
-// keys 9.5 / 12.7 / 15.7 / 32.3 us narrow and 11.8 / 11.6 / 12.3 / 19.3 wide, four over 1010 /
-// 1080 / 8192 13.3 / 16.8 / 41.0 and 12.6 / 12.5 / 28.8.
-#ifndef IMQ_ATTN_WIDE_PAIRS
-#define IMQ_ATTN_WIDE_PAIRS 64
-#endif
-#ifndef IMQ_ATTN_WIDE_WORKGROUPS
-#define IMQ_ATTN_WIDE_WORKGROUPS 256
-#endif
-constexpr int kWideWaves = IMQ_ATTN_WIDE_WAVES;
+// ceil(2^32 / splits) for shared_chunks; one split holds all of `fewest` chunks
+uint32_t per_split_of(int splits) {
+  return splits > 1 ? (uint32_t)((((uint64_t)1 << 32) + splits - 1) / splits) : 0u;
+}
 
-// The wide plan: a workgroup of kWideWaves wavefronts takes a split of at least one unit per
-// wavefront, and the splits fill at most one workgroup per CU: a few more than 256 workgroups
-// are a second round of whole splits (20 requests over 512 keys: 320 workgroups 25.5 us, 160
-// of them 14.3; 14 requests 336: 19.2, 224: 14.1).  Never more splits than attention_split's
-// plan, so its workspace size holds.
-bool attention_wide_split(int B, int Hkv, int span, int* splits, int* cps) {
-  const int pairs = B * Hkv;
-  const int chunks = (span + kChunk - 1) / kChunk;
-  if (pairs < IMQ_ATTN_WIDE_PAIRS && chunks <= kMergeBatch) return false;
-  const int min_c = (kWideWaves * kUnit + kChunk - 1) / kChunk;
-  int sp = IMQ_ATTN_WIDE_WORKGROUPS / pairs;
-  sp = sp < chunks ? sp : chunks;
-  sp = sp > 1 ? sp : 1;
-  int c = (chunks + sp - 1) / sp;
-  c = c > min_c ? c : min_c;
-  c = c < chunks ? c : chunks;
-  *cps = c;
-  *splits = (chunks + c - 1) / c;
-  int base_splits, base_cps;
-  attention_split(B, Hkv, span, &base_splits, &base_cps);
-  return *splits <= base_splits;
+// The plan of a fused launch: wavefronts per workgroup, splits of a pair's keys, the chunks of a
+// split, and whether the kernel shares the request's own chunks out (cps is then the fewest).
+struct AttnPlan {
+  int waves, splits, cps;
+  bool share;
+};
+
+constexpr int kManyWaves = 12, kFewWaves = 8;
+constexpr int kManyPairs = 64;
+constexpr int kWideWorkgroups = 256;  // one per CU
+
+// From 64 (request, KV head) pairs (8 requests over 8 KV heads) workgroups of 12 wavefronts: at 8
+// requests over 512 keys 12.4 us against 13.5 with 4, at 4 requests 11.7 against 10.6.  For fewer
+// pairs the narrow plan (4 wavefronts, a split per chunk up to 1024 workgroups) while the cache
+// spans no more chunks than a merge loads at once, for up to 8 pairs twice as many, two chunks a
+// split past 1024 keys (one request of 512 / 1000 / 2040 keys under max_len 2048: 9.2 / 10.1 / 11.9
+// us, a chunk a split 9.2 / 10.2 / 15.4, 8 wavefronts 10.4 / 10.8 / 11.6).  Longer caches take 8
+// wavefronts while a full one leaves a split at most 4 chunks, which is two units a wavefront, and
+// 12 beyond (four requests, cache full, 4 / 8 / 12 wavefronts: 2048 keys 30.5 / 14.4 / 15.2, 4096
+// 34.5 / 20.2 / 19.2, 8192 43.6 / 32.9 / 29.6).  What this gives up: one request of 60 to 1000 keys in
+// a cache of 3000 to 6000 takes 7.0 to 10.7 us, 6.5 to 10.2 by the narrow plan; at 3000 keys 13.3
+// against 22.
+//
+// A wide split has at least one unit per wavefront, and the splits fill at most one workgroup per
+// CU: a few more than 256 are a second round of whole splits (20 requests over 512 keys: 320
+// workgroups 25.5 us, 160 of them 14.3; 14 requests 336: 19.2, 224: 14.1).  Never more splits than
+// attention_splits' plan, so its workspace size holds.
+AttnPlan attention_plan(int B, int Hkv, int span) {
+  const int pairs = B * Hkv, chunks = (span + kChunk - 1) / kChunk;
+  AttnPlan narrow{kAttnWaves, 0, 0, false};
+  attention_splits(B, Hkv, span, &narrow.splits, &narrow.cps);
+  if (pairs < kManyPairs && chunks <= kMergeBatch) return narrow;
+  if (pairs <= 8 && chunks <= 2 * kMergeBatch) {
+    narrow.share = true;
+    return narrow;
+  }
+  const int sp = std::max(1, std::min(kWideWorkgroups / pairs, chunks));
+  const int share = (chunks + sp - 1) / sp;
+  AttnPlan p;
+  p.waves = pairs < kManyPairs && share <= 4 ? kFewWaves : kManyWaves;
+  const int fewest = (p.waves * kUnit + kChunk - 1) / kChunk;
+  p.cps = std::min(std::max(share, fewest), chunks);
+  p.splits = (chunks + p.cps - 1) / p.cps;
+  if (p.splits > narrow.splits) return narrow;
+  if (p.splits > 1) p.cps = std::min(p.cps, fewest);
+  p.share = true;
+  return p;
+}
+
+template <int W, bool kPlanes, bool kShare>
+int32_t launch_attention(const Stage& A, const StepArgs& a, int device, hipStream_t stream) {
+  const size_t lds = (sizeof(AttnLdsT<W>) + 15) & ~(size_t)15;
+  if (lds > 64 * 1024) {  // above the default dynamic limit: raised once per device
+    static std::atomic<bool> raised[imq_rt::kMaxDevices];
+    if (!raised[device].load(std::memory_order_acquire)) {
+      const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(attention_stage_kernel<W, kPlanes, kShare>),
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      if (attr != hipSuccess)
+        return fail(IMQ_ELAUNCH, std::string("fused attention LDS size: ") + hipGetErrorString(attr));
+      raised[device].store(true, std::memory_order_release);
+    }
+  }
+  hipLaunchKernelGGL((attention_stage_kernel<W, kPlanes, kShare>), dim3(A.count), dim3(64 * W), lds, stream, A, a);
+  return IMQ_OK;
 }
 
 int32_t attention_fused(const uint16_t* q, const uint16_t* k, const uint16_t* v, const float* planes,
@@ -1387,9 +1434,8 @@ int32_t attention_fused(const uint16_t* q, const uint16_t* k, const uint16_t* v,
   if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= imq_rt::kMaxDevices)
     return fail(IMQ_EUNAVAILABLE, "no current HIP device");
   const int span = std::min(max_len, capacity);
-  int splits, cps;
-  const bool wide = attention_wide_split(B, Hkv, span, &splits, &cps);
-  if (!wide) attention_split(B, Hkv, span, &splits, &cps);
+  const AttnPlan plan = attention_plan(B, Hkv, span);
+  const int splits = plan.splits;
   Stage A;
   memset(&A, 0, sizeof(A));
   A.kind = kKindAttention;
@@ -1418,7 +1464,8 @@ int32_t attention_fused(const uint16_t* q, const uint16_t* k, const uint16_t* v,
   A.num_slots = num_slots;
   A.max_len = span;
   A.splits = splits;
-  A.cps = cps;
+  A.cps = plan.cps;
+  A.per_split = per_split_of(splits);
   A.qkv = planes;
   A.qkv_pstride = pstride;
   A.qkv_splits = planes ? nplanes : 0;
@@ -1428,31 +1475,19 @@ int32_t attention_fused(const uint16_t* q, const uint16_t* k, const uint16_t* v,
   a.ntasks = A.count;
   a.staged = 1;
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  if (wide) {
-    const size_t lds = (sizeof(AttnLdsT<kWideWaves>) + 15) & ~(size_t)15;
-    // the launch's LDS is above the default dynamic limit: raised once per device, for both
-    // forms of the kernel
-    static std::atomic<bool> raised[imq_rt::kMaxDevices];
-    if (!raised[device].load(std::memory_order_acquire)) {
-      for (const void* fn : {reinterpret_cast<const void*>(attention_stage_kernel<kWideWaves, true>),
-                             reinterpret_cast<const void*>(attention_stage_kernel<kWideWaves, false>)}) {
-        const hipError_t attr = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (attr != hipSuccess)
-          return fail(IMQ_ELAUNCH, std::string("fused attention LDS size: ") + hipGetErrorString(attr));
-      }
-      raised[device].store(true, std::memory_order_release);
-    }
-    if (planes)
-      hipLaunchKernelGGL((attention_stage_kernel<kWideWaves, true>), dim3(A.count), dim3(64 * kWideWaves), lds, st, A, a);
-    else
-      hipLaunchKernelGGL((attention_stage_kernel<kWideWaves, false>), dim3(A.count), dim3(64 * kWideWaves), lds, st, A, a);
-  } else {
-    const size_t lds = (sizeof(AttnLds) + 15) & ~(size_t)15;
-    if (planes)
-      hipLaunchKernelGGL((attention_stage_kernel<kAttnWaves, true>), dim3(A.count), dim3(kThreads), lds, st, A, a);
-    else
-      hipLaunchKernelGGL((attention_stage_kernel<kAttnWaves, false>), dim3(A.count), dim3(kThreads), lds, st, A, a);
-  }
+  if (plan.waves == kManyWaves)
+    code = planes ? launch_attention<kManyWaves, true, true>(A, a, device, st)
+                  : launch_attention<kManyWaves, false, true>(A, a, device, st);
+  else if (plan.waves == kFewWaves)
+    code = planes ? launch_attention<kFewWaves, true, true>(A, a, device, st)
+                  : launch_attention<kFewWaves, false, true>(A, a, device, st);
+  else if (plan.share)
+    code = planes ? launch_attention<kAttnWaves, true, true>(A, a, device, st)
+                  : launch_attention<kAttnWaves, false, true>(A, a, device, st);
+  else
+    code = planes ? launch_attention<kAttnWaves, true, false>(A, a, device, st)
+                  : launch_attention<kAttnWaves, false, false>(A, a, device, st);
+  if (code != IMQ_OK) return code;
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(IMQ_ELAUNCH, std::string("fused attention launch: ") + hipGetErrorString(e));
   return ok();
@@ -1461,6 +1496,18 @@ int32_t attention_fused(const uint16_t* q, const uint16_t* k, const uint16_t* v,
 }  // namespace
 
 extern "C" {
+
+int32_t imq_attention_fused_plan(int32_t B, int32_t Hkv, int32_t max_len, int32_t keys, int32_t* wavefronts,
+                                 int32_t* splits, int32_t* chunks) {
+  if (!wavefronts || !splits || !chunks) return fail(IMQ_EINVAL, "null pointer");
+  if (B < 1 || Hkv < 1 || (int64_t)B * Hkv > (1 << 24) || max_len < 1 || max_len > (1 << 23) || keys < 0 || keys > max_len)
+    return fail(IMQ_EINVAL, "B, Hkv, max_len or keys out of range");
+  const AttnPlan p = attention_plan(B, Hkv, max_len);
+  *wavefronts = p.waves;
+  *splits = p.splits;
+  *chunks = p.share ? shared_chunks((keys + kChunk - 1) / kChunk, p.splits, per_split_of(p.splits), p.cps) : p.cps;
+  return ok();
+}
 
 int32_t imq_attention_fused(const uint16_t* q, const uint16_t* k, const uint16_t* v,
                             const uint16_t* q_norm, const uint16_t* k_norm,
@@ -1760,7 +1807,7 @@ int32_t imq_program_launch_staged(imq_program* p, void* stream) {
     const dim3 grid(S.count), block(kThreads);
     const size_t lds = p->stage_lds[i];
     if (S.kind == kKindAttention) {
-      hipLaunchKernelGGL((attention_stage_kernel<kAttnWaves, false>), grid, block, lds, st, S, a);
+      hipLaunchKernelGGL((attention_stage_kernel<kAttnWaves, false, false>), grid, block, lds, st, S, a);
       continue;
     }
 #define IMQ_STAGE_CASE(NCH, XR, XSRC, EPI, SHAPE)                                              \

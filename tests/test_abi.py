@@ -247,3 +247,44 @@ def test_malformed_expert_calls_are_refused(lib, over, code):
     P = ctypes.c_void_p(1 << 20)
     assert lib.imq_prompt_experts(P, P, P, a["experts"], P, a["ldx"], a["per"], ctypes.c_void_p(a["idx"]), a["pairs"], P,
                                   64, 64, 128, 64, 4, 0, P, a["nbytes"], None) == code
+
+
+def _attention_plan(lib, b, hkv, max_len, keys):
+    """(wavefronts, splits, chunks of a split) of a fused attention launch."""
+    out = [ctypes.c_int32(0) for _ in range(3)]
+    assert lib.imq_attention_fused_plan(b, hkv, max_len, keys, *(ctypes.byref(v) for v in out)) == 0
+    return tuple(v.value for v in out)
+
+
+def _per_kernel_plan(b, hkv, max_len):
+    """(splits, chunks of a split) of imq_attention_decode: a chunk each up to 1024 workgroups."""
+    chunks = -(-max_len // 64)
+    per = -(-chunks // max(1, min(chunks, -(-1024 // (b * hkv)))))
+    return -(-chunks // per), per
+
+
+@pytest.mark.parametrize("hkv", [1, 2, 8])
+@pytest.mark.parametrize("b", [1, 2, 3, 4, 5, 7, 8, 14, 20, 32])
+def test_attention_splits_follow_the_request_not_the_cache(lib, b, hkv):
+    """Whatever the cache's size: a request's splits in use never pass the launched ones nor the
+    workspace's, and up to 1024 keys (a merge's worth of chunks) no wavefront takes more units of 16
+    keys than two, or than it would by the per-kernel plan, or, one split a pair, than all of them."""
+    for max_len in (64, 1000, 1024, 1025, 2048, 2049, 3071, 4096, 8192, 8193, 20000, 32768, 100003):
+        base, per = _per_kernel_plan(b, hkv, max_len)
+        for keys in (0, 1, 60, 64, 65, 128, 500, 512, 1000, 1024, 1025, 2000, 4097, 8192, 8193, max_len):
+            if keys > max_len:
+                continue
+            waves, splits, chunks = _attention_plan(lib, b, hkv, max_len, keys)
+            held = -(-keys // 64)
+            assert waves in (4, 8, 12) and 1 <= splits <= base and chunks >= 1
+            assert -(-held // chunks) <= splits
+            if 0 < keys <= 1024 and splits > 1:
+                rounds = -(-min(held, chunks) * 4 // waves)
+                assert rounds <= max(2, -(-min(held, per) * 4 // 4), -(-held * 4 // (waves * splits))), (max_len, keys)
+
+
+def test_malformed_attention_plans_are_refused(lib):
+    out = [ctypes.byref(ctypes.c_int32(0)) for _ in range(3)]
+    for args in ((0, 8, 64, 1), (1, 0, 64, 1), (1, 8, 0, 0), (1, 8, 64, 65), (1, 8, 64, -1), (1, 8, (1 << 23) + 1, 1)):
+        assert lib.imq_attention_fused_plan(*args, *out) == _native.IMQ_EINVAL
+    assert lib.imq_attention_fused_plan(1, 8, 64, 1, None, *out[1:]) == _native.IMQ_EINVAL

@@ -256,6 +256,20 @@ def test_attention_fused_long_contexts_and_split_counts(env, B, positions, cap):
     assert np.array_equal(bf16_bits(b[0]), first)
 
 
+@pytest.mark.parametrize("B,positions,cap", [
+    # a cache of 17 to 32 chunks, narrow with shared chunks: 16 chunks, 17 (two a split), nearly all
+    (1, [1023], 1100), (1, [1024], 2048), (1, [2040], 2048), (1, [3], 2048),
+    # 8 wavefronts: two chunks a split and less, more splits than a merge loads, the last one in part
+    (1, [2047], 4096), (1, [2048], 4096), (1, [4090], 4096), (2, [129, 4000], 4096), (3, [0, 700, 2040], 2048),
+    # 12 wavefronts: short requests beside full ones, 128 chunks and 129
+    (4, [8191, 64, 1000, 8192], 8200), (5, [31, 4095, 900, 2000, 6], 4096), (2, [16383, 9000], 16384),
+    (8, [500 * r + 63 for r in range(8)], 4096), (14, [147 * r for r in range(14)], 2048)])
+def test_attention_fused_short_requests_in_roomy_caches(env, B, positions, cap):
+    """Each request's chunks shared over its own splits, at lengths around the shares' edges: the
+    oracle's attention and the composition's pools, counters back at zero, the same bits again."""
+    test_attention_fused_long_contexts_and_split_counts(env, B, positions, cap)
+
+
 def fused_q_rot(torch, n, fused):
     """The rotated q of the fused call's inputs, by imq_qk_norm_rope on fresh pools."""
     q, k, v, qn, kn, pos, sl, kp, vp, out, max_len, theta, eps, ws, counters = fused
