@@ -494,14 +494,19 @@ def dequant(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
             out_dtype: torch.dtype = torch.float32, out: torch.Tensor | None = None,
             stream=None) -> torch.Tensor:
     """The dense (N, K) weight, scale*q + bias, as fp32 (bit-exact) or rounded to
-    bf16/fp16."""
-    n, k = check_weights(w, scales, biases)
-    if out_dtype not in _DTYPE_CODE:
-        raise ValueError(f"out_dtype must be fp32, bf16 or fp16, got {out_dtype}")
-    if out is None:
-        out = torch.empty((n, k), dtype=out_dtype, device=w.device)
-    _check(lib().imq_dequant(_ptr(w), _ptr(scales), _ptr(biases), _ptr(out),
-                             _DTYPE_CODE[out_dtype], n, k, GROUP_SIZE, BITS, _stream(stream)))
+    bf16/fp16; in a torch.jit trace a constant."""
+    tracing = torch._C._get_tracing_state()
+    torch._C._set_tracing_state(None)  # a traced torch.empty would be replayed without the kernel
+    try:
+        n, k = check_weights(w, scales, biases)
+        if out_dtype not in _DTYPE_CODE:
+            raise ValueError(f"out_dtype must be fp32, bf16 or fp16, got {out_dtype}")
+        if out is None:
+            out = torch.empty((n, k), dtype=out_dtype, device=w.device)
+        _check(lib().imq_dequant(_ptr(w), _ptr(scales), _ptr(biases), _ptr(out),
+                                 _DTYPE_CODE[out_dtype], n, k, GROUP_SIZE, BITS, _stream(stream)))
+    finally:
+        torch._C._set_tracing_state(tracing)
     return out
 
 
@@ -521,7 +526,7 @@ def takes_prompt(x: torch.Tensor, k: int) -> bool:
             and type(x) in (torch.Tensor, torch.nn.Parameter)
             and not (x.requires_grad and torch.is_grad_enabled())
             and torch.autograd.forward_ad._current_level < 0
-            and torch._C._functorch.peek_interpreter_stack() is None
+            and torch._C._get_tracing_state() is None and torch._C._functorch.peek_interpreter_stack() is None
             and torch._C._len_torch_dispatch_stack() == 0)
 
 

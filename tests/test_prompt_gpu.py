@@ -136,6 +136,27 @@ def test_calls_that_autograd_follows_keep_the_torch_product(env):
     assert (x.grad.float() - want).abs().max() <= 2.0**-7 * want.abs().max()  # fp16 weights, bf16 gradient
 
 
+@pytest.mark.parametrize("native", [False, True])
+def test_a_traced_module_computes_new_inputs(env, native):
+    """torch.jit.trace records torch operations: the trace has to hold the product, not its result,
+    and the dequantised weight as a constant (device memory is overwritten before the replay)."""
+    torch, n_, orc = env
+    from ironmule_amd import hip_native
+    from ironmule_amd.quantized import QuantizedLinear
+    announce("traced module", native)
+    m, n, k = 40, 96, 256
+    w, s, b, x = to_device(orc.synthetic(n, k, m, seed=orc.SEED_BASE + 965))
+    module = (hip_native.NativeQuantizedLinear if native else QuantizedLinear)(w, s, b)
+    traced = torch.jit.trace(module, x, check_trace=False)
+    junk = [torch.full((n, k), 7.0, device="cuda") for _ in range(8)] + [torch.full((n, k), 7.0, device="cuda").half() for _ in range(8)]
+    del junk
+    other = torch.randn((m, k), device="cuda").to(torch.bfloat16)
+    dense = n_.dequant(w, s, b).double()
+    ref, mag = other.double() @ dense.T, other.double().abs() @ dense.abs().T
+    # bf16 outputs; weights rounded to fp16 in the native module, fp32 sums in the plain one
+    assert ((traced(other).double() - ref).abs() <= 2.0**-8 * ref.abs() + 2.0**(-11 if native else -20) * mag).all()
+
+
 @pytest.mark.parametrize("e,n,k,tokens,top", [(8, 130, 192, 13, 5), (32, 256, 768, 128, 8), (3, 100, 1600, 200, 2),
                                               (64, 64, 256, 9, 8), (2, 300, 512, 400, 1)])
 @pytest.mark.parametrize("shared", [True, False])
