@@ -540,7 +540,7 @@ def _same_device(w: torch.Tensor, **others: torch.Tensor) -> None:
 
 def _aligned_rows(x: torch.Tensor, k: int) -> tuple[torch.Tensor, int]:
     """x as (rows, k) bf16 rows the kernels can load 16 bytes at a time, and their stride."""
-    x2 = x.reshape(-1, k)
+    x2 = x.reshape(-1, k).resolve_neg()  # (a lazily negated view: its memory holds the other sign)
     ld = int(x2.stride(0)) if x2.shape[0] > 1 else k
     if x2.stride(1) != 1 or ld < k or ld % 8 or x2.data_ptr() % 16:
         x2, ld = x2.clone(memory_format=torch.contiguous_format), k

@@ -98,6 +98,16 @@ def test_gathered_rows_refuse_x_of_another_device(no_launch):
                            torch.empty(3, dtype=torch.int32, device="meta"))
 
 
+def test_rows_are_taken_as_their_values_whatever_the_view():
+    x = torch.randn((40, K + 8)).to(torch.bfloat16)
+    for view in (x[:, :K], x[:, 3:3 + K], x[::2, :K], x[:1, :K].expand(40, K), torch._neg_view(x[:, :K].contiguous()),
+                 x[:, :K].t().contiguous().t(), x[:32, :K].reshape(4, 8, K).transpose(0, 1)):
+        rows, ld = _native._aligned_rows(view, K)
+        assert not rows.is_neg() and rows.stride(1) == 1 and rows.data_ptr() % 16 == 0 and ld % 8 == 0 and ld >= K
+        assert rows.shape[0] == 1 or rows.stride(0) == ld
+        assert torch.equal(rows, view.reshape(-1, K))
+
+
 def test_only_whole_aligned_expert_stacks_are_read_in_place():
     from ironmule_amd.quantized import _stack_as_stored
 
