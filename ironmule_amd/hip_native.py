@@ -14,8 +14,7 @@ call                                                  path
 ====================================================  =====================================
 bf16 x with at most MAX_ROWS (32) rows                imq_qmv, one weight sweep for all rows
 bf16 x with more rows (prefill)                       imq_prompt_matmul on the packed weight
-the same where autograd or a transform needs it, or   imq_dequant to fp16, one GEMM
-x holds GEMM_MIN_VALUES or more, K >= GEMM_MIN_K
+the same where autograd or a transform needs it       imq_dequant to fp16, one GEMM
 expert call, one bf16 row per (token, expert) pair,   imq_gather_qmv
 at most GATHER_MAX pairs
 anything else (fp32 x, larger expert batches)         the module's library path
@@ -51,13 +50,6 @@ GATHER_MAX = 64
 PROBE_TOLERANCE = 1e-2
 #: A probe of a weight taller than this uses its first PROBE_ROWS rows (all of K).
 PROBE_ROWS = 8192
-#: A long enough x over a wide enough weight takes the dequantised GEMM: its conversions of x, y
-#: and the weight are then small next to the product, which the library runs at a higher rate.
-#: Product on the packed weight / dequantise + GEMM, us: 15360 x 3840 2048 rows 293 / 289, 4096 rows
-#: 622 / 539; 2560 x 9728 1024 rows 90 / 103, 2048 rows 175 / 152; 4096 x 4096 2048 rows 99 / 104, 4096
-#: rows 199 / 173; but 9728 x 2560 4096 rows 293 / 306, 16384 rows 1119 / 1147.
-GEMM_MIN_K = 3072
-GEMM_MIN_VALUES = 15 << 20
 #: Share of device memory that weights plus the head's fp16 prefill copy may take.
 PREFILL_HEADROOM = 0.9
 
@@ -72,8 +64,6 @@ def _route(x: torch.Tensor, k: int) -> str:
         return "library"
     if x.numel() // k <= MAX_ROWS:
         return "qmv"
-    if k >= GEMM_MIN_K and x.numel() >= GEMM_MIN_VALUES:
-        return "dequant_gemm"
     return "prompt" if _native.takes_prompt(x, k) else "dequant_gemm"
 
 
