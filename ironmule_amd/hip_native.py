@@ -24,8 +24,8 @@ The reference's qmv route stops at 8 rows; the gfx950 kernel sweeps the weight o
 up to 32 rows, so the limit here is 32.
 
 `install` keeps everything on one model: it refuses off gfx950 or when nothing is
-eligible, probes one module of each (type, weight shape) class against a float32
-dequantise-then-matmul reference, and changes module classes only when every probe is
+eligible, probes one module of each (type, weight shape) class, from one row to a prompt of
+512, against a float32 dequantise-then-matmul reference, and changes module classes only when every probe is
 within PROBE_TOLERANCE.
 """
 
@@ -50,6 +50,9 @@ GATHER_MAX = 64
 PROBE_TOLERANCE = 1e-2
 #: A probe of a weight taller than this uses its first PROBE_ROWS rows (all of K).
 PROBE_ROWS = 8192
+#: Activation rows of the probe's calls: a decode step, a few requests, a short and a longer prompt
+#: (for experts, tokens: the gather kernel and batches of 9, 33 and 512 rows per expert).
+PROBE_CALLS = (1, 9, MAX_ROWS + 1, 512)
 #: Share of device memory that weights plus the head's fp16 prefill copy may take.
 PREFILL_HEADROOM = 0.9
 
@@ -176,29 +179,38 @@ def _eligible(module: torch.nn.Module) -> bool:
             and int(module.weight.shape[-1]) * 8 % 32 == 0)
 
 
-def _probe_input(k: int, device: torch.device) -> torch.Tensor:
+def _probe_input(rows: int, k: int, device: torch.device) -> torch.Tensor:
     gen = torch.Generator(device=device)
     gen.manual_seed(0)
-    return torch.randn((1, k), generator=gen, device=device).to(torch.bfloat16)
+    return torch.randn((rows, k), generator=gen, device=device).to(torch.bfloat16)
 
 
 def _probe(module: torch.nn.Module) -> float:
-    """The kernel's max|y - ref| / max|ref| on one seeded bf16 row and the module's own
-    weight, ref = the row in fp32 times imq_dequant's fp32 weight (the measure of
-    ironmule/cuda_native.py:253-268).  An expert stack is probed as one token routed to
-    its first eight experts; a weight taller than PROBE_ROWS by its first PROBE_ROWS rows."""
+    """The largest max|y - ref| / max|ref| over seeded bf16 inputs of PROBE_CALLS rows and the
+    module's own weight, through the calls an installed module makes; ref = the rows in fp32 times
+    imq_dequant's fp32 weight (the measure of ironmule/cuda_native.py:253-268).  An expert stack is
+    probed with every token routed to its first eight experts; a weight taller than PROBE_ROWS by
+    its first PROBE_ROWS rows."""
     w, scales, biases = module.weight, module.scales, module.biases
-    x = _probe_input(int(w.shape[-1]) * 8, w.device)
-    if isinstance(module, QuantizedSwitchLinear):
-        chosen = torch.arange(min(8, int(w.shape[0])), device=w.device)
-        got = gather_matmul(x.reshape(1, 1, -1), w, scales, biases, chosen.to(torch.int32))
-        w, scales, biases = (t[chosen].flatten(0, 1).contiguous() for t in (w, scales, biases))
+    k, stacked = int(w.shape[-1]) * 8, isinstance(module, QuantizedSwitchLinear)
+    if stacked:
+        chosen = torch.arange(min(8, int(w.shape[0])), dtype=torch.int32, device=w.device)
+        dense = _native.dequant(*(t[chosen.long()].flatten(0, 1).contiguous() for t in (w, scales, biases)),
+                                torch.float32)
     else:
         w, scales, biases = w[:PROBE_ROWS], scales[:PROBE_ROWS], biases[:PROBE_ROWS]
-        got = _qmv(x, w, scales, biases)
-    ref = x.float() @ _native.dequant(w, scales, biases, torch.float32).T
-    scale = ref.abs().max().clamp_min(1e-6)
-    return float((got.float().reshape(ref.shape) - ref).abs().max() / scale)
+        dense = _native.dequant(w, scales, biases, torch.float32)
+    worst = []
+    with torch.no_grad():
+        for rows in PROBE_CALLS:
+            x = _probe_input(rows, k, w.device)
+            if stacked:
+                got = gather_matmul(x.reshape(rows, 1, 1, k), w, scales, biases, chosen.expand(rows, -1))
+            else:
+                got = matmul(x, w, scales, biases)
+            ref = x.float() @ dense.T
+            worst.append((got.float().reshape(ref.shape) - ref).abs().max() / ref.abs().max().clamp_min(1e-6))
+    return float(torch.stack(worst).max())  # (a NaN stays one)
 
 
 def device_class(device_info: dict[str, Any] | None) -> str | None:
