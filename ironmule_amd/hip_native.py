@@ -231,7 +231,7 @@ def install(model: torch.nn.Module, device_info: dict[str, Any] | None) -> dict[
         raise ValueError("the native plan found no 4-bit group-64 affine bfloat16 weights")
     classes = {(type(m).__name__, tuple(m.weight.shape)): m for m in reversed(modules)}
     started = time.perf_counter()
-    worst = max(_probe(m) for m in classes.values())
+    worst = max((_probe(m) for m in classes.values()), key=lambda error: (error != error, error))  # NaN first
     elapsed = time.perf_counter() - started
     if not worst <= PROBE_TOLERANCE:
         raise ValueError(f"the native kernel disagrees with the float32 reference by "
