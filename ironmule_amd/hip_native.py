@@ -53,7 +53,7 @@ PROBE_ROWS = 8192
 #: Activation rows of the probe's calls: a decode step, a few requests, a short and a longer prompt
 #: (for experts, tokens: the gather kernel and batches of 9, 33 and 512 rows per expert).
 PROBE_CALLS = (1, 9, MAX_ROWS + 1, 512)
-#: Share of device memory that weights plus the head's fp16 prefill copy may take.
+#: Share of device memory that weights plus the reserve for a whole prompt's head may take.
 PREFILL_HEADROOM = 0.9
 
 _HEAD_NAMES = ("lm_head", "embed_tokens")
@@ -255,11 +255,13 @@ def _device_memory(info: dict[str, Any]) -> int | None:
 def head_skip_needed(model: torch.nn.Module, device_info: dict[str, Any] | None) -> str | None:
     """A reason to compute the prefill's output head for the last position only, or None.
 
-    The prefill route dequantises a weight to fp16 for its GEMM; for the head (lm_head or
-    a tied embed_tokens) that copy is N*K*2 bytes.  When the model's tensors plus the
-    largest such copy exceed PREFILL_HEADROOM of device memory, the reason says so.
-    Nothing is decided (None) when the device reports no memory size or the model has
-    no 4-bit head."""
+    A head (lm_head or a tied embed_tokens) over a whole prompt needs room beyond the weights:
+    on the packed product the bf16 logits of every row (N*2 bytes each), and where autograd or a
+    transform follows the call the head's fp16 copy (N*K*2 bytes, the reference's measure:
+    ironmule/cuda_native.py:271-303).  N*K*2 bytes are reserved for either, logits of up to K
+    rows.  When the model's tensors plus the largest such reserve exceed PREFILL_HEADROOM of
+    device memory, the reason says so.  Nothing is decided (None) when the device reports no
+    memory size or the model has no 4-bit head."""
     total = _device_memory(device_info or {})
     heads = [m for name, m in model.named_modules()
              if name.rsplit(".", 1)[-1] in _HEAD_NAMES
@@ -268,10 +270,10 @@ def head_skip_needed(model: torch.nn.Module, device_info: dict[str, Any] | None)
         return None
     tensors = [*model.parameters(), *model.buffers()]
     resident = sum(t.numel() * t.element_size() for t in tensors)
-    head_copy = max(int(m.weight.shape[0]) * int(m.weight.shape[1]) * 8 * 2 for m in heads)
+    reserve = max(int(m.weight.shape[0]) * int(m.weight.shape[1]) * 8 * 2 for m in heads)
     budget = PREFILL_HEADROOM * total
-    if resident + head_copy <= budget:
+    if resident + reserve <= budget:
         return None
-    return (f"{resident / 1e9:.2f} GB of weights and the head's {head_copy / 1e9:.2f} GB fp16 "
-            f"prefill copy exceed {budget / 1e9:.2f} GB ({PREFILL_HEADROOM:.0%} of "
+    return (f"{resident / 1e9:.2f} GB of weights and {reserve / 1e9:.2f} GB for the head over a "
+            f"whole prompt exceed {budget / 1e9:.2f} GB ({PREFILL_HEADROOM:.0%} of "
             f"{total / 1e9:.2f} GB), so the prefill computes the head at the last position only")

@@ -5,7 +5,8 @@ Bars (the decode step's): the last position's logits within max|logit - ref| / m
 <= 5e-4 (1e-4 for the decode step after it) of the oracle with the same bf16 rounding points; every key and value written to
 the request's KV slot within 5% of that layer's largest oracle entry; nothing written to
 other slots; and a decode step continuing at position T meets the logit bar again.
-Prompts of 7 tokens take the qmv kernel, 40 and 96 tokens the fp16 dequantise + GEMM path.
+Prompts of every length run imq_prompt_layer: 7 tokens part of a packed block of 32 rows, 40 and 96 more
+than one and blocks of 64 queries in part and in full.
 """
 
 from __future__ import annotations
