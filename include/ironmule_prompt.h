@@ -48,6 +48,12 @@ IMQ_API int32_t imq_prompt_product(const imq_problem* p, int32_t count, const vo
                                    int32_t group_size, int32_t bits, int32_t y_dtype, void* workspace,
                                    size_t workspace_bytes, void* stream);
 
+/* The plan of a product of M rows by 1 to 3 weights of N[i] x K on `cus` compute units, with at most
+ * max_splits K-ranges (8 in imq_prompt_product; in a layer 1 for q/k/v and gate/up, 8 for o and
+ * down): rows of a workgroup's tile (32, 64 or 128) and K-ranges.  Needs no device. */
+IMQ_API int32_t imq_prompt_plan(const int32_t* N, int32_t count, int32_t M, int32_t K, int32_t max_splits, int32_t cus,
+                                int32_t* tile_rows, int32_t* splits);
+
 /* imq_prompt_pack and imq_prompt_product of one weight in one call; the workspace (16-byte
  * aligned) holds the packed rows and the product's. */
 IMQ_API size_t imq_prompt_matmul_workspace(int32_t M, int32_t N, int32_t K);
@@ -58,6 +64,9 @@ IMQ_API int32_t imq_prompt_matmul(const uint32_t* w, const uint16_t* scales, con
 
 /* Bytes of workspace imq_prompt_experts takes (0: a size out of range). */
 IMQ_API size_t imq_prompt_experts_workspace(int32_t experts, int32_t pairs, int32_t K);
+
+/* Rows of a tile in imq_prompt_experts (32, 64 or 128).  Needs no device. */
+IMQ_API int32_t imq_prompt_experts_plan(int32_t experts, int32_t pairs, int32_t* tile_rows);
 
 /* y[p] = x[p / rows_per_x] W[idx[p]]^T for `pairs` (token, expert) pairs over stacked expert
  * weights (E, N, K/8), scales and biases (E, N, K/64): the pairs are sorted by expert on the

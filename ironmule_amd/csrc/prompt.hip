@@ -1322,6 +1322,19 @@ int32_t imq_prompt_product(const imq_problem* p, int32_t count, const void* pack
   return ok();
 }
 
+int32_t imq_prompt_plan(const int32_t* N, int32_t count, int32_t M, int32_t K, int32_t max_splits, int32_t cus,
+                        int32_t* tile_rows, int32_t* splits) {
+  if (!N || !tile_rows || !splits || count < 1 || count > IMQ_PROMPT_MAX_PROBLEMS || M < 1 ||
+      M > IMQ_PROMPT_MAX_ROWS || K < 64 || K % 64 || K > IMQ_PROMPT_MAX_K || max_splits < 1 || cus < 1)
+    return fail(IMQ_EINVAL, "null pointer or a size out of range");
+  for (int i = 0; i < count; ++i)
+    if (N[i] < 1) return fail(IMQ_EINVAL, "N must be >= 1");
+  const Plan plan = plan_product(N, count, M, K, cus, max_splits);
+  *tile_rows = 32 * plan.tm;
+  *splits = plan.splits;
+  return ok();
+}
+
 size_t imq_prompt_matmul_workspace(int32_t M, int32_t N, int32_t K) {
   const size_t packed = imq_prompt_packed_bytes(M, K);
   if (!packed || N < 1) return 0;
@@ -1351,6 +1364,13 @@ size_t imq_prompt_experts_workspace(int32_t experts, int32_t pairs, int32_t K) {
     return 0;
   const ExpertPlan p = plan_experts(experts, pairs);
   return round_up((size_t)p.tiles * 4, 256) + 2 * round_up((size_t)p.blocks * 32 * 4, 256) + packed_bytes(p.blocks, K);
+}
+
+int32_t imq_prompt_experts_plan(int32_t experts, int32_t pairs, int32_t* tile_rows) {
+  if (!tile_rows || experts < 1 || experts > IMQ_PROMPT_MAX_EXPERTS || pairs < 1 || pairs > IMQ_PROMPT_MAX_ROWS)
+    return fail(IMQ_EINVAL, "null pointer or a size out of range");
+  *tile_rows = 32 * plan_experts(experts, pairs).tm;
+  return ok();
 }
 
 int32_t imq_prompt_experts(const uint32_t* w, const uint16_t* scales, const uint16_t* biases, int32_t experts,

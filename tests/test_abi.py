@@ -288,3 +288,25 @@ def test_malformed_attention_plans_are_refused(lib):
     for args in ((0, 8, 64, 1), (1, 0, 64, 1), (1, 8, 0, 0), (1, 8, 64, 65), (1, 8, 64, -1), (1, 8, (1 << 23) + 1, 1)):
         assert lib.imq_attention_fused_plan(*args, *out) == _native.IMQ_EINVAL
     assert lib.imq_attention_fused_plan(1, 8, 64, 1, None, *out[1:]) == _native.IMQ_EINVAL
+
+
+def test_prompt_plans_without_a_device(lib):
+    """Plans are reported without a GPU, cover the K of a product, and refuse sizes out of range."""
+    rows, splits = ctypes.c_int32(), ctypes.c_int32()
+
+    def plan(sizes, m, k, most=8, cus=256):
+        return lib.imq_prompt_plan((ctypes.c_int32 * len(sizes))(*sizes), len(sizes), m, k, most, cus, ctypes.byref(rows),
+                                   ctypes.byref(splits))
+
+    for m in (1, 33, 77, 512, 4200):
+        for sizes in ((64,), (2560,), (4096, 1024, 1024), (9728, 9728)):
+            for k in (64, 320, 2560, 9728):
+                for most in (1, 8):
+                    assert plan(sizes, m, k, most) == 0
+                    assert rows.value in (32, 64, 128) and 1 <= splits.value <= min(most, -(-k // 256))
+    for bad in (((0,), 64, 64), ((64,), 0, 64), ((64,), (1 << 20) + 1, 64), ((64,), 64, 96), ((64,), 64, (1 << 17) + 64),
+                ((64,), 64, 64, 0), ((64,), 64, 64, 8, 0), ((64,) * 4, 64, 64)):
+        assert plan(*bad) == _native.IMQ_EINVAL
+    assert lib.imq_prompt_experts_plan(8, 8 * 24, ctypes.byref(rows)) == 0 and rows.value == 32
+    assert lib.imq_prompt_experts_plan(0, 8, ctypes.byref(rows)) == _native.IMQ_EINVAL
+    assert lib.imq_prompt_experts_plan(1025, 8, ctypes.byref(rows)) == _native.IMQ_EINVAL

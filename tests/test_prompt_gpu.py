@@ -2,9 +2,10 @@
 through the C ABI, against the oracle's float64 product.
 
 Bars (the qmv kernels'): fp32 outputs within 2^-20 sum|w x| + 2^-23 |ref|, bf16 outputs within
-one ulp of the rounded reference plus that allowance.  Sizes: one row past a 32-row block,
-blocks that a tile of 64 or 128 rows fills in part, N off the 128 columns of a workgroup, K of
-one group, groups off the chunks of four (scales of every alignment), and K-ranges.
+one ulp of the rounded reference plus that allowance.  Sizes (32-row tiles; the taller ones, and
+layers one at a time, are in test_prompt_layer_gpu.py): one row past a 32-row block, N off the 128
+columns of a workgroup, K of one group, groups off the chunks of four (scales of every alignment),
+and K-ranges.
 """
 
 from __future__ import annotations
