@@ -65,8 +65,8 @@ IMQ_API int32_t imq_prompt_matmul(const uint32_t* w, const uint16_t* scales, con
 /* Bytes of workspace imq_prompt_experts takes (0: a size out of range). */
 IMQ_API size_t imq_prompt_experts_workspace(int32_t experts, int32_t pairs, int32_t K);
 
-/* Rows of a tile in imq_prompt_experts (32, 64 or 128).  Needs no device. */
-IMQ_API int32_t imq_prompt_experts_plan(int32_t experts, int32_t pairs, int32_t* tile_rows);
+/* Rows of a tile in imq_prompt_experts (32 or 64) on `cus` compute units.  Needs no device. */
+IMQ_API int32_t imq_prompt_experts_plan(int32_t experts, int32_t pairs, int32_t N, int32_t cus, int32_t* tile_rows);
 
 /* y[p] = x[p / rows_per_x] W[idx[p]]^T for `pairs` (token, expert) pairs over stacked expert
  * weights (E, N, K/8), scales and biases (E, N, K/64): the pairs are sorted by expert on the

@@ -175,7 +175,7 @@ _SIGNATURES = {
     "imq_prompt_matmul": ([_P, _P, _P, _P, _I64, _P, _I64, _I32, _I32, _I32, _I32, _I32, _I32, _P, ctypes.c_size_t,
                            _P], _I32),
     "imq_prompt_experts_workspace": ([_I32, _I32, _I32], ctypes.c_size_t),
-    "imq_prompt_experts_plan": ([_I32, _I32, ctypes.POINTER(_I32)], _I32),
+    "imq_prompt_experts_plan": ([_I32, _I32, _I32, _I32, ctypes.POINTER(_I32)], _I32),
     "imq_prompt_experts": ([_P, _P, _P, _I32, _P, _I64, _I32, _P, _I32, _P, _I64, _I32, _I32, _I32, _I32, _I32, _P,
                             ctypes.c_size_t, _P], _I32),
     "imq_prompt_layer_workspace": ([ctypes.POINTER(PromptShape)], ctypes.c_size_t),

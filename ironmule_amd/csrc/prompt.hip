@@ -7,6 +7,7 @@
 #include <stdint.h>
 #include <string.h>
 
+#include <algorithm>
 #include <string>
 
 #include "../../include/ironmule_prompt.h"
@@ -979,20 +980,27 @@ Plan plan_product(const int32_t* N, int count, int M, int K, int cus, int max_sp
 }
 
 // Tiles for rows sorted by expert: at most pairs / (32 tm) full ones and a part-full one per
-// expert.  The tile height follows the pairs an expert gets on average: short tiles while most
-// of a taller one would be rows of zeros (1024 pairs of 32 experts: 38.7 us with tiles of 32 rows,
-// half of them a second tile for a few rows, 37.2 with 64).
+// expert.  Tiles of 32 rows while the experts used get up to 28 pairs on average, mostly one tile
+// each, or while the tiles to expect (half of one part-full per expert) make at most three
+// workgroups per CU; 64 beyond, where the weights read twice count for more than the rows of zeros.
+// 32 / 64 / 128 rows, us, at pairs per expert: 32 experts of 2560 x 768 at 20 27.4 / 35.2 / 67.8, at 32
+// 39.9 / 36.6 / 65.9, at 256 127 / 115 / 146; 8 of 2048 x 2048 at 64 33.5 / 36.1 / 46.0, at 256 69.9 /
+// 59.3 / 68.4, at 4000 664 / 531 / 544; 64 of 512 x 1024 at 32 30.9 / 39.0 / 59.7, at 96 53.1 / 55.2 /
+// 64.4.  Over 117 such points of ten stacks the choice is at most 13% above the best of the
+// three, 0.7% on average; 128 rows are the best of none.
 struct ExpertPlan {
   int tm, tiles, blocks;
 };
 
-ExpertPlan plan_experts(int experts, int pairs) {
-  const int used = experts < pairs ? experts : pairs;
-  ExpertPlan p;
-  p.tm = pairs <= 24 * used ? 1 : pairs <= 160 * used ? 2 : 4;
-  p.tiles = pairs / (32 * p.tm) + used;
-  p.blocks = p.tiles * p.tm;
-  return p;
+ExpertPlan expert_tiles(int experts, int pairs, int tm) {
+  const int tiles = pairs / (32 * tm) + std::min(experts, pairs);
+  return ExpertPlan{tm, tiles, tiles * tm};
+}
+
+ExpertPlan plan_experts(int experts, int pairs, int N, int cus) {
+  const int64_t used = std::min(experts, pairs), columns = ceil_div(N, kColumns);
+  const bool small = pairs <= 28 * used || (pairs / 32 + used / 2) * columns <= 3 * (int64_t)cus;
+  return expert_tiles(experts, pairs, small ? 1 : 2);
 }
 
 size_t packed_bytes(int64_t blocks, int K) { return (size_t)blocks * ceil_div(K, 256) * kChunkBytes; }
@@ -1362,14 +1370,16 @@ size_t imq_prompt_experts_workspace(int32_t experts, int32_t pairs, int32_t K) {
   if (experts < 1 || experts > IMQ_PROMPT_MAX_EXPERTS || pairs < 1 || pairs > IMQ_PROMPT_MAX_ROWS || K < 64 ||
       K % 64 || K > IMQ_PROMPT_MAX_K)
     return 0;
-  const ExpertPlan p = plan_experts(experts, pairs);
-  return round_up((size_t)p.tiles * 4, 256) + 2 * round_up((size_t)p.blocks * 32 * 4, 256) + packed_bytes(p.blocks, K);
+  // for any N: the short tiles are the more, the tall ones the more blocks
+  const int tiles = expert_tiles(experts, pairs, 1).tiles, blocks = expert_tiles(experts, pairs, 2).blocks;
+  return round_up((size_t)tiles * 4, 256) + 2 * round_up((size_t)blocks * 32 * 4, 256) + packed_bytes(blocks, K);
 }
 
-int32_t imq_prompt_experts_plan(int32_t experts, int32_t pairs, int32_t* tile_rows) {
-  if (!tile_rows || experts < 1 || experts > IMQ_PROMPT_MAX_EXPERTS || pairs < 1 || pairs > IMQ_PROMPT_MAX_ROWS)
+int32_t imq_prompt_experts_plan(int32_t experts, int32_t pairs, int32_t N, int32_t cus, int32_t* tile_rows) {
+  if (!tile_rows || experts < 1 || experts > IMQ_PROMPT_MAX_EXPERTS || pairs < 1 || pairs > IMQ_PROMPT_MAX_ROWS ||
+      N < 1 || cus < 1)
     return fail(IMQ_EINVAL, "null pointer or a size out of range");
-  *tile_rows = 32 * plan_experts(experts, pairs).tm;
+  *tile_rows = 32 * plan_experts(experts, pairs, N, cus).tm;
   return ok();
 }
 
@@ -1387,9 +1397,10 @@ int32_t imq_prompt_experts(const uint32_t* w, const uint16_t* scales, const uint
   if (rows_per_x < 1) return fail(IMQ_EINVAL, "rows_per_x must be >= 1");
   if (workspace_bytes < imq_prompt_experts_workspace(experts, pairs, K))
     return fail(IMQ_EINVAL, "the workspace is too small");
-  if (!current_device(&code)) return code;
+  const DeviceInfo* dev = current_device(&code);
+  if (!dev) return code;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const ExpertPlan e = plan_experts(experts, pairs);
+  const ExpertPlan e = plan_experts(experts, pairs, N, dev->cu_count);
   char* at = static_cast<char*>(workspace);
   int32_t* const tile_expert = reinterpret_cast<int32_t*>(at);
   at += round_up((size_t)e.tiles * 4, 256);

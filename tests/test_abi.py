@@ -307,6 +307,29 @@ def test_prompt_plans_without_a_device(lib):
     for bad in (((0,), 64, 64), ((64,), 0, 64), ((64,), (1 << 20) + 1, 64), ((64,), 64, 96), ((64,), 64, (1 << 17) + 64),
                 ((64,), 64, 64, 0), ((64,), 64, 64, 8, 0), ((64,) * 4, 64, 64)):
         assert plan(*bad) == _native.IMQ_EINVAL
-    assert lib.imq_prompt_experts_plan(8, 8 * 24, ctypes.byref(rows)) == 0 and rows.value == 32
-    assert lib.imq_prompt_experts_plan(0, 8, ctypes.byref(rows)) == _native.IMQ_EINVAL
-    assert lib.imq_prompt_experts_plan(1025, 8, ctypes.byref(rows)) == _native.IMQ_EINVAL
+
+
+def test_expert_tiles_by_pairs_and_workgroups(lib):
+    """Tiles of 64 rows only past 28 pairs per expert and three workgroups per CU (the measured table
+    beside the rule), and a workspace that holds either."""
+    rows = ctypes.c_int32()
+
+    def plan(*args):
+        assert lib.imq_prompt_experts_plan(*args, ctypes.byref(rows)) == 0
+        return rows.value
+
+    for experts, per, n, want in ((32, 20, 2560, 32), (32, 28, 2560, 32), (32, 32, 2560, 64), (32, 256, 2560, 64),
+                                  (8, 64, 2048, 32), (8, 128, 2048, 32), (8, 256, 2048, 64), (64, 32, 512, 32),
+                                  (64, 96, 512, 64), (16, 128, 1024, 32), (16, 400, 1024, 64), (128, 28, 1536, 32),
+                                  (128, 40, 1536, 64), (1, 64, 64, 32), (1, 1 << 20, 64, 64)):
+        assert plan(experts, experts * per, n, 256) == want, (experts, per, n)
+    for experts in (1, 7, 1024):
+        for pairs in (1, 63, 64, 65, 1000, 9999):
+            used, k = min(experts, pairs), 320
+            nbytes = lib.imq_prompt_experts_workspace(experts, pairs, k)
+            for tm in (1, 2):
+                tiles = pairs // (32 * tm) + used
+                packed = lib.imq_prompt_packed_bytes(32, k) * tiles * tm
+                assert nbytes >= tiles * 4 + 2 * tiles * tm * 32 * 4 + packed
+    for bad in ((0, 8, 64, 256), (1025, 8, 64, 256), (8, 0, 64, 256), (8, 8, 0, 256), (8, 8, 64, 0)):
+        assert lib.imq_prompt_experts_plan(*bad, ctypes.byref(rows)) == _native.IMQ_EINVAL

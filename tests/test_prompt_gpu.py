@@ -162,7 +162,7 @@ def test_a_traced_module_computes_new_inputs(env, native):
                                               (64, 64, 256, 9, 8), (2, 300, 512, 400, 1)])
 @pytest.mark.parametrize("shared", [True, False])
 def test_expert_batches_against_the_oracle(env, e, n, k, tokens, top, shared):
-    """Pairs sorted by expert, tiles of 32, 64 and 128 rows, experts without pairs (64 experts,
+    """Pairs sorted by expert, experts without pairs (64 experts,
     72 pairs on the even ones), a token's row shared by its experts or a row per pair."""
     torch, n_, orc = env
     from ironmule_amd.quantized import library_gather_matmul

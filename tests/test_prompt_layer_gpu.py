@@ -282,16 +282,18 @@ def test_grouped_products_in_k_ranges(env, m, sizes, k, rows, dtype):
         assert (y[:, n:] == 7.0).all()
 
 
-@pytest.mark.parametrize("experts,tokens,top,rows", [(8, 24, 8, 32), (8, 25, 8, 64), (8, 160, 8, 64), (8, 161, 8, 128),
-                                                     (1, 700, 1, 128), (1024, 40, 8, 32)])
-def test_expert_batches_of_each_tile_height(env, experts, tokens, top, rows):
+@pytest.mark.parametrize("experts,tokens,top,n,rows", [
+    (8, 28, 8, 12290, 32), (8, 29, 8, 12290, 64), (8, 160, 8, 66, 32), (8, 161, 8, 2200, 64), (1, 700, 1, 66, 32),
+    (1, 3000, 1, 1100, 64), (1024, 40, 8, 66, 32)])
+def test_expert_batches_of_each_tile_height(env, experts, tokens, top, n, rows):
     """Around the edges of the tile rule, with uneven experts: half of the pairs on the first one."""
     torch, n_, orc = env
     from ironmule_amd.quantized import library_gather_matmul
-    announce("experts plan", experts, tokens, top)
+    announce("experts plan", experts, tokens, top, n)
     made = ctypes.c_int32()
-    assert n_.lib().imq_prompt_experts_plan(experts, tokens * top, ctypes.byref(made)) == 0 and made.value == rows
-    n, k = 66, 192
+    assert n_.lib().imq_prompt_experts_plan(experts, tokens * top, n, n_.device_check()[2], ctypes.byref(made)) == 0
+    assert made.value == rows
+    k = 192
     gen = torch.Generator(device="cuda")
     gen.manual_seed(tokens)
     stack = tuple(t.view(experts, n, -1) for t in _weight(torch, gen, experts * n, k))
