@@ -1384,20 +1384,25 @@ AttnPlan attention_plan(int B, int Hkv, int span) {
   return p;
 }
 
-template <int W, bool kPlanes, bool kShare>
-int32_t launch_attention(const Stage& A, const StepArgs& a, int device, hipStream_t stream) {
+template <int W, bool kShare>
+int32_t launch_attention(const Stage& A, const StepArgs& a, bool planes, int device, hipStream_t stream) {
   const size_t lds = (sizeof(AttnLdsT<W>) + 15) & ~(size_t)15;
-  if (lds > 64 * 1024) {  // above the default dynamic limit: raised once per device
+  if (lds > 64 * 1024) {  // above the default dynamic limit: raised once per device, for both forms of the kernel
     static std::atomic<bool> raised[imq_rt::kMaxDevices];
     if (!raised[device].load(std::memory_order_acquire)) {
-      const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(attention_stage_kernel<W, kPlanes, kShare>),
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      if (attr != hipSuccess)
-        return fail(IMQ_ELAUNCH, std::string("fused attention LDS size: ") + hipGetErrorString(attr));
+      for (const void* fn : {reinterpret_cast<const void*>(attention_stage_kernel<W, true, kShare>),
+                             reinterpret_cast<const void*>(attention_stage_kernel<W, false, kShare>)}) {
+        const hipError_t attr = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (attr != hipSuccess)
+          return fail(IMQ_ELAUNCH, std::string("fused attention LDS size: ") + hipGetErrorString(attr));
+      }
       raised[device].store(true, std::memory_order_release);
     }
   }
-  hipLaunchKernelGGL((attention_stage_kernel<W, kPlanes, kShare>), dim3(A.count), dim3(64 * W), lds, stream, A, a);
+  if (planes)
+    hipLaunchKernelGGL((attention_stage_kernel<W, true, kShare>), dim3(A.count), dim3(64 * W), lds, stream, A, a);
+  else
+    hipLaunchKernelGGL((attention_stage_kernel<W, false, kShare>), dim3(A.count), dim3(64 * W), lds, stream, A, a);
   return IMQ_OK;
 }
 
@@ -1475,18 +1480,10 @@ int32_t attention_fused(const uint16_t* q, const uint16_t* k, const uint16_t* v,
   a.ntasks = A.count;
   a.staged = 1;
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  if (plan.waves == kManyWaves)
-    code = planes ? launch_attention<kManyWaves, true, true>(A, a, device, st)
-                  : launch_attention<kManyWaves, false, true>(A, a, device, st);
-  else if (plan.waves == kFewWaves)
-    code = planes ? launch_attention<kFewWaves, true, true>(A, a, device, st)
-                  : launch_attention<kFewWaves, false, true>(A, a, device, st);
-  else if (plan.share)
-    code = planes ? launch_attention<kAttnWaves, true, true>(A, a, device, st)
-                  : launch_attention<kAttnWaves, false, true>(A, a, device, st);
-  else
-    code = planes ? launch_attention<kAttnWaves, true, false>(A, a, device, st)
-                  : launch_attention<kAttnWaves, false, false>(A, a, device, st);
+  code = plan.waves == kManyWaves  ? launch_attention<kManyWaves, true>(A, a, planes, device, st)
+         : plan.waves == kFewWaves ? launch_attention<kFewWaves, true>(A, a, planes, device, st)
+         : plan.share              ? launch_attention<kAttnWaves, true>(A, a, planes, device, st)
+                                   : launch_attention<kAttnWaves, false>(A, a, planes, device, st);
   if (code != IMQ_OK) return code;
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(IMQ_ELAUNCH, std::string("fused attention launch: ") + hipGetErrorString(e));
