@@ -112,17 +112,19 @@ __global__ __launch_bounds__(kThreads) void pack_rows_kernel(const uint16_t* __r
 // One barrier per group.  Within a wavefront the scaling of one tile, the LDS reads of the
 // next and the unpacking of the next group's weights are issued between a tile's MFMAs.
 //
-// What bounds it (K = 2560, 512 workgroups of TM = 4, two per CU; a group takes 1.0 us): the
-// MFMAs (half of that time) and the 16 FMAs and 8 unpackings per four of them, which overlap only
-// in part.  Without loads and LDS reads, on constant data, a group takes 0.61 us; taking out the
-// waits, the barriers or the distance to memory (every load from one line) changes it by 3% or
-// less.  860 TFLOP/s on large launches, 755 at 512 workgroups with a launch's start and end.
-// Not faster: 64 x 64 per wavefront (half the LDS reads, twice the unpacking), eight wavefronts
-// over 256 columns, one wait for a unit's four operands in place of one each (large launches 4%
-// faster, 1024 x 9728 2% slower); 128 x 64 per wavefront took 930 TFLOP/s in an earlier form, but
-// its 256-column tiles leave a prompt of 512 rows with too few workgroups.  Against imq_dequant and a library product (two conversions of the
-// activations besides): 1024 x 9728 x 2560 90 -> 80 us in fp16, 77 x 2560 x 9728 70.9 -> 26 us in
-// fp32.
+// What bounds it: issue.  By the counters of a 512-token prompt's layer the MFMAs are busy 38% of
+// gate/up's CU cycles (TM = 2, 1216 workgroups, 79 us) and 34% of down's (TM = 4, three K-ranges,
+// 45.5 us), with no LDS bank conflicts; the 16 FMAs and 8 unpackings per four MFMAs overlap them only
+// in part, and waves spend a quarter to half of their cycles waiting to issue.  Taking out the
+// counted waits, the barriers or the distance to memory (every load from one line) changed a group
+// by 3% or less.  Small launches add a start and an end: q/k/v (TM = 1) 39 us, o (160 workgroups) 36.
+// 2048 x 4096 x 2560 60 us, 712 TFLOP/s; 8192 x 15360 x 3840 1338 us, 722.  Not faster: 64 x 64 per
+// wavefront (half the LDS reads, twice the unpacking), eight wavefronts over 256 columns, one wait for
+// a unit's four operands in place of one each (large launches 4% faster, 1024 x 9728 2% slower).
+// Against imq_dequant and a library product (two conversions of the activations besides): 1024 x 9728
+// x 2560 90 -> 80 us in fp16, 77 x 2560 x 9728 70.9 -> 26 us in fp32; from about 2048 rows over weights
+// of 2500 rows and more that way is the faster one (4096 x 15360 x 3840 524 us, 613 here), at fp16's
+// range and rounding.
 struct ProductProblem {
   const uint32_t* w;
   const uint16_t* s;
@@ -956,7 +958,9 @@ int column_tiles(const int32_t* N, int count) {
 // groups) over 32 to 2048 workgroups, a launch takes about 14 / 11 / 9 us, and per group and
 // workgroup of the busiest CU 0.56 / 0.31 / 0.20 us, with tiles of 128 / 64 / 32 rows: tall
 // tiles reuse the weights, short ones fill the CUs.  K-ranges add the planes' traffic (about
-// 4 TB/s each way) and the launch that adds them.
+// 4 TB/s each way) and the launch that adds them; a layer's o and down are charged both too, though
+// norm_pack_kernel adds their planes.  Predicted / traced for 512 tokens of 2560 hidden: q/k/v 33 /
+// 39 us, o 31 / 36, gate/up 73 / 79, down in three ranges 56 / 45.
 Plan plan_product(const int32_t* N, int count, int M, int K, int cus, int max_splits = 8) {
   const int chunks = ceil_div(K, 256), col_tiles = column_tiles(N, count);
   double columns = 0.0, best = 0.0;

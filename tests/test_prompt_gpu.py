@@ -137,6 +137,7 @@ def test_calls_that_autograd_follows_keep_the_torch_product(env):
     assert (x.grad.float() - want).abs().max() <= 2.0**-7 * want.abs().max()  # fp16 weights, bf16 gradient
 
 
+@pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning")
 @pytest.mark.parametrize("native", [False, True])
 def test_a_traced_module_computes_new_inputs(env, native):
     """torch.jit.trace records torch operations: the trace has to hold the product, not its result,
@@ -162,8 +163,8 @@ def test_a_traced_module_computes_new_inputs(env, native):
                                               (64, 64, 256, 9, 8), (2, 300, 512, 400, 1)])
 @pytest.mark.parametrize("shared", [True, False])
 def test_expert_batches_against_the_oracle(env, e, n, k, tokens, top, shared):
-    """Pairs sorted by expert, experts without pairs (64 experts,
-    72 pairs on the even ones), a token's row shared by its experts or a row per pair."""
+    """Pairs sorted by expert, experts without pairs (64 experts, 72 pairs on the even ones), a token's
+    row shared by its experts or a row per pair."""
     torch, n_, orc = env
     from ironmule_amd.quantized import library_gather_matmul
     announce("experts", e, n, k, tokens, top, shared)

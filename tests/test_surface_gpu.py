@@ -140,7 +140,7 @@ def test_native_plan_install_and_routing(oracle):
     y = model.proj(x[None])
     _bound(oracle, pr, y)
     assert torch.equal(model.embed_tokens.as_linear(x[None]), y)
-    # more than 32 rows: dequantise to fp16 and one GEMM, within the probe tolerance
+    # more than 32 rows: one product on the packed weight, within the probe tolerance
     rows = torch.randn((1, 40, 2560), device="cuda").to(torch.bfloat16)
     got = model.proj(rows).float()
     ref = rows.float() @ _native.dequant(w, s, b, torch.float32).T
