@@ -533,18 +533,20 @@ def takes_prompt(x: torch.Tensor, k: int) -> bool:
             and torch._C._len_torch_dispatch_stack() == 0)
 
 
-def _same_device(w: torch.Tensor, **others: torch.Tensor) -> None:
-    """The kernels read every operand through its address: one on the host or on another GPU would
-    be a stray access there, or one that its own device's streams do not order."""
-    for name, t in others.items():
-        if t.device != w.device:
-            raise ValueError(f"{name} is on {t.device}, expected {w.device}")
+def _same_device(index: int, *tensors: torch.Tensor) -> None:
+    """The kernels read every operand through its address: one on the host (index -1) or on another
+    GPU would be a stray access there, or one that its own device's streams do not order."""
+    for t in tensors:
+        if t.get_device() != index:  # (half the time of comparing .device)
+            raise ValueError(f"a tensor of shape {tuple(t.shape)} is on {t.device}, the weights on GPU {index}")
 
 
 def _aligned_rows(x: torch.Tensor, k: int) -> tuple[torch.Tensor, int]:
     """x as (rows, k) bf16 rows the kernels can load 16 bytes at a time, and their stride."""
-    x2 = x.reshape(-1, k).resolve_neg()  # (a lazily negated view: its memory holds the other sign)
-    ld = int(x2.stride(0)) if x2.shape[0] > 1 else k
+    x2 = x.reshape(-1, k)
+    if x2.is_neg():  # a lazily negated view: its memory holds the other sign
+        x2 = x2.resolve_neg()
+    ld = x2.stride(0) if x2.shape[0] > 1 else k
     if x2.stride(1) != 1 or ld < k or ld % 8 or x2.data_ptr() % 16:
         x2, ld = x2.clone(memory_format=torch.contiguous_format), k
     return x2, ld
@@ -556,17 +558,35 @@ def prompt_matmul(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor, x
     exact products of the 4-bit weights as they are stored, fp32 sums, y bf16 or fp32 (M, N),
     on the current stream."""
     n, k = check_weights(w, scales, biases)
-    if x.dtype != torch.bfloat16 or x.dim() < 1 or int(x.shape[-1]) != k:
+    if x.dtype != torch.bfloat16 or x.dim() < 1 or x.shape[-1] != k:
         raise ValueError(f"x must be bf16 rows of {k} values")
-    _same_device(w, scales=scales, biases=biases, x=x)
+    _same_device(w.get_device(), scales, biases, x)
     x2, ld = _aligned_rows(x, k)
-    m = int(x2.shape[0])
+    m = x2.shape[0]
     out = torch.empty((m, n), dtype=out_dtype, device=w.device)
-    nbytes = int(lib().imq_prompt_matmul_workspace(m, n, k))
+    library = _lib or lib()
+    nbytes = library.imq_prompt_matmul_workspace(m, n, k)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=w.device)
-    _check(lib().imq_prompt_matmul(_ptr(w), _ptr(scales), _ptr(biases), _ptr(x2), ld, _ptr(out), n, m, n, k,
-                                   GROUP_SIZE, BITS, _DTYPE_CODE[out_dtype], _ptr(ws), nbytes, _stream(None)))
+    _check(library.imq_prompt_matmul(w.data_ptr(), scales.data_ptr(), biases.data_ptr(), x2.data_ptr(), ld,
+                                     out.data_ptr(), n, m, n, k, GROUP_SIZE, BITS, _DTYPE_CODE[out_dtype],
+                                     ws.data_ptr(), nbytes, _stream(None)))
     return out
+
+
+def _check_stack(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor) -> tuple[int, int, int]:
+    """(experts, N, K) of a well-formed stack of 4-bit weights, whole and in order, else ValueError."""
+    if w.dim() != 3 or scales.dim() != 3 or biases.dim() != 3:
+        raise ValueError("w, scales and biases must be stacked by expert")
+    e, n, words = w.shape
+    groups = (e, n, words >> 3)
+    if not (words & 7 == 0 and (w.dtype is torch.int32 or w.dtype is torch.uint32)
+            and scales.dtype is torch.bfloat16 and biases.dtype is torch.bfloat16
+            and scales.shape == groups and biases.shape == groups and w.is_cuda
+            and w.is_contiguous() and scales.is_contiguous() and biases.is_contiguous()):
+        check_weights(*(t.reshape(-1, t.shape[2]) for t in (w, scales, biases)))  # says what is wrong
+        if scales.shape != groups or biases.shape != groups or not all(t.is_contiguous() for t in (w, scales, biases)):
+            raise ValueError("w, scales and biases must be contiguous and agree expert by expert")
+    return e, n, words * 8
 
 
 def prompt_experts(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor, x: torch.Tensor,
@@ -575,13 +595,10 @@ def prompt_experts(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor, 
     pairs (imq_prompt_experts), the pairs sorted by expert on the device; w (E, N, K/8), scales
     and biases (E, N, K/64), x bf16 rows, idx integers on the device (negative ones count from
     the last expert).  Returns (pairs, N), on the current stream."""
-    if w.dim() != 3 or scales.dim() != 3 or biases.dim() != 3:
-        raise ValueError("w, scales and biases must be stacked by expert")
-    e, n = int(w.shape[0]), int(w.shape[1])
-    k = check_weights(*(t.view(e * n, -1) for t in (w, scales, biases)))[1]
+    e, n, k = _check_stack(w, scales, biases)
     if x.dtype != torch.bfloat16 or int(x.shape[-1]) != k:
         raise ValueError(f"x must be bf16 rows of {k} values")
-    _same_device(w, scales=scales, biases=biases, x=x, idx=idx)
+    _same_device(w.get_device(), scales, biases, x, idx)
     x2, ld = _aligned_rows(x, k)
     idx = idx.reshape(-1).to(torch.int32).contiguous()
     pairs = int(idx.numel())
@@ -618,12 +635,12 @@ class PromptLayers:
         self.workspace = torch.empty(self.nbytes, dtype=torch.uint8, device=h.device)
 
     def layer(self, layer: dict, k_pool: torch.Tensor, v_pool: torch.Tensor) -> None:
-        quants = []
+        quants, index = [], self.h.get_device()
         for name, size in self.config.projections.items():
             if check_weights(*layer[name]) != tuple(size):
                 raise ValueError(f"{name} must be {tuple(size)}")
             w, scales, biases = layer[name]
-            _same_device(self.h, **{name: w, f"{name} scales": scales, f"{name} biases": biases})
+            _same_device(index, w, scales, biases)
             quants.append(QWeight(w.data_ptr(), scales.data_ptr(), biases.data_ptr()))
         norms = [layer[name] for name in ("input_norm", "post_norm", "q_norm", "k_norm")]
         for t, want in zip(norms, (self.config.hidden, self.config.hidden, 128, 128)):
@@ -634,8 +651,7 @@ class PromptLayers:
             _require(t, torch.bfloat16, "a pool")
             if tuple(t.shape) != self.pool_shape:
                 raise ValueError(f"a pool must be {self.pool_shape}")
-        for t in (*norms, k_pool, v_pool):
-            _same_device(self.h, **{"a norm weight or pool": t})
+        _same_device(index, *norms, k_pool, v_pool)
         desc = StepLayer(*quants, *[t.data_ptr() for t in norms], k_pool.data_ptr(), v_pool.data_ptr())
         _check(lib().imq_prompt_layer(ctypes.byref(desc), ctypes.byref(self.shape), _ptr(self.h), self.first,
                                       _ptr(self.workspace), self.nbytes, _stream(None)))

@@ -168,8 +168,7 @@ def _stack_as_stored(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor
     """Whether the kernels can read an expert stack where it lies: whole, in order, 16-byte
     aligned.  A slice of a fused stack, every other expert or a view off that alignment is copied
     expert by expert instead."""
-    return (w.dim() == scales.dim() == biases.dim() == 3 and w.is_contiguous() and scales.is_contiguous()
-            and biases.is_contiguous() and w.data_ptr() % 16 == 0)
+    return w.is_contiguous() and scales.is_contiguous() and biases.is_contiguous() and w.data_ptr() % 16 == 0
 
 
 def library_gather_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor,
